@@ -565,10 +565,22 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   sp.tile_sx = swe::kStepShape[c->shape].sx;
   sp.tile_sy = swe::kStepShape[c->shape].sy;
 
-  // colour-ordered cascade: every window's step kernel only moves the
-  // particles (MODE 2), and its relax follows at once as one launch per
-  // colour class; no closing relax-only window
-  const bool colour = colour_mode(c->p);
+  // colour-ordered cascade: inside the step kernel (k_colour_step), with the
+  // same windows as the synchronous one.  On maps under three cells along an
+  // axis a cell's neighbours alias across the wrap; there every window's step
+  // kernel only moves the particles (MODE 2), and its relax follows at once
+  // as one launch per colour class, with no closing relax-only window.
+  bool alias = false;
+  sa.chalo = swe::kColourHalo;
+  for (int32_t k = 0; k < c->nterr; k++) {
+    alias = alias || c->tnx[(size_t)k] < 3 || c->tny[(size_t)k] < 3;
+    const swe::ColourHalo h = swe::colour_halo(c->tnx[(size_t)k], c->tny[(size_t)k], c->p.periodic != 0);
+    sa.chalo.xl = std::max(sa.chalo.xl, h.xl);
+    sa.chalo.xh = std::max(sa.chalo.xh, h.xh);
+    sa.chalo.yl = std::max(sa.chalo.yl, h.yl);
+    sa.chalo.yh = std::max(sa.chalo.yh, h.yh);
+  }
+  const bool colour = colour_mode(c->p) && alias, fused = colour_mode(c->p) && !alias;
   swe::RelaxArgs ra{};
   ra.nx = c->nx;
   ra.ny = c->ny;
@@ -634,7 +646,7 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
         int rr;
         if ((rr = timed_begin(c, &e0, &e1))) return rr;
         swe::launch_step(c->shape, sa, c->p.periodic != 0, c->p.track != 0, c->p.layers,
-                         c->p.deposit_on_death != 0, colour ? 2 : (w == nwin ? 1 : 0), c->stream);
+                         c->p.deposit_on_death != 0, colour ? 2 : (w == nwin ? 1 : 0) + (fused ? 3 : 0), c->stream);
         HIPCHK(c, hipGetLastError());
         if ((rr = timed_end(c, e0, e1, 2))) return rr;
         if (colour) {  // the step kernel wrote the masters with the pickups and their snapshots

@@ -22,6 +22,28 @@ constexpr StepShape kStepShape[kStepShapes] = {
 };
 constexpr int kStepChunk = 32;                 // tiles per chunk sum of the input counts
 
+// Halo of the cells that the colour-ordered relax of a tile and its one-cell
+// halo can depend on: a cascade reads and writes its 3 x 3 block, so a
+// dependence runs through cells of decreasing class at most two cells apart.
+// Away from the extra classes of a periodic axis, with classes x-major, x
+// changes only between the three x classes and y in every step, which gives
+// (-4 .. +6) x (-10 .. +18) around a cell.  A region that meets one of the
+// last n mod 3 cells of a periodic axis sees up to five classes an axis:
+// (-5 .. +6) x (-14 .. +24) when no axis has two such cells and both are at
+// least 16 cells, (-6 .. +6) x (-26 .. +30) otherwise.  The extents, one
+// larger each way for the tile's one-cell halo, are checked against the full
+// dependence sets in tests/test_colour_halo.py.
+struct ColourHalo {
+  int32_t xl, xh, yl, yh;
+};
+constexpr ColourHalo kColourHalo = {5, 7, 11, 19};
+constexpr ColourHalo kColourHaloSeam = {6, 7, 15, 25};
+constexpr ColourHalo kColourHaloMax = {7, 7, 27, 31};
+inline ColourHalo colour_halo(int32_t nx, int32_t ny, bool periodic) {
+  if (!periodic || (nx % 3 == 0 && ny % 3 == 0)) return kColourHalo;
+  return nx % 3 <= 1 && ny % 3 <= 1 && nx >= 16 && ny >= 16 ? kColourHaloSeam : kColourHaloMax;
+}
+
 // One terrain of a context: its cells, tiles and particles are contiguous
 // ranges of the context's buffers
 struct Terrain {
@@ -105,6 +127,7 @@ struct StepArgs {
   int32_t default_slots;     // workgroups of the usual order: ntiles (a multiple of 8 with light slots)
   int32_t light_slots;       // 0 = off, else a multiple of 8: light tiles last, per XCD
   int32_t window;            // window index within the cycle
+  ColourHalo chalo;          // colour-ordered relax: halo of tiles near a seam (the widest of all terrains)
   const uint32_t* heavy_cur; // this launch's listed tiles: kHeavySlotsMax heavy, then light_slots light,
                              // each part in 8 equal per-XCD lists
   uint32_t* heavy_next;      // the next launch's (appended here)

@@ -73,6 +73,8 @@ struct TileAcc {
   }
 };
 
+extern __shared__ __attribute__((aligned(16))) unsigned char s_dyn[];  // k_colour_step's working sets
+
 // a copy of a uniform float in a vector register
 __device__ __forceinline__ float in_vgpr(float x) {
   float y;
@@ -94,9 +96,11 @@ __device__ __forceinline__ int32_t wrapt(int32_t v, int32_t n) {
 // MODE 2: the fly() calls only -- the previous window was relaxed before the
 // launch by the colour-ordered cascade (one launch per colour class), so the
 // tile reads the snapshot and masters as they are.
-template <int SX, int SY, int NT, int WPE, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(StepArgs a) {
-  constexpr bool RELAX_ONLY = MODE == 1, EXT = MODE == 2;
+// MODE 3, 4 (k_colour_step below): as 0 and 1 with the colour-ordered
+// cascade run inside the tile.
+template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
+__device__ __forceinline__ void step_body(const StepArgs& a) {
+  constexpr bool RELAX_ONLY = MODE == 1 || MODE == 4, EXT = MODE == 2, COLOUR = MODE >= 3;
   constexpr int kSX = SX, kSY = SY;
   constexpr int kH3X = kSX + 6, kH3Y = kSY + 6;  // snapshot halo 3
   constexpr int kH2X = kSX + 4, kH2Y = kSY + 4;  // events halo 2
@@ -110,7 +114,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       4 * kH3X * kH3Y * (LAYERS == 2 ? 2 : 1) + 4 * kH2X * kH2Y + 8 * kH1X * kH1Y + 2 * kH2X * kH2Y;
   constexpr int kMarchBytes = 8 * kCell * (LAYERS == 2 ? 2 : 1) + 4 * kCell + (TRACK ? 32 * kCell : 0);
   constexpr int kWorkBytes = kRelaxBytes > kMarchBytes ? kRelaxBytes : kMarchBytes;
-  __shared__ __attribute__((aligned(16))) unsigned char s_work[kWorkBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char s_static[COLOUR ? 16 : kWorkBytes];
+  unsigned char* s_work = COLOUR ? s_dyn : s_static;
   __shared__ uint32_t s_slot[9];     // particles sent in direction d
   __shared__ int64_t s_rbase[9];     // arrivals: sub-range d of the source tile
   __shared__ uint32_t s_rpre[10];    // exclusive prefix of the sub-range lengths
@@ -118,6 +123,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   __shared__ uint64_t s_wstat[kStepThreads / 64];  // per wave: far moves << 32 | steps
   __shared__ int64_t s_base;
   __shared__ uint32_t s_ncas;        // cells whose cascade moves material
+  __shared__ uint32_t s_ccnt[COLOUR ? 32 : 1];  // visited cells per colour class
+  __shared__ uint32_t s_cpre[COLOUR ? 33 : 1];  // exclusive prefix of s_ccnt
+  __shared__ uint32_t s_more[2];                // a cell is still waiting (by round parity)
 
   // XCD-aware order (workgroup b runs on XCD b % 8).  tile_order 0: XCD k
   // takes a contiguous range of tiles, so neighbouring tiles share halo
@@ -224,6 +232,46 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 
   PRec rec0{};       // this thread's first arrival (loaded in the relax phase)
   uint32_t sr0 = 0;  // its sub-range
+  // arrivals of this window: the source tile in direction -d of this one
+  // wrote the particles that moved by d into its sub-range d
+  auto load_arrivals = [&]() __attribute__((always_inline)) {
+    if (threadIdx.x < 9) {
+      const int32_t d = threadIdx.x, dx = d / 3 - 1, dy = d % 3 - 1;
+      int32_t sx = tx - dx, sy = ty - dy;
+      bool ok = !RELAX_ONLY;
+      if (PERIODIC) {
+        sx = wrapt(sx, tiles_x);
+        sy = wrapt(sy, tiles_y);
+      } else {
+        ok = ok && sx >= 0 && sy >= 0 && sx < tiles_x && sy < tiles_y;
+      }
+      int64_t rb = 0;
+      uint32_t rc = 0;
+      if (ok) {
+        const int64_t s9 = (int64_t)(t0 + sx * tiles_y + sy) * 9 + d;
+        rb = a.sub_base_prev[s9];
+        rc = a.sub_cnt_prev[s9];
+      }
+      s_rbase[d] = rb;
+      s_slot[d] = rc;  // lengths, turned into s_rpre by prefix_arrivals
+    }
+  };
+  auto prefix_arrivals = [&]() __attribute__((always_inline)) {
+    if (threadIdx.x == 0) {
+      uint32_t r = 0;
+      for (int d = 0; d < 9; d++) {
+        s_rpre[d] = r;
+        r += s_slot[d];
+      }
+      s_rpre[9] = r;
+    }
+  };
+  auto first_arrival = [&]() __attribute__((always_inline)) {
+    if (threadIdx.x < s_rpre[9]) {
+      while (sr0 < 8 && threadIdx.x >= s_rpre[sr0 + 1]) sr0++;
+      rec0 = a.in[s_rbase[sr0] + (int64_t)(threadIdx.x - s_rpre[sr0])];
+    }
+  };
   if constexpr (EXT) {
     // ---------------- 1'. the relaxed map of the previous window ----------------
     // one-halo snapshot into LDS for the particles' stencils, the tile's
@@ -255,26 +303,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       zt[i] = ok ? zm_in[g] : 0;
       if (LAYERS == 2) st[i] = ok ? sm_in[g] : 0;
     }
-    if (threadIdx.x < 9) {
-      const int32_t d = threadIdx.x, dx = d / 3 - 1, dy = d % 3 - 1;
-      int32_t sx = tx - dx, sy = ty - dy;
-      bool ok = true;
-      if (PERIODIC) {
-        sx = wrapt(sx, tiles_x);
-        sy = wrapt(sy, tiles_y);
-      } else {
-        ok = sx >= 0 && sy >= 0 && sx < tiles_x && sy < tiles_y;
-      }
-      int64_t rb = 0;
-      uint32_t rc = 0;
-      if (ok) {
-        const int64_t s9 = (int64_t)(t0 + sx * tiles_y + sy) * 9 + d;
-        rb = a.sub_base_prev[s9];
-        rc = a.sub_cnt_prev[s9];
-      }
-      s_rbase[d] = rb;
-      s_slot[d] = rc;
-    }
+    load_arrivals();
     int64_t* acc_z = (int64_t*)s_work;
 #pragma unroll
     for (int i = 0; i < kH1Per; i++) {
@@ -293,19 +322,264 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t r = 0;
-      for (int d = 0; d < 9; d++) {
-        s_rpre[d] = r;
-        r += s_slot[d];
+    prefix_arrivals();
+    __syncthreads();
+    first_arrival();
+  } else if constexpr (COLOUR) {
+  // ---------------- 1''. colour-ordered relax of the previous window ----------------
+  // The masters (with the previous window's pickups) of the tile and the
+  // halo its result depends on, in LDS; every visited cell's cascade there
+  // runs on them in class order.
+  {
+    // a tile whose widest halo meets a cell of the classes past 2 (the last
+    // n mod 3 cells of a periodic axis) takes that halo, any other the
+    // interior one (swe_step.h: kColourHalo, colour_halo)
+    ColourHalo hl = kColourHalo;
+    const int32_t limx = PERIODIC ? nx - nx % 3 : nx, limy = PERIODIC ? ny - ny % 3 : ny;
+    if (PERIODIC) {
+      const ColourHalo w = a.chalo;
+      const bool sx = limx != nx && (x0 - w.xl < 0 || x0 + kSX + w.xh > limx);
+      const bool sy = limy != ny && (y0 - w.yl < 0 || y0 + kSY + w.yh > limy);
+      if (sx || sy) hl = w;
+    }
+    const int32_t RX = kSX + hl.xl + hl.xh, RY = kSY + hl.yl + hl.yh, R = RX * RY;
+    const float rcp_ry = 1.0f / (float)RY;
+    int64_t* z_r = (int64_t*)s_work;
+    int64_t* s_r = z_r + R;  // LAYERS == 2
+    uint32_t* v_r = (uint32_t*)(z_r + R * LAYERS);
+    uint16_t* list = (uint16_t*)(v_r + R);
+    // class of a visited cell whose cascade has not run yet (1 ..), else 0;
+    // one row and two cells of zeros before and after it, so that the 5 x 5
+    // neighbourhood of any listed cell can be read
+    uint8_t* cls = (uint8_t*)(list + R) + RY + 2;
+    if (threadIdx.x < 32) s_ccnt[threadIdx.x] = 0;
+    if (threadIdx.x < 2) s_more[threadIdx.x] = 0;
+    for (int32_t e = threadIdx.x; e < RY + 2; e += kStepThreads) {
+      cls[e - RY - 2] = 0;
+      cls[R + e] = 0;
+    }
+    // region cell of index e (e < 2^16: the product is within 1/2 of a step of exact)
+    auto row_of = [=](int32_t e) __attribute__((always_inline)) {
+      return (int32_t)(((float)e + 0.5f) * rcp_ry);
+    };
+    constexpr int kMaxR = (kSX + kColourHaloMax.xl + kColourHaloMax.xh) * (kSY + kColourHaloMax.yl + kColourHaloMax.yh);
+    constexpr int kRPer = (kMaxR + kStepThreads - 1) / kStepThreads;
+    constexpr int kB = 4;  // cells a thread loads at once
+    uint32_t where[kRPer];  // class << 16 | rank within it; 0: not listed
+    __syncthreads();
+#pragma unroll
+    for (int b0 = 0; b0 < kRPer; b0 += 2 * kB) {
+      int64_t zv[2 * kB], sv[LAYERS == 2 ? 2 * kB : 1];
+      uint32_t vv[2 * kB];
+      int32_t cv[2 * kB];
+#pragma unroll
+      for (int j = 0; j < 2 * kB; j++) {
+        const int i = b0 + j;
+        if (i >= kRPer) continue;
+        const int32_t e = (int32_t)threadIdx.x + i * kStepThreads;
+        zv[j] = 0;
+        if (LAYERS == 2) sv[j] = 0;
+        vv[j] = 0;
+        cv[j] = 0;
+        if (e >= R) continue;
+        const int32_t lx = row_of(e), ly = e - lx * RY;
+        int32_t gx = x0 - hl.xl + lx, gy = y0 - hl.yl + ly;
+        bool ok = true;
+        if (PERIODIC) {
+          gx = wrap(gx, nx, rcp_nx);
+          gy = wrap(gy, ny, rcp_ny);
+        } else {
+          ok = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
+        }
+        if (!ok) continue;
+        const int64_t g = (int64_t)gx * ny + gy;
+        zv[j] = zm_in[g];
+        if (LAYERS == 2) sv[j] = sm_in[g];
+        // the outermost ring only lends its values
+        if (lx >= 1 && ly >= 1 && lx < RX - 1 && ly < RY - 1) {
+          vv[j] = v_in[g];
+          const int32_t ccx = gx < limx ? gx % 3 : 3 + gx - limx, ccy = gy < limy ? gy % 3 : 3 + gy - limy;
+          cv[j] = ccx * kColourAxisMax + ccy + 1;
+        }
       }
-      s_rpre[9] = r;
+      if (b0 == 0) load_arrivals();
+#pragma unroll
+      for (int j = 0; j < 2 * kB; j++) {
+        const int i = b0 + j;
+        if (i >= kRPer) continue;
+        const int32_t e = (int32_t)threadIdx.x + i * kStepThreads;
+        const bool in = e < R, act = in && vv[j] != 0;
+        if (in) {
+          z_r[e] = zv[j];
+          if (LAYERS == 2) s_r[e] = sv[j];
+          v_r[e] = vv[j];
+          cls[e] = (uint8_t)(act ? cv[j] : 0);
+        }
+        // rank within the class: one counter update per wave and class
+        where[i] = 0;
+        uint64_t rem = __ballot(act);
+        while (rem) {
+          const int32_t l = __builtin_ctzll(rem);
+          const int32_t c = __builtin_amdgcn_readlane(cv[j], l);
+          const uint64_t m = __ballot(act && cv[j] == c);
+          uint32_t base = 0;
+          if ((int32_t)(threadIdx.x & 63) == l) base = atomicAdd(&s_ccnt[c], (uint32_t)__popcll(m));
+          base = __builtin_amdgcn_readlane(base, l);
+          if (act && cv[j] == c)
+            where[i] = (uint32_t)c << 16 |
+                       (base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)));
+          rem &= ~m;
+        }
+      }
     }
     __syncthreads();
-    if (threadIdx.x < s_rpre[9]) {
-      while (sr0 < 8 && threadIdx.x >= s_rpre[sr0 + 1]) sr0++;
-      rec0 = a.in[s_rbase[sr0] + (int64_t)(threadIdx.x - s_rpre[sr0])];
+    prefix_arrivals();
+    if (threadIdx.x >= kStepThreads - 64) {  // the last wave: prefix over the classes
+      const int32_t l = (int32_t)threadIdx.x & 63;
+      const uint32_t v = l < 32 ? s_ccnt[l] : 0u;
+      uint32_t t = v;
+#pragma unroll
+      for (int off = 1; off < 32; off <<= 1) {
+        const uint32_t y = __shfl_up(t, off, 64);
+        if (l >= off) t += y;
+      }
+      if (l < 32) s_cpre[l] = t - v;
+      if (l == 31) s_cpre[32] = t;
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kRPer; i++)
+      if (where[i]) list[s_cpre[where[i] >> 16] + (where[i] & 0xffffu)] = (uint16_t)(threadIdx.x + i * kStepThreads);
+    const uint32_t nvis = s_cpre[32];
+    if (!RELAX_ONLY) first_arrival();
+    __syncthreads();
+
+    // one cell's cascade on the LDS masters
+    auto relax = [&](int32_t e) __attribute__((always_inline)) {
+      const int32_t lx = row_of(e), ly = e - lx * RY;
+      const int32_t gx = x0 - hl.xl + lx, gy = y0 - hl.yl + ly;
+      const float hc = f32_from_fx(z_r[e]);
+      float hn[8];
+      uint32_t valid = 0;
+      bool act = false;
+      const float dd = __builtin_sqrtf(2.0f);
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        hn[k] = f32_from_fx(z_r[e + c_ox[k] * RY + c_oy[k]]);
+        bool ok = true;
+        if (!PERIODIC) {
+          const int32_t qx = gx + c_ox[k], qy = gy + c_oy[k];
+          ok = qx >= 0 && qy >= 0 && qx < nx && qy < ny;
+        }
+        valid |= (ok ? 1u : 0u) << k;
+        const float diff = hc - hn[k];
+        const float d = (c_ox[k] != 0 && c_oy[k] != 0) ? dd : 1.0f;
+        const float excess = __builtin_fabsf(diff) - (d * a.maxdiff) * 1.0f;
+        act = act || (ok && diff != 0.0f && !(excess <= 0.0f));
+      }
+      if (!act) return;  // no neighbour beyond the threshold: the walk moves nothing
+      const auto sed_of = [&](int32_t k) { return f32_from_fx(s_r[e + off_x(k) * RY + off_y(k)]); };
+      int64_t centre = 0;
+      cascade_cell_dev<LAYERS>(hn, sed_of, hc, LAYERS == 2 ? f32_from_fx(s_r[e]) : 0.0f, valid,
+                               settle_factor_dev(a.settling, v_r[e]), a.maxdiff, [&](int32_t k, int64_t amt) {
+                                 centre -= amt;
+                                 const int32_t q = e + off_x(k) * RY + off_y(k);
+                                 z_r[q] += amt;
+                                 if (LAYERS == 2) s_r[q] += amt;
+                               });
+      z_r[e] += centre;
+      if (LAYERS == 2) s_r[e] += centre;
+    };
+    // Few visited cells (at most one a thread): each thread holds one and runs
+    // its cascade as soon as no visited cell of an earlier class within two
+    // cells is waiting (cells further apart share no neighbour, and of two
+    // closer ones the earlier class goes first).  Dependences run down the
+    // classes, so at most as many rounds as classes; scattered cells need
+    // two or three.  Many: one class after another, a thread a cell.
+    const bool few = nvis <= (uint32_t)kStepThreads;
+    bool pend = few && threadIdx.x < nvis;
+    const int32_t own = pend ? list[threadIdx.x] : 0;
+    const uint8_t own_cls = pend ? cls[own] : 0;
+    int32_t c = 0;               // class of the current chunk (many)
+    uint32_t pos = 0, end = 0;   // its unread part of the list
+    for (int32_t round = 0; !few || round < kColourAxisMax * kColourAxisMax; round++) {
+      int32_t e = -1;
+      if (few) {
+        if (pend) {
+          const uint8_t* p = cls + own;
+          bool ready = true;
+#pragma unroll
+          for (int dx = -2; dx <= 2; dx++)
+#pragma unroll
+            for (int dy = -2; dy <= 2; dy++) {
+              if (dx == 0 && dy == 0) continue;
+              const uint8_t o = p[dx * RY + dy];
+              ready = ready && (o == 0 || o >= own_cls);
+            }
+          if (ready) e = own;
+        }
+        if (threadIdx.x == 0) s_more[round & 1] = 0;
+        __syncthreads();
+      } else {
+        while (pos >= end && c < kColourAxisMax * kColourAxisMax) {
+          c++;
+          pos = s_cpre[c];
+          end = pos + s_ccnt[c];
+        }
+        if (pos >= end) break;
+        if (pos + threadIdx.x < end) e = list[pos + threadIdx.x];
+        pos += kStepThreads;
+      }
+      if (e >= 0) relax(e);
+      if (few) {
+        if (e >= 0) {
+          cls[e] = 0;
+          pend = false;
+        }
+        if (pend) s_more[round & 1] = 1;
+      }
+      __syncthreads();
+      if (few && s_more[round & 1] == 0) break;
+    }
+
+    // the relaxed masters of the tile and its one-cell halo; the sediment
+    // layer clamped at zero after the last class
+    constexpr int kH1Per = (kH1X * kH1Y + kStepThreads - 1) / kStepThreads;
+    int64_t zt[kH1Per], st[LAYERS == 2 ? kH1Per : 1];
+#pragma unroll
+    for (int i = 0; i < kH1Per; i++) {
+      const int e = threadIdx.x + i * kStepThreads;
+      zt[i] = 0;
+      if (LAYERS == 2) st[i] = 0;
+      if (e >= kH1X * kH1Y) continue;
+      const int32_t q = (hl.xl - 1 + e / kH1Y) * RY + hl.yl - 1 + e % kH1Y;
+      zt[i] = z_r[q];
+      if (LAYERS == 2) st[i] = s_r[q] < 0 ? 0 : s_r[q];
+    }
+    __syncthreads();
+    int64_t* acc_z = (int64_t*)s_work;
+#pragma unroll
+    for (int i = 0; i < kH1Per; i++) {
+      const int e = threadIdx.x + i * kStepThreads;
+      if (e >= kH1X * kH1Y) continue;
+      const int32_t lx = e / kH1Y, ly = e % kH1Y;
+      const float zf = f32_from_fx(zt[i]);
+      s_new[e] = zf;  // cells off a bounded map hold 0
+      const bool mine = lx >= 1 && ly >= 1 && lx <= kSX && ly <= kSY;
+      const int32_t gx = x0 - 1 + lx, gy = y0 - 1 + ly, li = (lx - 1) * kSY + (ly - 1);
+      const bool on = mine && gx < nx && gy < ny;
+      const int64_t g = (int64_t)gx * ny + gy;
+      if (mine) acc_z[li] = zt[i];
+      if (RELAX_ONLY && on) snap_out[g] = zf;  // the cycle's last window leaves the snapshot
+      if (LAYERS == 2) {
+        const float sf = f32_from_fx(st[i]);
+        s_snew[e] = sf;
+        if (mine) acc_z[kCell + li] = st[i];
+        if (RELAX_ONLY && on) ssnap_out[g] = sf;
+      }
+    }
+    __syncthreads();
+  }
   } else {
   // ---------------- 1. relax of the previous window ----------------
   {
@@ -366,29 +640,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
       }
       vv[i] = ok ? v_in[(int64_t)gx * ny + gy] : 0u;
     }
-    // arrivals of this window: the source tile in direction -d of this one
-    // wrote the particles that moved by d into its sub-range d (loaded after
-    // the map loads are out, so that their wait overlaps those)
-    if (threadIdx.x < 9) {
-      const int32_t d = threadIdx.x, dx = d / 3 - 1, dy = d % 3 - 1;
-      int32_t sx = tx - dx, sy = ty - dy;
-      bool ok = !RELAX_ONLY;
-      if (PERIODIC) {
-        sx = wrapt(sx, tiles_x);
-        sy = wrapt(sy, tiles_y);
-      } else {
-        ok = ok && sx >= 0 && sy >= 0 && sx < tiles_x && sy < tiles_y;
-      }
-      int64_t rb = 0;
-      uint32_t rc = 0;
-      if (ok) {
-        const int64_t s9 = (int64_t)(t0 + sx * tiles_y + sy) * 9 + d;
-        rb = a.sub_base_prev[s9];
-        rc = a.sub_cnt_prev[s9];
-      }
-      s_rbase[d] = rb;
-      s_slot[d] = rc;  // lengths, turned into s_rpre below
-    }
+    // loaded after the map loads are out, so that their wait overlaps those
+    load_arrivals();
 #pragma unroll
     for (int i = 0; i < kH3Per; i++) {
       const int e = threadIdx.x + i * kStepThreads;
@@ -408,14 +661,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     __syncthreads();
     // start of each arrival sub-range in this tile's arrival order (read
     // after the next barrier)
-    if (threadIdx.x == 0) {
-      uint32_t r = 0;
-      for (int d = 0; d < 9; d++) {
-        s_rpre[d] = r;
-        r += s_slot[d];
-      }
-      s_rpre[9] = r;
-    }
+    prefix_arrivals();
 
     // visited cells within two cells of the tile whose cascade moves
     // material: one neighbour beyond the threshold at the window's start
@@ -488,10 +734,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     }
     // each thread's first arrival record, loaded now so that it arrives
     // while the other threads finish their cascades and the relax ends
-    if (!RELAX_ONLY && threadIdx.x < s_rpre[9]) {
-      while (sr0 < 8 && threadIdx.x >= s_rpre[sr0 + 1]) sr0++;
-      rec0 = a.in[s_rbase[sr0] + (int64_t)(threadIdx.x - s_rpre[sr0])];
-    }
+    if (!RELAX_ONLY) first_arrival();
     __syncthreads();
 
     // master += cascade; next snapshot for the tile and its halo.  The
@@ -887,6 +1130,36 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
   }
 }
 
+template <int SX, int SY, int NT, int WPE, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(StepArgs a) {
+  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>(a);
+}
+
+// The colour-ordered cascade in the same single launch per window: the tile
+// re-runs every cascade its cells (and their one-cell halo) depend on from
+// an LDS copy of the masters, instead of one launch per class over the map
+// (9 to 25 launches, each two memory round trips: 7.5 us apiece on 512^2).
+// Redundant work is 3.4 regions per tile, but a window pays one launch and
+// one load of the region; its time is the most crowded tile's rounds of
+// dependent cascades.  Measured against the class launches: 512^2 bounded,
+// 4096 particles 46.2 -> 17.5 ms a cycle; 400 x 301 periodic, two layers,
+// 30,000 particles 85.5 -> 35.9 ms; 1024^2 with a million particles, where a
+// class launch fills the chip, 110 -> 111 ms.
+template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colour_step(StepArgs a) {
+  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>(a);
+}
+
+// dynamic LDS of k_colour_step: the region's masters, events, list and
+// classes, or the march's accumulators
+template <int SX, int SY>
+inline size_t colour_lds(const ColourHalo& h, bool track, int layers) {
+  const size_t ry = (size_t)(SY + h.yl + h.yh), r = (size_t)(SX + h.xl + h.xh) * ry;
+  const size_t relax = r * (8 * (size_t)layers + 4 + 2 + 1) + 2 * (ry + 2);
+  const size_t march = (size_t)SX * SY * (8 * (size_t)layers + 4 + (track ? 32 : 0));
+  return ((relax > march ? relax : march) + 15) & ~(size_t)15;
+}
+
 // ---------------------------------------------------------------------------
 // Launchers of one shape (instantiated per shape in swe_step_shapes.hip)
 // ---------------------------------------------------------------------------
@@ -895,7 +1168,18 @@ struct StepLauncher {
   template <bool P, bool T, int L, bool D>
   static void step4(const StepArgs& a, int mode, hipStream_t s) {
     const unsigned g = (unsigned)(a.heavy_slots + a.default_slots + a.light_slots);
-    if (mode == 1)
+    if (mode >= 3) {
+      ColourHalo h = kColourHalo;  // the larger of the launch's two regions
+      h.xl = a.chalo.xl > h.xl ? a.chalo.xl : h.xl;
+      h.xh = a.chalo.xh > h.xh ? a.chalo.xh : h.xh;
+      h.yl = a.chalo.yl > h.yl ? a.chalo.yl : h.yl;
+      h.yh = a.chalo.yh > h.yh ? a.chalo.yh : h.yh;
+      const unsigned lds = (unsigned)colour_lds<SX, SY>(h, T, L);
+      if (mode == 3)
+        hipLaunchKernelGGL((k_colour_step<SX, SY, NT, P, T, L, D, 3>), dim3(g), dim3(NT), lds, s, a);
+      else
+        hipLaunchKernelGGL((k_colour_step<SX, SY, NT, P, T, L, D, 4>), dim3(g), dim3(NT), lds, s, a);
+    } else if (mode == 1)
       hipLaunchKernelGGL((k_step<SX, SY, NT, WPE, P, T, L, D, 1>), dim3(g), dim3(NT), 0, s, a);
     else if (mode == 2)
       hipLaunchKernelGGL((k_step<SX, SY, NT, WPE, P, T, L, D, 2>), dim3(g), dim3(NT), 0, s, a);
