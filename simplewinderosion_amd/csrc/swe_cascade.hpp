@@ -29,18 +29,21 @@ __device__ __forceinline__ int32_t off_y(int32_t k) { return (int32_t)((kOffYPac
 
 // Sort key of a neighbour: descending order of the key is descending height,
 // ties in ascending offset order -- the order the stable insertion sort of
-// world.hpp:118-120 leaves eight elements in.  The height bits are mapped to
-// an unsigned integer of the same order (-0 first folded into +0, which the
-// float comparison treats as equal); map heights are finite.  Out-of-map
-// neighbours get key 0, below every in-map key.
-__device__ __forceinline__ uint64_t cascade_key(float h, int32_t k, bool valid) {
-  const uint32_t u = f2u(h + 0.0f);
-  const uint32_t o = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-  return valid ? (((uint64_t)o << 32) | (uint32_t)(7 - k)) : 0ull;
+// world.hpp:118-120 leaves eight elements in.  The key is the height as a
+// float64 (exact; -0 first folded into +0, which the float comparison treats
+// as equal) with the offset in the three lowest of its 29 spare bits, so
+// that a compare-exchange is one v_max_f64 and one v_min_f64.  Those bits
+// grow the magnitude, so a negative height holds k and a positive 7 - k;
+// rounding the key to float32 gives the height back.  Map heights are
+// finite; out-of-map neighbours get -infinity.
+__device__ __forceinline__ double cascade_key(float h, int32_t k, bool valid) {
+  const float z = h + 0.0f;
+  const uint64_t u = (uint64_t)__double_as_longlong((double)z) | (uint32_t)(z < 0.0f ? k : 7 - k);
+  return valid ? __longlong_as_double((long long)u) : -__builtin_inf();
 }
-__device__ __forceinline__ float cascade_key_height(uint64_t key) {
-  const uint32_t o = (uint32_t)(key >> 32);
-  return u2f((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+__device__ __forceinline__ int32_t cascade_key_offset(double key) {
+  const int32_t lo = (int32_t)(__double_as_longlong(key) & 7);
+  return key < 0.0 ? lo : 7 - lo;
 }
 
 // One cell's cascade of the window: World::cascade (world.hpp:79-153)
@@ -54,15 +57,14 @@ __device__ __forceinline__ float cascade_key_height(uint64_t key) {
 template <int LAYERS, class SedOf, class Emit>
 __device__ __forceinline__ void cascade_cell_dev(const float hn[8], const SedOf& sed_of, float hc, float sc,
                                                  uint32_t validmask, float settling, float maxdiff, Emit&& emit) {
-  uint64_t key[8];
+  double key[8];
 #pragma unroll
   for (int k = 0; k < 8; k++) key[k] = cascade_key(hn[k], k, (validmask >> k) & 1u);
-#define SWE_CAS(i, j)                        \
-  {                                          \
-    const uint64_t a = key[i], b = key[j];   \
-    const bool sw = b > a;                   \
-    key[i] = sw ? b : a;                     \
-    key[j] = sw ? a : b;                     \
+#define SWE_CAS(i, j)                      \
+  {                                        \
+    const double a = key[i], b = key[j];   \
+    key[i] = __builtin_fmax(a, b);         \
+    key[j] = __builtin_fmin(a, b);         \
   }
   SWE_CAS(0, 2) SWE_CAS(1, 3) SWE_CAS(4, 6) SWE_CAS(5, 7)
   SWE_CAS(0, 4) SWE_CAS(1, 5) SWE_CAS(2, 6) SWE_CAS(3, 7)
@@ -74,9 +76,9 @@ __device__ __forceinline__ void cascade_cell_dev(const float hn[8], const SedOf&
   const float dd = __builtin_sqrtf(2.0f);
 #pragma unroll
   for (int r = 0; r < 8; r++) {
-    if (key[r] == 0ull) break;  // the out-of-map neighbours come last
-    const int32_t k = 7 - (int32_t)(key[r] & 7u);
-    const float diff = hc - cascade_key_height(key[r]);
+    if (key[r] == -__builtin_inf()) break;  // the out-of-map neighbours come last
+    const int32_t k = cascade_key_offset(key[r]);
+    const float diff = hc - (float)key[r];
     const float d = ((kDiagMask >> k) & 1u) ? dd : 1.0f;
     const float excess = __builtin_fabsf(diff) - (d * maxdiff) * 1.0f;
     float t = settling * excess / 2.0f;

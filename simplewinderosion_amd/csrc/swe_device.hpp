@@ -20,43 +20,19 @@ namespace swe {
 __device__ __forceinline__ float u2f(uint32_t u) { return __uint_as_float(u); }
 __device__ __forceinline__ uint32_t f2u(float f) { return __float_as_uint(f); }
 
-// round_half_even(v * 2^32), computed on the IEEE encoding. NaN -> 0,
-// overflow saturates.  The general (slow) form; fx_from_f32 below takes it
-// only for |v| >= 2^31 and NaN.
-__device__ __forceinline__ int64_t fx_from_f32_bits(float v) {
-  const uint32_t u = f2u(v);
-  const uint32_t e = (u >> 23) & 0xffu;
-  const uint64_t sgn = u >> 31;
-  if (e == 0xffu) {
-    if (u & 0x7fffffu) return 0;
-    return sgn ? INT64_MIN : INT64_MAX;
-  }
-  if (e == 0) return 0;
-  const uint64_t m = (u & 0x7fffffu) | 0x800000u;
-  const int sh = (int)e - 118;
-  uint64_t r;
-  if (sh >= 0) {
-    if (sh > 39) return sgn ? INT64_MIN : INT64_MAX;
-    r = m << sh;
-    if (r > (uint64_t)INT64_MAX) return sgn ? INT64_MIN : INT64_MAX;
-  } else {
-    const int k = -sh;
-    if (k > 25) return 0;
-    const uint64_t q = m >> k;
-    const uint64_t rem = m & ((1ull << k) - 1ull);
-    const uint64_t half = 1ull << (k - 1);
-    r = q + ((rem > half || (rem == half && (q & 1ull))) ? 1ull : 0ull);
-  }
-  return sgn ? -(int64_t)r : (int64_t)r;
-}
-
-// Same result for every input: for |v| < 2^31, v * 2^32 is exact and below
-// 2^63, rint rounds it half-to-even to an integral float, and the integral
-// float converts to int64 exactly (denormal v give 0 either way).
+// round_half_even(v * 2^32) as int64; NaN -> 0, |v| >= 2^31 saturates.
+// Below 2^18 the product is formed exactly in float64 (a power-of-two scale
+// of v) and 1.5 * 2^52 added: that sum's last bit is worth 1, so the addition
+// rounds to an integer, ties to even, and the integer is the sum's encoding
+// minus the constant's -- four instructions in place of the fourteen of a
+// float -> int64 conversion.
 __device__ __forceinline__ int64_t fx_from_f32(float v) {
-  if (__builtin_expect(__builtin_fabsf(v) < 2147483648.0f, 1))
-    return (int64_t)__builtin_rintf(v * 4294967296.0f);
-  return fx_from_f32_bits(v);
+  if (__builtin_expect(__builtin_fabsf(v) < 262144.0f, 1)) {
+    const double d = (double)(v * 4294967296.0f) + 6755399441055744.0;
+    return (int64_t)((uint64_t)__double_as_longlong(d) - 0x4338000000000000ull);
+  }
+  if (!(__builtin_fabsf(v) < 2147483648.0f)) return v != v ? 0 : (v < 0.0f ? INT64_MIN : INT64_MAX);
+  return (int64_t)(v * 4294967296.0f);  // a float of 2^18 or more is a multiple of 2^-5
 }
 
 // round_half_even(m * 2^-32) to float32: the int64 -> float32 conversion
@@ -64,36 +40,11 @@ __device__ __forceinline__ int64_t fx_from_f32(float v) {
 // keeps the result far from the denormal range).
 __device__ __forceinline__ float f32_from_fx(int64_t m) { return (float)m * 2.3283064365386963e-10f; }
 
-// The same by integer operations (reference form of f32_from_fx).
-__device__ __forceinline__ float f32_from_fx_bits(int64_t m) {
-  if (m == 0) return 0.0f;
-  const bool neg = m < 0;
-  const uint64_t a = neg ? (uint64_t)0 - (uint64_t)m : (uint64_t)m;
-  const int msb = 63 - __clzll((long long)a);
-  uint64_t q;
-  int ex;
-  if (msb <= 23) {
-    q = a;
-    ex = -32;
-  } else {
-    const int k = msb - 23;
-    q = a >> k;
-    const uint64_t rem = a & ((1ull << k) - 1ull);
-    const uint64_t half = 1ull << (k - 1);
-    if (rem > half || (rem == half && (q & 1ull))) q += 1;
-    ex = k - 32;
-  }
-  const float r = (float)(uint32_t)q * u2f((uint32_t)(ex + 127) << 23);
-  return neg ? -r : r;
-}
-
 // exp for float32: Cody-Waite reduction with a two-part ln2, degree-7
-// Taylor polynomial in Horner form, exact power-of-two scaling (two steps
-// below 2^-125).
+// Taylor polynomial in Horner form, exact power-of-two scaling (two steps,
+// the first by 1 except below 2^-125).  The special cases are selected at
+// the end, without branches.
 __device__ __forceinline__ float exp_f32(float x) {
-  if (x != x) return x;
-  if (x > 88.72283935546875f) return u2f(0x7f800000u);
-  if (x < -104.0f) return 0.0f;
   const float log2e = 1.44269502162933349609375f;
   const float ln2_hi = 0.693145751953125f;
   const float ln2_lo = 1.428606765330187045e-06f;
@@ -107,12 +58,38 @@ __device__ __forceinline__ float exp_f32(float x) {
   p = p * r + 0.5f;
   p = p * r + 1.0f;
   p = p * r + 1.0f;
-  int k = (int)kf;
-  if (k < -125) {
-    p = p * u2f((uint32_t)(127 - 64) << 23);
-    k += 64;
+  const int k = (int)kf;
+  const int k1 = k < -125 ? -64 : 0;
+  p = p * u2f((uint32_t)(127 + k1) << 23);
+  p = p * u2f((uint32_t)(k - k1 + 127) << 23);
+  p = x < -104.0f ? 0.0f : p;
+  p = x > 88.72283935546875f ? u2f(0x7f800000u) : p;
+  return x != x ? x : p;
+}
+
+// s = sqrt(d) and r = 1 / s, both correctly rounded.  In the normal range one
+// v_rsq_f32 seeds the coupled iteration g -> sqrt, h -> 1 / (2 sqrt), whose final
+// residual rounds s; one residual step from v_rcp_f32 rounds r (from 2h in
+// its place 450 of the range's quotients come out one ulp low, at s with all
+// mantissa bits set).  Equal to the IEEE square root and quotient for every
+// float in the range, checked exhaustively on the device: 13 instructions in
+// place of 26.  Zero, tiny, huge, negative and NaN take the IEEE operations.
+struct Root {
+  float s, r;
+};
+__device__ __forceinline__ Root root_of(float d) {
+  if (__builtin_expect(d >= 0x1p-90f && d <= 0x1p90f, 1)) {
+    const float y = __builtin_amdgcn_rsqf(d);
+    float g = d * y, h = 0.5f * y;
+    const float e = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    h = __builtin_fmaf(h, e, h);
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, d), h, g);
+    const float z = __builtin_amdgcn_rcpf(s);
+    return Root{s, __builtin_fmaf(__builtin_fmaf(-s, z, 1.0f), z, z)};
   }
-  return p * u2f((uint32_t)(k + 127) << 23);
+  const float s = __builtin_sqrtf(d);
+  return Root{s, 1.0f / s};
 }
 
 // ---------------------------------------------------------------------------
@@ -151,8 +128,7 @@ __device__ __forceinline__ float dot(f3 a, f3 b) { return (a.x * b.x + a.y * b.y
 __device__ __forceinline__ f3 cross(f3 a, f3 b) {
   return mk(a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y);
 }
-__device__ __forceinline__ float length(f3 a) { return __builtin_sqrtf(dot(a, a)); }
-__device__ __forceinline__ f3 normalize(f3 a) { return muls(a, 1.0f / __builtin_sqrtf(dot(a, a))); }
+__device__ __forceinline__ f3 normalize(f3 a) { return muls(a, root_of(dot(a, a)).r); }
 __device__ __forceinline__ f3 mix(f3 x, f3 y, float a) { return add(muls(x, 1.0f - a), muls(y, a)); }
 
 // quad::_normal (cellpool.h:200-223) from the five stencil heights.  gNE,
@@ -165,24 +141,28 @@ __device__ __forceinline__ f3 surface_normal(float hp, float hyp, float hxp, flo
   if (g2) n = add(n, cross(mul(s, mk(0.0f, hym - hp, -1.0f)), mul(s, mk(-1.0f, hxm - hp, 0.0f))));
   if (g3) n = add(n, cross(mul(s, mk(1.0f, hxp - hp, 0.0f)), mul(s, mk(0.0f, hym - hp, -1.0f))));
   if (g4) n = add(n, cross(mul(s, mk(-1.0f, hxm - hp, 0.0f)), mul(s, mk(0.0f, hyp - hp, 1.0f))));
-  if (length(n) > 0.0f) n = normalize(n);
+  const Root l = root_of(dot(n, n));
+  if (l.s > 0.0f) n = muls(n, l.r);
   return n;
 }
 
-// Euclidean remainder of v by n (n > 0), exact for all int32 v: a float
-// reciprocal estimate corrected by at most one step, integer fallback for
-// |v| >= 2^23.
+// Euclidean remainder of v by n (n > 0) for |v| <= 2^30: two rounds of a
+// float quotient estimate (the first leaves at most a few hundred multiples
+// of n, the second less than one) and a correction by one step.
 __device__ __forceinline__ int32_t wrap(int32_t v, int32_t n, float rcp_n) {
   if ((uint32_t)v < (uint32_t)n) return v;
-  if (v > -(1 << 23) && v < (1 << 23)) {
-    int32_t q = (int32_t)__builtin_floorf((float)v * rcp_n);
-    int32_t r = v - q * n;
-    if (r < 0) r += n;
-    if (r >= n) r -= n;
-    return r;
-  }
-  int32_t r = v % n;
-  return r < 0 ? r + n : r;
+  int32_t r = v - (int32_t)__builtin_floorf((float)v * rcp_n) * n;
+  r -= (int32_t)__builtin_floorf((float)r * rcp_n) * n;
+  if (r < 0) r += n;
+  if (r >= n) r -= n;
+  return r;
+}
+
+// The same for -n <= v < 2n: as unsigned numbers the wanted one of v, v + n
+// (v - n) is the smaller.
+__device__ __forceinline__ int32_t wrap_near(int32_t v, int32_t n) {
+  const uint32_t a = (uint32_t)v, b = a + (uint32_t)n, c = a < b ? a : b, d = c - (uint32_t)n;
+  return (int32_t)(c < d ? c : d);
 }
 
 }  // namespace swe

@@ -87,6 +87,15 @@ __device__ __forceinline__ bool cell_of(float px, float pz, const FlyConsts& k, 
   return true;
 }
 
+// v % 1001 for v < 2^21, in float: (v + 1/2) / 1001 is at least 1/2002 from
+// an integer and the estimate off by less than 3e-4, so its floor is the
+// quotient; the products are below 2^24, so the remainder is exact (integer
+// multiplies run at a quarter of the rate).
+__device__ __forceinline__ float mod1001(uint32_t v) {
+  const float f = (float)v, c = 1.0f / 1001.0f;
+  return __builtin_fmaf(-1001.0f, __builtin_floorf(__builtin_fmaf(f, c, 0.5f * c)), f);
+}
+
 // One fly() call for a particle whose current cell (cx, cy) is valid.
 // `Map` provides h(dx, dy) -- snapshot height at (cx+dx, cy+dy) for the
 // five-point stencil -- and s0() -- sediment snapshot at the cell.
@@ -146,9 +155,9 @@ __device__ __forceinline__ FlyOutcome fly(Particle& w, uint64_t pk, int32_t cx, 
 
   {  // :83 turbulence, three draws in [0,1000] for this call
     const uint64_t t = mix64(pk + (uint64_t)(call + 3) * kGolden);
-    const float r0 = (float)(int32_t)((t & 0x1fffffull) % 1001ull);
-    const float r1 = (float)(int32_t)(((t >> 21) & 0x1fffffull) % 1001ull);
-    const float r2 = (float)(int32_t)(((t >> 42) & 0x1fffffull) % 1001ull);
+    const float r0 = mod1001((uint32_t)t & 0x1fffffu);
+    const float r1 = mod1001((uint32_t)(t >> 21) & 0x1fffffu);
+    const float r2 = mod1001((uint32_t)(t >> 42) & 0x1fffffu);
     const float kk = 0.1f * hfac * collision;
     const f3 tb = smul(kk, subs(mk(r0, r1, r2), 500.0f));
     sp = add(sp, mk(swe_div500(tb.x), swe_div500(tb.y), swe_div500(tb.z)));
@@ -162,9 +171,10 @@ __device__ __forceinline__ FlyOutcome fly(Particle& w, uint64_t pk, int32_t cx, 
 
   if (TRACK) acc.add_track(cell, w.sed, sp);  // :93-96 on the pre-move cell
 
-  float force = -dot(normalize(sp), n) * length(sp);  // :100-102
+  const Root sr = root_of(dot(sp, sp));
+  float force = -dot(muls(sp, sr.r), n) * sr.s;  // :100-102
   if (force < 0.0f) force = 0.0f;
-  const float lift = (1.0f - collision) * length(sp);  // :104
+  const float lift = (1.0f - collision) * sr.s;  // :104
   const float capacity = force * hfac + 0.02f * lift * hfac;  // :106
 
   const float diff = capacity - w.sed;  // :110-112

@@ -75,18 +75,22 @@ struct TileAcc {
 
 extern __shared__ __attribute__((aligned(16))) unsigned char s_dyn[];  // k_colour_step's working sets
 
-// a copy of a uniform float in a vector register
-__device__ __forceinline__ float in_vgpr(float x) {
-  float y;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(y) : "s"(x));
-  return y;
-}
-
 __device__ __forceinline__ int32_t wrapt(int32_t v, int32_t n) {
   // small-range wrap for tile coordinates (|v| < 2n)
   if (v < 0) v += n;
   if (v >= n) v -= n;
   return v;
+}
+
+// The kernel's arguments, read where they are used: they exceed the scalar
+// registers, and a value loaded at the start and held through the particle
+// loop would be spilled to vector lanes and come back by v_readlane.  Each
+// phase takes the pointer through step_args, which the compiler cannot see
+// through, so its loads are not moved above it.
+typedef const __attribute__((address_space(4))) StepArgs* StepArgsPtr;
+__device__ __forceinline__ StepArgsPtr step_args(StepArgsPtr p) {
+  asm volatile("" : "+s"(p));
+  return p;
 }
 
 // the register budget keeps WPE waves per SIMD (the default shape: five, and
@@ -99,7 +103,8 @@ __device__ __forceinline__ int32_t wrapt(int32_t v, int32_t n) {
 // MODE 3, 4 (k_colour_step below): as 0 and 1 with the colour-ordered
 // cascade run inside the tile.
 template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
-__device__ __forceinline__ void step_body(const StepArgs& a) {
+__device__ __forceinline__ void step_body() {
+  StepArgsPtr ap = step_args((StepArgsPtr)__builtin_amdgcn_kernarg_segment_ptr());
   constexpr bool RELAX_ONLY = MODE == 1 || MODE == 4, EXT = MODE == 2, COLOUR = MODE >= 3;
   constexpr int kSX = SX, kSY = SY;
   constexpr int kH3X = kSX + 6, kH3Y = kSY + 6;  // snapshot halo 3
@@ -111,7 +116,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   __shared__ float s_snew[LAYERS == 2 ? kH1X * kH1Y : 1];
   // relax-phase and march-phase working sets share one buffer
   constexpr int kRelaxBytes =
-      4 * kH3X * kH3Y * (LAYERS == 2 ? 2 : 1) + 4 * kH2X * kH2Y + 8 * kH1X * kH1Y + 2 * kH2X * kH2Y;
+      4 * kH3X * kH3Y * (LAYERS == 2 ? 2 : 1) + 4 * kH2X * kH2Y + 8 * kH1X * kH1Y * (LAYERS == 2 ? 2 : 1) + 2 * kH2X * kH2Y;
   constexpr int kMarchBytes = 8 * kCell * (LAYERS == 2 ? 2 : 1) + 4 * kCell + (TRACK ? 32 * kCell : 0);
   constexpr int kWorkBytes = kRelaxBytes > kMarchBytes ? kRelaxBytes : kMarchBytes;
   __shared__ __attribute__((aligned(16))) unsigned char s_static[COLOUR ? 16 : kWorkBytes];
@@ -119,8 +124,9 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   __shared__ uint32_t s_slot[9];     // particles sent in direction d
   __shared__ int64_t s_rbase[9];     // arrivals: sub-range d of the source tile
   __shared__ uint32_t s_rpre[10];    // exclusive prefix of the sub-range lengths
-  __shared__ int64_t s_lost[kStepThreads / 64];
-  __shared__ uint64_t s_wstat[kStepThreads / 64];  // per wave: far moves << 32 | steps
+  __shared__ int64_t s_part[kStepThreads / 64];
+  __shared__ int64_t s_lost;         // load of the particles that died here
+  __shared__ uint32_t s_far;         // particles that skipped a tile
   __shared__ int64_t s_base;
   __shared__ uint32_t s_ncas;        // cells whose cascade moves material
   __shared__ uint32_t s_ccnt[COLOUR ? 32 : 1];  // visited cells per colour class
@@ -139,57 +145,57 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   // empty slots return at once.  The rest follow the usual order and skip
   // a listed tile.  heavy_slots and default_slots (with light slots) are
   // multiples of 8, so slot b of each part runs on XCD b % 8.
-  const uint32_t hs = RELAX_ONLY ? 0u : (uint32_t)a.heavy_slots;
-  const uint32_t ls = RELAX_ONLY ? 0u : (uint32_t)a.light_slots;
-  const uint32_t nb = (uint32_t)a.default_slots, b = blockIdx.x - (uint32_t)a.heavy_slots;
+  const uint32_t hs = RELAX_ONLY ? 0u : (uint32_t)ap->heavy_slots;
+  const uint32_t ls = RELAX_ONLY ? 0u : (uint32_t)ap->light_slots;
+  const uint32_t nb = (uint32_t)ap->default_slots, b = blockIdx.x - (uint32_t)ap->heavy_slots;
   const uint32_t xcd = b % 8;
   // a single map's terrain record does not depend on the tile: its load goes
   // out with the slot's list or stamp loads below, not after them
-  const Terrain T1 = a.terr[0];
+  const Terrain T1 = ap->terr[0];
   int32_t u;  // global tile
   bool listed = false;
-  if (blockIdx.x < (uint32_t)a.heavy_slots) {
+  if (blockIdx.x < (uint32_t)ap->heavy_slots) {
     const uint32_t k = blockIdx.x / 8;  // heavy slot k of this XCD (blockIdx.x % 8 == xcd)
     if (hs == 0) return;
     // the list entry is read together with the list length (k < hs / 8, so
     // it lies inside the list whatever the length; unused when k >= length)
-    const uint32_t cnt = a.hcnt_cur[xcd];
-    const uint32_t cand = a.heavy_cur[xcd * (hs / 8) + k];
+    const uint32_t cnt = ap->hcnt_cur[xcd];
+    const uint32_t cand = ap->heavy_cur[xcd * (hs / 8) + k];
     if (k >= cnt) return;
     u = (int32_t)cand;
     listed = true;
   } else if (b >= nb) {
     const uint32_t bl = b - nb, k = bl / 8;  // k < ls / 8
     if (ls == 0) return;
-    const uint32_t cnt = a.hcnt_cur[8 + xcd];
-    const uint32_t cand = a.heavy_cur[kHeavySlotsMax + xcd * (ls / 8) + k];
+    const uint32_t cnt = ap->hcnt_cur[8 + xcd];
+    const uint32_t cand = ap->heavy_cur[kHeavySlotsMax + xcd * (ls / 8) + k];
     if (k >= cnt) return;
     u = (int32_t)cand;
     listed = true;
-  } else if (a.tile_order <= 0) {
+  } else if (ap->tile_order <= 0) {
     const uint32_t q8 = nb / 8, r8 = nb % 8;
     u = (int32_t)(xcd * q8 + (xcd < r8 ? xcd : r8) + b / 8);
   } else {
-    const uint32_t C = (uint32_t)a.tile_order, full = nb / (8 * C) * (8 * C), j = b / 8;
+    const uint32_t C = (uint32_t)ap->tile_order, full = nb / (8 * C) * (8 * C), j = b / 8;
     u = b < full ? (int32_t)(((j / C) * 8 + xcd) * C + j % C) : (int32_t)b;
   }
-  if (u >= a.ntiles) return;  // padding of the usual order to a multiple of 8
+  if (u >= ap->ntiles) return;  // padding of the usual order to a multiple of 8
   // home XCD of tile t in the usual order: the XCD whose workgroups take it
-  auto home_of = [=](uint32_t t) __attribute__((always_inline)) -> uint32_t {
-    if (a.tile_order <= 0) {
+  auto home_of = [&](uint32_t t) __attribute__((always_inline)) -> uint32_t {
+    if (ap->tile_order <= 0) {
       const uint32_t q8 = nb / 8, r8 = nb % 8;
       return t < r8 * (q8 + 1) ? t / (q8 + 1) : r8 + (t - r8 * (q8 + 1)) / q8;
     }
-    const uint32_t C = (uint32_t)a.tile_order, full = nb / (8 * C) * (8 * C);
+    const uint32_t C = (uint32_t)ap->tile_order, full = nb / (8 * C) * (8 * C);
     return t < full ? (t / C) % 8 : t % 8;
   };
   // a listed tile's stamp is window + 1 (or window + 2 once its listed
   // workgroup has listed it again): either way the usual one skips it,
   // before it loads anything
-  if ((hs | ls) > 0 && !listed && a.hstamp[u] > (uint32_t)a.window) return;
+  if ((hs | ls) > 0 && !listed && ap->hstamp[u] > (uint32_t)ap->window) return;
   // the terrain this tile belongs to; all map indices below are terrain-local
   Terrain T = T1;
-  if (a.nterr != 1) T = a.terr[a.tile_terrain[u]];
+  if (ap->nterr != 1) T = ap->terr[ap->tile_terrain[u]];
   const int32_t nx = T.nx, ny = T.ny;
   const int32_t tiles_x = T.tiles_x, tiles_y = T.tiles_y;
   const int32_t t0 = T.tile0;
@@ -198,17 +204,21 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   const int32_t x0 = tx * kSX, y0 = ty * kSY;
   const float rcp_nx = T.rcp_nx, rcp_ny = T.rcp_ny;
   const int64_t c0 = T.cell0;
-  const int64_t* zm_in = a.zm_in + c0;
-  int64_t* zm_out = a.zm_out + c0;
-  const float* snap_in = a.snap_in + c0;
-  float* snap_out = a.snap_out + c0;
-  const int64_t* sm_in = LAYERS == 2 ? a.sm_in + c0 : nullptr;
-  int64_t* sm_out = LAYERS == 2 ? a.sm_out + c0 : nullptr;
-  const float* ssnap_in = LAYERS == 2 ? a.ssnap_in + c0 : nullptr;
-  float* ssnap_out = LAYERS == 2 ? a.ssnap_out + c0 : nullptr;
-  const uint32_t* v_in = a.v_in + c0;
-  uint32_t* v_out = a.v_out + c0;
-  int64_t* trk = TRACK ? a.trk + c0 : nullptr;
+  const int64_t* zm_in = ap->zm_in + c0;
+  const float* snap_in = ap->snap_in + c0;
+  float* snap_out = ap->snap_out + c0;
+  const int64_t* sm_in = LAYERS == 2 ? ap->sm_in + c0 : nullptr;
+  const float* ssnap_in = LAYERS == 2 ? ap->ssnap_in + c0 : nullptr;
+  float* ssnap_out = LAYERS == 2 ? ap->ssnap_out + c0 : nullptr;
+  const uint32_t* v_in = ap->v_in + c0;
+  // a halo coordinate's wrap: within one period on an axis of 64 cells or
+  // more (the halo is at most 31 cells, the last tile's overhang 31)
+  auto wrap_x = [&](int32_t v) __attribute__((always_inline)) {
+    return nx >= 64 ? wrap_near(v, nx) : wrap(v, nx, rcp_nx);
+  };
+  auto wrap_y = [&](int32_t v) __attribute__((always_inline)) {
+    return ny >= 64 ? wrap_near(v, ny) : wrap(v, ny, rcp_ny);
+  };
 
   constexpr int kCellPer = (kCell + kStepThreads - 1) / kStepThreads;
 
@@ -221,14 +231,14 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   {
     const int32_t cu = u / kChunk;
     if (cu <= kStepThreads) {
-      if ((int32_t)threadIdx.x < cu) part_c = a.csum_cur[threadIdx.x];
+      if ((int32_t)threadIdx.x < cu) part_c = ap->csum_cur[threadIdx.x];
     } else {
-      for (int32_t c = threadIdx.x; c < cu; c += kStepThreads) part_c += a.csum_cur[c];
+      for (int32_t c = threadIdx.x; c < cu; c += kStepThreads) part_c += ap->csum_cur[c];
     }
     const int32_t t = cu * kChunk + (int32_t)threadIdx.x;
-    if (t < u) part_n = a.nin_cur[t];
+    if (t < u) part_n = ap->nin_cur[t];
   }
-  const uint32_t nin_u = RELAX_ONLY ? 0u : a.nin_cur[u];
+  const uint32_t nin_u = RELAX_ONLY ? 0u : ap->nin_cur[u];
 
   PRec rec0{};       // this thread's first arrival (loaded in the relax phase)
   uint32_t sr0 = 0;  // its sub-range
@@ -249,8 +259,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       uint32_t rc = 0;
       if (ok) {
         const int64_t s9 = (int64_t)(t0 + sx * tiles_y + sy) * 9 + d;
-        rb = a.sub_base_prev[s9];
-        rc = a.sub_cnt_prev[s9];
+        rb = ap->sub_base_prev[s9];
+        rc = ap->sub_cnt_prev[s9];
       }
       s_rbase[d] = rb;
       s_slot[d] = rc;  // lengths, turned into s_rpre by prefix_arrivals
@@ -269,7 +279,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   auto first_arrival = [&]() __attribute__((always_inline)) {
     if (threadIdx.x < s_rpre[9]) {
       while (sr0 < 8 && threadIdx.x >= s_rpre[sr0 + 1]) sr0++;
-      rec0 = a.in[s_rbase[sr0] + (int64_t)(threadIdx.x - s_rpre[sr0])];
+      rec0 = ap->in[s_rbase[sr0] + (int64_t)(threadIdx.x - s_rpre[sr0])];
     }
   };
   if constexpr (EXT) {
@@ -285,8 +295,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       int32_t gx = x0 - 1 + e / kH1Y, gy = y0 - 1 + e % kH1Y;
       bool ok = e < kH1X * kH1Y;
       if (PERIODIC) {
-        gx = wrap(gx, nx, rcp_nx);
-        gy = wrap(gy, ny, rcp_ny);
+        gx = wrap_x(gx);
+        gy = wrap_y(gy);
       } else {
         ok = ok && gx >= 0 && gy >= 0 && gx < nx && gy < ny;
       }
@@ -337,7 +347,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     ColourHalo hl = kColourHalo;
     const int32_t limx = PERIODIC ? nx - nx % 3 : nx, limy = PERIODIC ? ny - ny % 3 : ny;
     if (PERIODIC) {
-      const ColourHalo w = a.chalo;
+      const ColourHalo w = {ap->chalo.xl, ap->chalo.xh, ap->chalo.yl, ap->chalo.yh};
       const bool sx = limx != nx && (x0 - w.xl < 0 || x0 + kSX + w.xh > limx);
       const bool sy = limy != ny && (y0 - w.yl < 0 || y0 + kSY + w.yh > limy);
       if (sx || sy) hl = w;
@@ -358,77 +368,86 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       cls[e - RY - 2] = 0;
       cls[R + e] = 0;
     }
-    // region cell of index e (e < 2^16: the product is within 1/2 of a step of exact)
+    // region row of index e (e < 2^16: the product is within 1/2 of a step of exact)
     auto row_of = [=](int32_t e) __attribute__((always_inline)) {
       return (int32_t)(((float)e + 0.5f) * rcp_ry);
     };
-    constexpr int kMaxR = (kSX + kColourHaloMax.xl + kColourHaloMax.xh) * (kSY + kColourHaloMax.yl + kColourHaloMax.yh);
-    constexpr int kRPer = (kMaxR + kStepThreads - 1) / kStepThreads;
-    constexpr int kB = 4;  // cells a thread loads at once
-    uint32_t where[kRPer];  // class << 16 | rank within it; 0: not listed
+    // A wave loads whole rows, 64 columns at a time (the interior region is 62
+    // wide): the row's address and x class are scalar, the column's part is
+    // computed once.
+    constexpr int kWaves = kStepThreads / 64;
+    constexpr int kRows = (kSX + kColourHaloMax.xl + kColourHaloMax.xh + kWaves - 1) / kWaves;
+    constexpr int kChunks = (kSY + kColourHaloMax.yl + kColourHaloMax.yh + 63) / 64;
+    constexpr int kB = kRows < 8 ? kRows : 8;  // rows a wave has in flight
+    const int32_t wv = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x >> 6), lane = (int32_t)threadIdx.x & 63;
+    uint32_t where[kChunks][kRows];  // class << 16 | rank within it; 0: not listed
     __syncthreads();
 #pragma unroll
-    for (int b0 = 0; b0 < kRPer; b0 += 2 * kB) {
-      int64_t zv[2 * kB], sv[LAYERS == 2 ? 2 * kB : 1];
-      uint32_t vv[2 * kB];
-      int32_t cv[2 * kB];
+    for (int cc = 0; cc < kChunks; cc++) {
 #pragma unroll
-      for (int j = 0; j < 2 * kB; j++) {
-        const int i = b0 + j;
-        if (i >= kRPer) continue;
-        const int32_t e = (int32_t)threadIdx.x + i * kStepThreads;
-        zv[j] = 0;
-        if (LAYERS == 2) sv[j] = 0;
-        vv[j] = 0;
-        cv[j] = 0;
-        if (e >= R) continue;
-        const int32_t lx = row_of(e), ly = e - lx * RY;
-        int32_t gx = x0 - hl.xl + lx, gy = y0 - hl.yl + ly;
-        bool ok = true;
-        if (PERIODIC) {
-          gx = wrap(gx, nx, rcp_nx);
-          gy = wrap(gy, ny, rcp_ny);
-        } else {
-          ok = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
-        }
-        if (!ok) continue;
-        const int64_t g = (int64_t)gx * ny + gy;
-        zv[j] = zm_in[g];
-        if (LAYERS == 2) sv[j] = sm_in[g];
-        // the outermost ring only lends its values
-        if (lx >= 1 && ly >= 1 && lx < RX - 1 && ly < RY - 1) {
-          vv[j] = v_in[g];
-          const int32_t ccx = gx < limx ? gx % 3 : 3 + gx - limx, ccy = gy < limy ? gy % 3 : 3 + gy - limy;
-          cv[j] = ccx * kColourAxisMax + ccy + 1;
-        }
-      }
-      if (b0 == 0) load_arrivals();
+      for (int i = 0; i < kRows; i++) where[cc][i] = 0;
+      if (64 * cc >= RY) continue;
+      const int32_t ly = 64 * cc + lane;
+      int32_t gy = y0 - hl.yl + ly;
+      bool okc = ly < RY;
+      if (PERIODIC) gy = wrap_y(gy);
+      else okc = okc && gy >= 0 && gy < ny;
+      const int32_t ccy = gy < limy ? gy % 3 : 3 + gy - limy;
+      // the outermost ring only lends its values
+      const bool okl = okc && ly >= 1 && ly < RY - 1;
 #pragma unroll
-      for (int j = 0; j < 2 * kB; j++) {
-        const int i = b0 + j;
-        if (i >= kRPer) continue;
-        const int32_t e = (int32_t)threadIdx.x + i * kStepThreads;
-        const bool in = e < R, act = in && vv[j] != 0;
-        if (in) {
-          z_r[e] = zv[j];
-          if (LAYERS == 2) s_r[e] = sv[j];
-          v_r[e] = vv[j];
-          cls[e] = (uint8_t)(act ? cv[j] : 0);
+      for (int b0 = 0; b0 < kRows; b0 += kB) {
+        int64_t zv[kB], sv[LAYERS == 2 ? kB : 1];
+        uint32_t vv[kB];
+#pragma unroll
+        for (int j = 0; j < kB; j++) {
+          const int32_t lx = wv + (b0 + j) * kWaves;
+          zv[j] = 0;
+          if (LAYERS == 2) sv[j] = 0;
+          vv[j] = 0;
+          int32_t gx = x0 - hl.xl + lx;
+          bool okr = b0 + j < kRows && lx < RX;
+          if (PERIODIC) gx = wrap_x(gx);
+          else okr = okr && gx >= 0 && gx < nx;
+          if (!okr) continue;
+          const int64_t g = (int64_t)gx * ny + gy;
+          if (okc) {
+            zv[j] = zm_in[g];
+            if (LAYERS == 2) sv[j] = sm_in[g];
+          }
+          if (okl && lx >= 1 && lx < RX - 1) vv[j] = v_in[g];
         }
-        // rank within the class: one counter update per wave and class
-        where[i] = 0;
-        uint64_t rem = __ballot(act);
-        while (rem) {
-          const int32_t l = __builtin_ctzll(rem);
-          const int32_t c = __builtin_amdgcn_readlane(cv[j], l);
-          const uint64_t m = __ballot(act && cv[j] == c);
-          uint32_t base = 0;
-          if ((int32_t)(threadIdx.x & 63) == l) base = atomicAdd(&s_ccnt[c], (uint32_t)__popcll(m));
-          base = __builtin_amdgcn_readlane(base, l);
-          if (act && cv[j] == c)
-            where[i] = (uint32_t)c << 16 |
-                       (base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)));
-          rem &= ~m;
+        if (cc == 0 && b0 == 0) load_arrivals();
+#pragma unroll
+        for (int j = 0; j < kB; j++) {
+          const int32_t lx = wv + (b0 + j) * kWaves;
+          if (b0 + j >= kRows || lx >= RX) continue;
+          int32_t gx = x0 - hl.xl + lx;
+          if (PERIODIC) gx = wrap_x(gx);
+          const int32_t cv = (gx < limx ? gx % 3 : 3 + gx - limx) * kColourAxisMax + ccy + 1;
+          const int32_t e = lx * RY + ly;
+          const bool act = vv[j] != 0;
+          if (ly < RY) {
+            z_r[e] = zv[j];
+            if (LAYERS == 2) s_r[e] = sv[j];
+            v_r[e] = vv[j];
+            cls[e] = (uint8_t)(act ? cv : 0);
+          }
+          // rank within the class: one counter update per wave and class
+          uint64_t rem = __ballot(act);
+          while (rem) {
+            const int32_t l = __builtin_ctzll(rem);
+            const int32_t c = __builtin_amdgcn_readlane(cv, l);
+            const bool in = act && cv == c;
+            const uint64_t m = __ballot(in);
+            uint32_t base = 0;
+            if (lane == l) base = atomicAdd(&s_ccnt[c], (uint32_t)__popcll(m));
+            base = __builtin_amdgcn_readlane(base, l);
+            const uint32_t below =
+                __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            if (in) where[cc][b0 + j] = (uint32_t)c << 16 | (base + below);
+            rem &= ~m;
+          }
         }
       }
     }
@@ -448,8 +467,12 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kRPer; i++)
-      if (where[i]) list[s_cpre[where[i] >> 16] + (where[i] & 0xffffu)] = (uint16_t)(threadIdx.x + i * kStepThreads);
+    for (int cc = 0; cc < kChunks; cc++)
+#pragma unroll
+      for (int i = 0; i < kRows; i++)
+        if (where[cc][i])
+          list[s_cpre[where[cc][i] >> 16] + (where[cc][i] & 0xffffu)] =
+              (uint16_t)((wv + i * kWaves) * RY + 64 * cc + lane);
     const uint32_t nvis = s_cpre[32];
     if (!RELAX_ONLY) first_arrival();
     __syncthreads();
@@ -474,14 +497,14 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
         valid |= (ok ? 1u : 0u) << k;
         const float diff = hc - hn[k];
         const float d = (c_ox[k] != 0 && c_oy[k] != 0) ? dd : 1.0f;
-        const float excess = __builtin_fabsf(diff) - (d * a.maxdiff) * 1.0f;
+        const float excess = __builtin_fabsf(diff) - (d * ap->maxdiff) * 1.0f;
         act = act || (ok && diff != 0.0f && !(excess <= 0.0f));
       }
       if (!act) return;  // no neighbour beyond the threshold: the walk moves nothing
       const auto sed_of = [&](int32_t k) { return f32_from_fx(s_r[e + off_x(k) * RY + off_y(k)]); };
       int64_t centre = 0;
       cascade_cell_dev<LAYERS>(hn, sed_of, hc, LAYERS == 2 ? f32_from_fx(s_r[e]) : 0.0f, valid,
-                               settle_factor_dev(a.settling, v_r[e]), a.maxdiff, [&](int32_t k, int64_t amt) {
+                               settle_factor_dev(ap->settling, v_r[e]), ap->maxdiff, [&](int32_t k, int64_t amt) {
                                  centre -= amt;
                                  const int32_t q = e + off_x(k) * RY + off_y(k);
                                  z_r[q] += amt;
@@ -586,78 +609,85 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     float* s_old = (float*)s_work;
     float* s_sold = s_old + kH3X * kH3Y;  // valid when LAYERS == 2
     uint32_t* s_vold = (uint32_t*)(s_old + kH3X * kH3Y * (LAYERS == 2 ? 2 : 1));
+    // the 1-halo masters, to which the cascades' transfers are added; with two
+    // layers also sediment minus height master, which a transfer leaves alone
     int64_t* s_casc = (int64_t*)(s_vold + kH2X * kH2Y);
-    // master (with the previous window's pickups) of the tile and its halo,
-    // loaded before the cascades are computed
-    constexpr int kH1Per = (kH1X * kH1Y + kStepThreads - 1) / kStepThreads;
-    int64_t zpre[kH1Per], spre[LAYERS == 2 ? kH1Per : 1];
+    int64_t* s_sdif = s_casc + kH1X * kH1Y;  // LAYERS == 2
+    // Cells of the halo region by thread: kPass passes of whole rows (a thread
+    // keeps its column, kRPP rows a pass), then the six halo columns.  One
+    // address serves a cell's five arrays (snapshot and sediment snapshot on
+    // the 3-halo, events on the 2-halo, the masters with the previous window's
+    // pickups on the 1-halo), and every load is issued before the first LDS
+    // store, so the fill costs one memory round trip.  (Linear indices into
+    // each region cost a division and a wrap per load: a sixth of the
+    // kernel's vector instructions.)
+    constexpr int kRPP = kStepThreads / kSY;
+    constexpr int kPass = (kH3X + kRPP - 1) / kRPP;
+    constexpr int kHaloCells = 6 * kH3X;
+    constexpr int kItems = kPass + (kHaloCells + kStepThreads - 1) / kStepThreads;
+    static_assert(kStepThreads % kSY == 0, "whole rows a pass");
+    const int32_t trow = (int32_t)threadIdx.x / kSY, tcol = (int32_t)threadIdx.x % kSY + 3;
+    // row and column of item i in the 3-halo region; false past its end
+    auto item = [&](int i, int32_t& row, int32_t& col) __attribute__((always_inline)) {
+      if (i < kPass) {
+        row = trow + i * kRPP;
+        col = tcol;
+        return row < kH3X;
+      }
+      const int32_t h = (int32_t)threadIdx.x + (i - kPass) * kStepThreads;
+      row = h / 6;
+      const int32_t c = h - row * 6;
+      col = c < 3 ? c : kSY + c;
+      return h < kHaloCells;
+    };
+    float hv[kItems], hs3[LAYERS == 2 ? kItems : 1];
+    uint32_t vv[kItems];
+    int64_t zv[kItems], sv[LAYERS == 2 ? kItems : 1];
 #pragma unroll
-    for (int i = 0; i < kH1Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      int32_t gx = x0 - 1 + e / kH1Y, gy = y0 - 1 + e % kH1Y;
-      bool ok = e < kH1X * kH1Y;
+    for (int i = 0; i < kItems; i++) {
+      int32_t row, col;
+      bool ok = item(i, row, col);
+      int32_t gx = x0 - 3 + row, gy = y0 - 3 + col;
       if (PERIODIC) {
-        gx = wrap(gx, nx, rcp_nx);
-        gy = wrap(gy, ny, rcp_ny);
+        gx = wrap_x(gx);
+        gy = wrap_y(gy);
       } else {
         ok = ok && gx >= 0 && gy >= 0 && gx < nx && gy < ny;
       }
       const int64_t g = (int64_t)gx * ny + gy;
-      zpre[i] = ok ? zm_in[g] : 0;
-      if (LAYERS == 2) spre[i] = ok ? sm_in[g] : 0;
-    }
-    // snapshot (3-halo) and events (2-halo): every load is issued before the
-    // first LDS store, so the fill costs one memory round trip
-    constexpr int kH3Per = (kH3X * kH3Y + kStepThreads - 1) / kStepThreads;
-    constexpr int kH2Per = (kH2X * kH2Y + kStepThreads - 1) / kStepThreads;
-    float hv[kH3Per], hs3[LAYERS == 2 ? kH3Per : 1];
-    uint32_t vv[kH2Per];
-#pragma unroll
-    for (int i = 0; i < kH3Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      int32_t gx = x0 - 3 + e / kH3Y, gy = y0 - 3 + e % kH3Y;
-      bool ok = e < kH3X * kH3Y;
-      if (PERIODIC) {
-        gx = wrap(gx, nx, rcp_nx);
-        gy = wrap(gy, ny, rcp_ny);
-      } else {
-        ok = ok && gx >= 0 && gy >= 0 && gx < nx && gy < ny;
+      hv[i] = 0.0f;
+      vv[i] = 0;
+      zv[i] = 0;
+      if (LAYERS == 2) {
+        hs3[i] = 0.0f;
+        sv[i] = 0;
       }
-      const int64_t g = (int64_t)gx * ny + gy;
-      hv[i] = ok ? snap_in[g] : 0.0f;
-      if (LAYERS == 2) hs3[i] = ok ? ssnap_in[g] : 0.0f;
-    }
-#pragma unroll
-    for (int i = 0; i < kH2Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      int32_t gx = x0 - 2 + e / kH2Y, gy = y0 - 2 + e % kH2Y;
-      bool ok = e < kH2X * kH2Y;
-      if (PERIODIC) {
-        gx = wrap(gx, nx, rcp_nx);
-        gy = wrap(gy, ny, rcp_ny);
-      } else {
-        ok = ok && gx >= 0 && gy >= 0 && gx < nx && gy < ny;
+      if (ok) {
+        hv[i] = snap_in[g];
+        if (LAYERS == 2) hs3[i] = ssnap_in[g];
+        if (row >= 1 && row <= kH3X - 2 && col >= 1 && col <= kH3Y - 2) vv[i] = v_in[g];
+        if (row >= 2 && row <= kH3X - 3 && col >= 2 && col <= kH3Y - 3) {
+          zv[i] = zm_in[g];
+          if (LAYERS == 2) sv[i] = sm_in[g];
+        }
       }
-      vv[i] = ok ? v_in[(int64_t)gx * ny + gy] : 0u;
     }
     // loaded after the map loads are out, so that their wait overlaps those
     load_arrivals();
+    uint16_t* s_cas = (uint16_t*)(s_casc + kH1X * kH1Y * LAYERS);  // H2 cells with a transfer: row << 8 | column
+    if (threadIdx.x == 0) s_ncas = 0;
 #pragma unroll
-    for (int i = 0; i < kH3Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      if (e < kH3X * kH3Y) {
-        s_old[e] = hv[i];
-        if (LAYERS == 2) s_sold[e] = hs3[i];
+    for (int i = 0; i < kItems; i++) {
+      int32_t row, col;
+      if (!item(i, row, col)) continue;
+      s_old[row * kH3Y + col] = hv[i];
+      if (LAYERS == 2) s_sold[row * kH3Y + col] = hs3[i];
+      if (row >= 1 && row <= kH3X - 2 && col >= 1 && col <= kH3Y - 2) s_vold[(row - 1) * kH2Y + col - 1] = vv[i];
+      if (row >= 2 && row <= kH3X - 3 && col >= 2 && col <= kH3Y - 3) {
+        s_casc[(row - 2) * kH1Y + col - 2] = zv[i];
+        if (LAYERS == 2) s_sdif[(row - 2) * kH1Y + col - 2] = sv[i] - zv[i];
       }
     }
-#pragma unroll
-    for (int i = 0; i < kH2Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      if (e < kH2X * kH2Y) s_vold[e] = vv[i];
-    }
-    uint16_t* s_cas = (uint16_t*)(s_casc + kH1X * kH1Y);  // H2 cells with a transfer
-    for (int e = threadIdx.x; e < kH1X * kH1Y; e += kStepThreads) s_casc[e] = 0;
-    if (threadIdx.x == 0) s_ncas = 0;
     __syncthreads();
     // start of each arrival sub-range in this tile's arrival order (read
     // after the next barrier)
@@ -668,14 +698,15 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     // height.  The walk changes the centre only after a transfer, so a cell
     // with none such moves nothing and is skipped.  Listed in LDS so that
     // the cascades below run on full waves.
-    for (int e0 = 0; e0 < kH2X * kH2Y; e0 += kStepThreads) {
-      const int e = e0 + (int)threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+      int32_t row, col;
+      (void)item(i, row, col);
       bool act = false;
-      if (e < kH2X * kH2Y && s_vold[e] != 0) {
-        const int32_t lx = e / kH2Y, ly = e % kH2Y;
-        const int32_t gx = x0 - 2 + lx, gy = y0 - 2 + ly;
-        const int32_t ic = (lx + 1) * kH3Y + (ly + 1);
-        const float hc = s_old[ic];
+      if (vv[i] != 0) {
+        const int32_t gx = x0 - 3 + row, gy = y0 - 3 + col;
+        const int32_t ic = row * kH3Y + col;
+        const float hc = hv[i];
         const float dd = __builtin_sqrtf(2.0f);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -686,7 +717,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
           }
           const float diff = hc - s_old[ic + c_ox[k] * kH3Y + c_oy[k]];
           const float d = (c_ox[k] != 0 && c_oy[k] != 0) ? dd : 1.0f;
-          const float excess = __builtin_fabsf(diff) - (d * a.maxdiff) * 1.0f;
+          const float excess = __builtin_fabsf(diff) - (d * ap->maxdiff) * 1.0f;
           act = act || (ok && diff != 0.0f && !(excess <= 0.0f));
         }
       }
@@ -694,8 +725,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
       uint32_t base = 0;
       if ((threadIdx.x & 63) == 0 && m) base = atomicAdd(&s_ncas, (uint32_t)__popcll(m));
-      base = __shfl(base, 0, 64);
-      if (act) s_cas[base + below] = (uint16_t)e;
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (act) s_cas[base + below] = (uint16_t)(row << 8 | col);
     }
     __syncthreads();
 
@@ -703,8 +734,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     const uint32_t ncas = s_ncas;
     for (uint32_t i = threadIdx.x; i < ncas; i += kStepThreads) {
       const int32_t e = s_cas[i];
-      const uint32_t v = s_vold[e];
-      const int32_t lx = e / kH2Y, ly = e % kH2Y;  // H2 coords; H3 = +1, H1 = -1
+      const int32_t lx = (e >> 8) - 1, ly = (e & 255) - 1;  // H2 coords; H3 = +1, H1 = -1
+      const uint32_t v = s_vold[lx * kH2Y + ly];
       const int32_t gx = x0 - 2 + lx, gy = y0 - 2 + ly;
       float hn[8];
       uint32_t valid = 0;
@@ -722,7 +753,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       const auto sed_of = [&](int32_t k) { return s_sold[ic + off_x(k) * kH3Y + off_y(k)]; };
       int64_t centre = 0;
       cascade_cell_dev<LAYERS>(hn, sed_of, s_old[ic], LAYERS == 2 ? s_sold[ic] : 0.0f, valid,
-                               settle_factor_dev(a.settling, v), a.maxdiff, [&](int32_t k, int64_t amt) {
+                               settle_factor_dev(ap->settling, v), ap->maxdiff, [&](int32_t k, int64_t amt) {
                                  centre -= amt;
                                  const int32_t hx = lx - 1 + off_x(k), hy = ly - 1 + off_y(k);
                                  if (amt != 0 && hx >= 0 && hy >= 0 && hx < kH1X && hy < kH1Y)
@@ -737,7 +768,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     if (!RELAX_ONLY) first_arrival();
     __syncthreads();
 
-    // master += cascade; next snapshot for the tile and its halo.  The
+    // next snapshot for the tile and its halo.  The
     // tile's own masters seed the particle phase's pickup accumulators
     // (acc_d / acc_ds below: the front of s_work, whose relax-phase arrays
     // are dead once the cascades are summed, and clear of s_casc)
@@ -745,39 +776,27 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
                   "the pickup accumulators must not overlap s_casc");
     int64_t* acc_z = (int64_t*)s_work;
 #pragma unroll
-    for (int i = 0; i < kH1Per; i++) {
-      const int e = threadIdx.x + i * kStepThreads;
-      if (e >= kH1X * kH1Y) continue;
-      const int32_t lx = e / kH1Y, ly = e % kH1Y;
-      int32_t gx = x0 - 1 + lx, gy = y0 - 1 + ly;
-      bool ok = true;
-      if (PERIODIC) {
-        gx = wrap(gx, nx, rcp_nx);
-        gy = wrap(gy, ny, rcp_ny);
-      } else {
-        ok = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
-      }
-      if (!ok) {
-        s_new[e] = 0.0f;
-        if (LAYERS == 2) s_snew[e] = 0.0f;
-        continue;
-      }
+    for (int i = 0; i < kItems; i++) {
+      int32_t row, col;
+      if (!item(i, row, col) || row < 2 || row > kH3X - 3 || col < 2 || col > kH3Y - 3) continue;
+      const int32_t lx = row - 2, ly = col - 2, e = lx * kH1Y + ly;  // 1-halo coordinates
+      const int32_t gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+      const bool ok = PERIODIC || (gx >= 0 && gy >= 0 && gx < nx && gy < ny);
+      const bool mine = lx >= 1 && ly >= 1 && lx <= kSX && ly <= kSY && gx < nx && gy < ny;
       const int64_t g = (int64_t)gx * ny + gy;
-      const int64_t cas = s_casc[e];
-      const int64_t z = zpre[i] + cas;
+      const int64_t z = s_casc[e];
       const float zf = f32_from_fx(z);
-      s_new[e] = zf;
-      const bool mine = lx >= 1 && ly >= 1 && lx <= kSX && ly <= kSY && x0 - 1 + lx < nx && y0 - 1 + ly < ny;
+      s_new[e] = ok ? zf : 0.0f;
       const int32_t li = (lx - 1) * kSY + (ly - 1);
       if (mine) {
         acc_z[li] = z;
         snap_out[g] = zf;
       }
       if (LAYERS == 2) {
-        int64_t s = spre[i] + cas;
+        int64_t s = z + s_sdif[e];
         if (s < 0) s = 0;
         const float sf = f32_from_fx(s);
-        s_snew[e] = sf;
+        s_snew[e] = ok ? sf : 0.0f;
         if (mine) {
           acc_z[kCell + li] = s;
           ssnap_out[g] = sf;
@@ -790,16 +809,19 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   {
     int64_t part = (int64_t)part_c + (int64_t)part_n;
     for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-    if ((threadIdx.x & 63) == 0) s_lost[threadIdx.x >> 6] = part;
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = part;
     __syncthreads();
     if (threadIdx.x == 0) {
       int64_t b0 = 0;
-      for (int i = 0; i < kStepThreads / 64; i++) b0 += s_lost[i];
+      for (int i = 0; i < kStepThreads / 64; i++) b0 += s_part[i];
       s_base = 9 * b0;
+      s_lost = 0;
+      s_far = 0;
     }
   }
 
   // ---------------- 2. particles of the tile ----------------
+  ap = step_args(ap);
   int64_t* acc_d = (int64_t*)s_work;
   int64_t* acc_ds = acc_d + kCell;  // LAYERS == 2
   uint32_t* acc_v = (uint32_t*)(acc_d + kCell * (LAYERS == 2 ? 2 : 1));
@@ -815,8 +837,6 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
   }
   __syncthreads();  // s_rpre is read from s_slot before s_slot restarts
   if (threadIdx.x < 9) s_slot[threadIdx.x] = 0;
-  int64_t lost_here = 0;
-  uint32_t steps_here = 0, far_here = 0;
   __syncthreads();
 
   if (!RELAX_ONLY) {
@@ -825,30 +845,18 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     k.ny = ny;
     k.rcp_nx = rcp_nx;
     k.rcp_ny = rcp_ny;
-    k.mapscale = a.mapscale;
-    k.max_age = a.max_age;
-    set_boundarylayer(k, a.boundarylayer);
-    k.suspension = a.suspension;
-    k.gravity = a.gravity;
-    k.abrasion = a.abrasion;
+    k.mapscale = ap->mapscale;
+    k.max_age = ap->max_age;
+    set_boundarylayer(k, ap->boundarylayer);
+    k.suspension = ap->suspension;
+    k.gravity = ap->gravity;
+    k.abrasion = ap->abrasion;
     k.ps = mk(T.ps[0], T.ps[1], T.ps[2]);
     k.nps = mk(T.nps[0], T.nps[1], T.nps[2]);
-    // uniform constants of fly() held in vector registers (one each) rather
-    // than scalar ones, which this kernel has too few of
-    k.mapscale = in_vgpr(k.mapscale);
-    k.boundarylayer = in_vgpr(k.boundarylayer);
-    k.gravity = in_vgpr(k.gravity);
-    if (!EXT) {  // in the step-only mode these stay scalar: pinning them too spills vector registers there
-      k.rcp_bl = in_vgpr(k.rcp_bl);
-      k.suspension = in_vgpr(k.suspension);
-      k.abrasion = in_vgpr(k.abrasion);
-    }
-    k.ps = mk(in_vgpr(k.ps.x), in_vgpr(k.ps.y), in_vgpr(k.ps.z));
-    k.nps = mk(in_vgpr(k.nps.x), in_vgpr(k.nps.y), in_vgpr(k.nps.z));
-    const uint64_t ck = cycle_key(T.seed, *a.cycle);
+    const uint64_t ck = cycle_key(T.seed, *ap->cycle);
     const int64_t p0 = T.part0;
     const int64_t out_base = s_base;  // 9 x the input counts of tiles 0 .. u-1
-    const uint32_t far_n = *a.far_cnt_in;
+    const uint32_t far_n = *ap->far_cnt_in;
 
     // one input record
     using Rec = PRec;
@@ -857,10 +865,10 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     // cell (fx, fy) counts it among its next window's arrivals
     auto send_far = [&](f4a8 o0, f4a8 o1, int64_t ledger, int32_t fx, int32_t fy) __attribute__((always_inline)) {
       const int32_t dest = t0 + (fx / kSX) * tiles_y + fy / kSY;
-      atomicAdd(&a.nin_next[dest], 1u);
-      atomicAdd(&a.csum_next[dest / kChunk], 1u);
-      const uint32_t fslot = atomicAdd(a.far_cnt_out, 1u);
-      a.far_out[fslot] = PRec{o0, o1, ledger};
+      atomicAdd(&ap->nin_next[dest], 1u);
+      atomicAdd(&ap->csum_next[dest / kChunk], 1u);
+      const uint32_t fslot = atomicAdd(ap->far_cnt_out, 1u);
+      ap->far_out[fslot] = PRec{o0, o1, ledger};
     };
     // step one record and write it out
     auto process = [&](const Rec& r) __attribute__((always_inline)) {
@@ -869,7 +877,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       const f4a8 q1 = r.q1;
       w.px = q0.x; w.py = q0.y; w.pz = q0.z; w.sed = q0.w;
       w.sx = q1.x; w.sy = q1.y; w.sz = q1.z;
-      w.age = a.window;
+      w.age = ap->window;
       w.ledger = r.ledger;
       w.lastc = 0;
       const uint32_t pid = f2u(q1.w);
@@ -904,11 +912,10 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
             if (LAYERS == 2) atomicAdd((unsigned long long*)&acc_ds[li], (unsigned long long)w.ledger);
           }
         } else {
-          lost_here += w.ledger;
+          atomicAdd((unsigned long long*)&s_lost, (unsigned long long)w.ledger);
         }
         return;
       }
-      steps_here++;
       // route by the cell the particle now occupies; one that leaves a
       // bounded map (or whose position stops being finite) stays with the
       // tile of its last cell and dies there at its next call
@@ -934,13 +941,13 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
                           : f4a8{w.px, w.py, w.pz, w.sed};
       const f4a8 o1 = {w.sx, w.sy, w.sz, u2f(pid)};
       if (code == 255) {
-        far_here++;
+        atomicAdd(&s_far, 1u);
         send_far(o0, o1, w.ledger, ncx, ncy);
         return;
       }
       // sub-range `code` of this tile's output region holds up to nin_u records
       const int64_t o = out_base + (int64_t)code * nin_u + atomicAdd(&s_slot[code], 1u);
-      a.out[o] = PRec{o0, o1, w.ledger};
+      ap->out[o] = PRec{o0, o1, w.ledger};
     };
 
     // the arrivals, e = 0 .. n_in - 1 over the nine sub-ranges in order; each
@@ -956,16 +963,16 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       Rec cur = rec0;
       for (uint32_t e = threadIdx.x; e < n_in; e += kStepThreads) {
         Rec nxt{};
-        if (e + kStepThreads < n_in) nxt = load(a.in, index_of(e + kStepThreads));
+        if (e + kStepThreads < n_in) nxt = load(ap->in, index_of(e + kStepThreads));
         process(cur);
         cur = nxt;
       }
     }
     for (int64_t j = threadIdx.x; j < (int64_t)far_n; j += kStepThreads) {
-      const int64_t fp = (int64_t)f2u(a.far_in[j].q1.w);
+      const int64_t fp = (int64_t)f2u(ap->far_in[j].q1.w);
       if (fp < p0 || fp >= p0 + T.npart) continue;  // another terrain's particle
       int32_t cx, cy;
-      const f4a8 q0 = a.far_in[j].q0;
+      const f4a8 q0 = ap->far_in[j].q0;
       int32_t ctx, cty;
       if (cell_of<PERIODIC>(q0.x, q0.z, k, cx, cy)) {
         ctx = cx / kSX;
@@ -975,12 +982,21 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
         ctx = (lc / ny) / kSX;
         cty = (lc % ny) / kSY;
       }
-      if (ctx == tx && cty == ty) process(load(a.far_in, j));
+      if (ctx == tx && cty == ty) process(load(ap->far_in, j));
     }
   }
   __syncthreads();
 
   // ---------------- 3. write the tile's window results ----------------
+  ap = step_args(ap);
+  int64_t* zm_out = ap->zm_out + c0;
+  int64_t* sm_out = LAYERS == 2 ? ap->sm_out + c0 : nullptr;
+  uint32_t* v_out = ap->v_out + c0;
+  int64_t* trk = TRACK ? ap->trk + c0 : nullptr;
+  if (EXT) {
+    snap_out = ap->snap_out + c0;
+    if (LAYERS == 2) ssnap_out = ap->ssnap_out + c0;
+  }
 #pragma unroll
   for (int i = 0; i < kCellPer; i++) {
     const int e = threadIdx.x + i * kStepThreads;
@@ -1016,7 +1032,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
 #pragma unroll
     for (int i = 0; i < kCellPer; i++)
 #pragma unroll
-      for (int f = 0; f < 4; f++) old[i][f] = tv[i][f] != 0 ? trk[f * a.ncell + gi[i]] : 0;
+      for (int f = 0; f < 4; f++) old[i][f] = tv[i][f] != 0 ? trk[f * ap->ncell + gi[i]] : 0;
   }
   // s_rbase is free again (the arrivals are consumed): it carries the chunk
   // of each direction's destination tile to the aggregation below
@@ -1026,8 +1042,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     // and the next window's arrivals of the tile in direction d
     const int32_t d = threadIdx.x;
     const uint32_t n = s_slot[d];
-    a.sub_base_cur[(int64_t)u * 9 + d] = s_base + (int64_t)d * nin_u;
-    a.sub_cnt_cur[(int64_t)u * 9 + d] = n;
+    ap->sub_base_cur[(int64_t)u * 9 + d] = s_base + (int64_t)d * nin_u;
+    ap->sub_cnt_cur[(int64_t)u * 9 + d] = n;
     int32_t chunk = -1;
     if (n) {
       const int32_t dx = d / 3 - 1, dy = d % 3 - 1;
@@ -1037,47 +1053,36 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
         dty = wrapt(dty, tiles_y);
       }
       const int32_t dest = t0 + dtx * tiles_y + dty;
-      atomicAdd(&a.nin_next[dest], n);
+      atomicAdd(&ap->nin_next[dest], n);
       chunk = dest / kChunk;
     }
     s_dchunk[d] = chunk;
   }
   if (threadIdx.x == 0) {
-    a.nin_clear[u] = 0;  // the window after next accumulates here
-    if (u % kChunk == 0) a.csum_clear[u / kChunk] = 0;
+    ap->nin_clear[u] = 0;  // the window after next accumulates here
+    if (u % kChunk == 0) ap->csum_clear[u / kChunk] = 0;
     if (u == 0) {
-      *a.far_cnt_clear = 0;
+      *ap->far_cnt_clear = 0;
       if ((hs | ls) > 0)
-        for (int i = 0; i < 16; i++) a.hcnt_clear[i] = 0;
+        for (int i = 0; i < 16; i++) ap->hcnt_clear[i] = 0;
     }
     // crowded (or light) now: listed for the next launch (the count moves
     // little from one window to the next)
     if (hs > 0 && nin_u > kHeavyMin) {
       const uint32_t home = home_of((uint32_t)u);
-      const uint32_t slot = atomicAdd(&a.hcnt_next[home], 1u);
+      const uint32_t slot = atomicAdd(&ap->hcnt_next[home], 1u);
       if (slot < hs / 8) {
-        a.heavy_next[home * (hs / 8) + slot] = (uint32_t)u;
-        a.hstamp[u] = (uint32_t)a.window + 2u;
+        ap->heavy_next[home * (hs / 8) + slot] = (uint32_t)u;
+        ap->hstamp[u] = (uint32_t)ap->window + 2u;
       }
     } else if (ls > 0 && nin_u <= kLightMax) {
       const uint32_t home = home_of((uint32_t)u);
-      const uint32_t slot = atomicAdd(&a.hcnt_next[8 + home], 1u);
+      const uint32_t slot = atomicAdd(&ap->hcnt_next[8 + home], 1u);
       if (slot < ls / 8) {
-        a.heavy_next[kHeavySlotsMax + home * (ls / 8) + slot] = (uint32_t)u;
-        a.hstamp[u] = (uint32_t)a.window + 2u;
+        ap->heavy_next[kHeavySlotsMax + home * (ls / 8) + slot] = (uint32_t)u;
+        ap->hstamp[u] = (uint32_t)ap->window + 2u;
       }
     }
-  }
-  if (!DEPOSIT) {
-    for (int off = 32; off > 0; off >>= 1) lost_here += __shfl_xor(lost_here, off, 64);
-    if ((threadIdx.x & 63) == 0) s_lost[threadIdx.x >> 6] = lost_here;
-  }
-  if (!RELAX_ONLY) {
-    for (int off = 32; off > 0; off >>= 1) {
-      steps_here += __shfl_xor(steps_here, off, 64);
-      far_here += __shfl_xor(far_here, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) s_wstat[threadIdx.x >> 6] = ((uint64_t)far_here << 32) | steps_here;
   }
   __syncthreads();
   if (!RELAX_ONLY && threadIdx.x < 9) {
@@ -1093,32 +1098,29 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
       uint32_t n = 0;
 #pragma unroll
       for (int e = 0; e < 9; e++) n += e >= d && s_dchunk[e] == ch ? s_slot[e] : 0u;
-      atomicAdd(&a.csum_next[ch], n);
+      atomicAdd(&ap->csum_next[ch], n);
     }
   }
   if (!RELAX_ONLY && threadIdx.x == 0) {
-    // statistics: one atomic per workgroup and kind
-    uint64_t steps = 0, far = 0;
-    for (int i = 0; i < kStepThreads / 64; i++) {
-      steps += (uint32_t)s_wstat[i];
-      far += s_wstat[i] >> 32;
-    }
+    // statistics: one atomic per workgroup and kind; a particle that made its
+    // step was sent on, to a sub-range or the far list
+    const uint64_t far = s_far;
+    uint64_t steps = far;
+    for (int d = 0; d < 9; d++) steps += s_slot[d];
     const uint32_t slot = (uint32_t)u & (kStatSlots - 1);
-    if (steps) atomicAdd((unsigned long long*)&a.stat[kStatSteps * kStatSlots + slot], (unsigned long long)steps);
-    if (far) atomicAdd((unsigned long long*)&a.stat[kStatFar * kStatSlots + slot], (unsigned long long)far);
-    if (nin_u) atomicMax((unsigned long long*)&a.stat[kStatMaxTile * kStatSlots + slot], (unsigned long long)nin_u);
-    if (nin_u > kCrowded) atomicAdd((unsigned long long*)&a.stat[kStatCrowded * kStatSlots + slot], 1ull);
+    if (steps) atomicAdd((unsigned long long*)&ap->stat[kStatSteps * kStatSlots + slot], (unsigned long long)steps);
+    if (far) atomicAdd((unsigned long long*)&ap->stat[kStatFar * kStatSlots + slot], (unsigned long long)far);
+    if (nin_u) atomicMax((unsigned long long*)&ap->stat[kStatMaxTile * kStatSlots + slot], (unsigned long long)nin_u);
+    if (nin_u > kCrowded) atomicAdd((unsigned long long*)&ap->stat[kStatCrowded * kStatSlots + slot], 1ull);
     if (listed) {
-      const bool light_slot = blockIdx.x >= (uint32_t)(a.heavy_slots + a.default_slots);
-      atomicAdd((unsigned long long*)&a.stat[(light_slot ? kStatLight : kStatHeavy) * kStatSlots + slot], 1ull);
+      const bool light_slot = blockIdx.x >= (uint32_t)(ap->heavy_slots + ap->default_slots);
+      atomicAdd((unsigned long long*)&ap->stat[(light_slot ? kStatLight : kStatHeavy) * kStatSlots + slot], 1ull);
     }
   }
-  __syncthreads();
   if (!DEPOSIT && threadIdx.x == 0) {
-    int64_t l = 0;
-    for (int i = 0; i < kStepThreads / 64; i++) l += s_lost[i];
+    const int64_t l = s_lost;
     if (l != 0)
-      atomicAdd((unsigned long long*)&a.lost[(int64_t)a.tile_terrain[u] * kLostSlots + (u & (kLostSlots - 1))],
+      atomicAdd((unsigned long long*)&ap->lost[(int64_t)ap->tile_terrain[u] * kLostSlots + (u & (kLostSlots - 1))],
                 (unsigned long long)l);
   }
   if (TRACK && !RELAX_ONLY) {
@@ -1126,13 +1128,20 @@ __device__ __forceinline__ void step_body(const StepArgs& a) {
     for (int i = 0; i < kCellPer; i++)
 #pragma unroll
       for (int f = 0; f < 4; f++)
-        if (tv[i][f] != 0) trk[f * a.ncell + gi[i]] = old[i][f] + tv[i][f];
+        if (tv[i][f] != 0) trk[f * ap->ncell + gi[i]] = old[i][f] + tv[i][f];
   }
 }
 
+// Bound by the latency of a workgroup's phases (halo load, cascades,
+// particles, write-out) and by vector issue within them.  Phase-wise argument
+// reads, one address per halo cell and branch-free primitives took the
+// kernel from 10,470 to 7,000 instructions (70 to 46 KB of code, past and
+// within the instruction cache) and from 18.8 to 16.2 us a window on 256^2
+// (2,000 particles), 17.2 to 13.9 us on 75 x 101 (300), 73.0 to 70.9 us on
+// 1024^2 (a million).
 template <int SX, int SY, int NT, int WPE, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(StepArgs a) {
-  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>(a);
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(StepArgs) {
+  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
 }
 
 // The colour-ordered cascade in the same single launch per window: the tile
@@ -1146,8 +1155,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 // 30,000 particles 85.5 -> 35.9 ms; 1024^2 with a million particles, where a
 // class launch fills the chip, 110 -> 111 ms.
 template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colour_step(StepArgs a) {
-  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>(a);
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colour_step(StepArgs) {
+  step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
 }
 
 // dynamic LDS of k_colour_step: the region's masters, events, list and
