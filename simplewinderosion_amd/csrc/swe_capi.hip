@@ -256,6 +256,17 @@ int32_t heavy_first_mode(const swe_ctx* c) {
   return c->heavy_first >= 0 ? c->heavy_first : (c->ntiles <= 4096 ? 2 : 1);
 }
 
+// Tiles whose workgroups are all resident at once: the chip's 256 CUs times
+// the workgroups a CU holds (the shape's waves per SIMD; three of the
+// colour-ordered kernel's, by its LDS).  A launch of no more has no order to
+// choose, so by default it lists no tiles: the lists cost a dependent load
+// before the halo and a returning atomic at the end (256^2 map, 128 tiles:
+// 25.7 ms for three cycles with them, 24.0 ms without).
+int64_t resident_tiles(const swe_ctx* c) {
+  const swe::StepShape sh = swe::kStepShape[c->shape];
+  return 256 * (colour_mode(c->p) ? 3 : 4 * sh.waves / (sh.threads / 64));
+}
+
 // light-tile slots of a launch: half the tiles, a multiple of 8
 int64_t light_cap(int64_t ntiles) { return (ntiles / 2 + 7) / 8 * 8; }
 
@@ -481,7 +492,7 @@ int erode_global(swe_ctx* c, int64_t particles, int32_t n_cycles, int64_t nwin, 
 
 // terrain records for the device: seed / pspeed from the params unless a
 // terrain overrides them
-int push_terrains(swe_ctx* c, const int64_t* particles) {
+int push_terrains(swe_ctx* c, const int64_t* particles, swe::Terrain* first) {
   std::vector<swe::Terrain> t((size_t)c->nterr);
   int64_t part0 = 0;
   for (int32_t k = 0; k < c->nterr; k++) {
@@ -503,6 +514,7 @@ int push_terrains(swe_ctx* c, const int64_t* particles) {
     normalize3(ps, T.nps);
   }
   HIPCHK(c, hipMemcpyAsync(c->dterr, t.data(), sizeof(swe::Terrain) * t.size(), hipMemcpyHostToDevice, c->stream));
+  *first = t[0];
   return 0;
 }
 
@@ -515,9 +527,9 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   int64_t total = 0;
   for (int32_t k = 0; k < c->nterr; k++) total += particles[k];
   if ((r = ensure_step(c, total > 0 ? total : 1))) return r;
-  if ((r = push_terrains(c, particles))) return r;
-  const bool layers2 = c->p.layers == 2;
   swe::StepArgs sa{};
+  if ((r = push_terrains(c, particles, &sa.t0))) return r;
+  const bool layers2 = c->p.layers == 2;
   sa.trk = c->trk;
   sa.lost = c->lost;
   sa.stat = c->dstat;
@@ -538,7 +550,7 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   sa.tile_order = c->tile_order;
   // listed crowded tiles get the first workgroups of a launch; at most one
   // slot per 8 tiles, a multiple of 8 (none on maps under 64 tiles)
-  const int32_t hf = heavy_first_mode(c);
+  const int32_t hf = c->ntiles <= resident_tiles(c) && c->heavy_first < 0 ? 0 : heavy_first_mode(c);
   sa.heavy_slots = hf ? (int32_t)std::min<int64_t>(swe::kHeavySlotsMax, (c->ntiles / 8) & ~7LL) : 0;
   // light tiles last (heavy-first mode 2, maps of 64 tiles or more): the
   // usual order is padded to a multiple of 8 so that slot b runs on XCD b % 8
@@ -692,6 +704,7 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
     key.append((const char*)&c->shape, sizeof(c->shape));
     key.append((const char*)&nwin, sizeof(nwin));
     key.append((const char*)&c->alloc_gen, sizeof(c->alloc_gen));
+    key.append((const char*)&sa.t0, sizeof(sa.t0));  // a single map's terrain is a kernel argument
   }
   const uint64_t windows_per_cycle = total > 0 ? (uint64_t)nwin + (colour ? 0 : 1) : 0;
 

@@ -53,7 +53,9 @@ __device__ __forceinline__ int32_t cascade_key_offset(double key) {
 // neighbours.  The neighbours are sorted by a sorting network on their keys
 // and walked in that order with the centre evolving; emit(k, amount) is
 // called with the fixed-point amount neighbour k receives (the centre loses
-// the same amount) for every transfer.
+// the same amount; zero for no transfer).  A wave's time is the dependent
+// chain: 230 cycles for the sort on float64 keys (760 with 64-bit integer
+// ones) and some 70 a walk step.
 template <int LAYERS, class SedOf, class Emit>
 __device__ __forceinline__ void cascade_cell_dev(const float hn[8], const SedOf& sed_of, float hc, float sc,
                                                  uint32_t validmask, float settling, float maxdiff, Emit&& emit) {
@@ -73,33 +75,51 @@ __device__ __forceinline__ void cascade_cell_dev(const float hn[8], const SedOf&
   SWE_CAS(1, 4) SWE_CAS(3, 6)
   SWE_CAS(1, 2) SWE_CAS(3, 4) SWE_CAS(5, 6)
 #undef SWE_CAS
+  // the walk's inputs in its order, read before it so that the reads overlap
+  // (each would otherwise wait its turn in the chain); an out-of-map
+  // neighbour's NaN compares false and takes nothing
   const float dd = __builtin_sqrtf(2.0f);
+  int32_t kk[8];
+  float hh[8], sn[8], thr[8], ts[8];
 #pragma unroll
   for (int r = 0; r < 8; r++) {
-    if (key[r] == -__builtin_inf()) break;  // the out-of-map neighbours come last
-    const int32_t k = cascade_key_offset(key[r]);
-    const float diff = hc - (float)key[r];
-    const float d = ((kDiagMask >> k) & 1u) ? dd : 1.0f;
-    const float excess = __builtin_fabsf(diff) - (d * maxdiff) * 1.0f;
-    float t = settling * excess / 2.0f;
-    bool go = diff != 0.0f && !(excess <= 0.0f);
-    if (LAYERS == 2 && go) {
-      const float avail = diff > 0.0f ? sc : sed_of(k);
-      if (t > avail) t = avail;
-      go = t > 0.0f;
-    }
-    if (!go) continue;
-    const int64_t tf = fx_from_f32(t);
-    if (diff > 0.0f) {
-      hc -= t;
-      sc -= t;
-      emit(k, tf);
-    } else {
-      hc += t;
-      sc += t;
-      emit(k, -tf);
-    }
+    kk[r] = cascade_key_offset(key[r]);
+    const bool in = key[r] != -__builtin_inf();
+    hh[r] = in ? (float)key[r] : __builtin_nanf("");
+    sn[r] = LAYERS == 2 && in ? sed_of(kk[r]) : 0.0f;
+    const float d = ((kDiagMask >> kk[r]) & 1u) ? dd : 1.0f;
+    thr[r] = (d * maxdiff) * 1.0f;
   }
+  // the serial chain, without branches: a neighbour that takes nothing (no
+  // difference, or none beyond the threshold) moves zero.  Transfers are
+  // signed: positive from the centre to the neighbour.
+  bool big = false;
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    const float diff = hc - hh[r], ad = __builtin_fabsf(diff);
+    const float excess = ad - thr[r];
+    float t = settling * excess / 2.0f;
+    if (LAYERS == 2) {
+      const float avail = diff > 0.0f ? sc : sn[r];
+      if (t > avail) t = avail;
+      t = t > 0.0f ? t : 0.0f;
+    }
+    t = __builtin_fminf(excess, ad) > 0.0f ? t : 0.0f;
+    ts[r] = __builtin_copysignf(t, diff);
+    if (t < 0.0f) ts[r] = -ts[r];  // a negative settling factor moves material uphill
+    hc -= ts[r];
+    if (LAYERS == 2) sc -= ts[r];
+    big = big || !(__builtin_fabsf(t) < 262144.0f);
+  }
+  int64_t amt[8];
+#pragma unroll
+  for (int r = 0; r < 8; r++) amt[r] = fx_from_small_f32(ts[r]);
+  if (__builtin_expect(big, 0)) {
+#pragma unroll
+    for (int r = 0; r < 8; r++) amt[r] = fx_from_f32(ts[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 8; r++) emit(kk[r], amt[r]);
 }
 
 }  // namespace swe

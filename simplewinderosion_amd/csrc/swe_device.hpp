@@ -26,11 +26,12 @@ __device__ __forceinline__ uint32_t f2u(float f) { return __float_as_uint(f); }
 // rounds to an integer, ties to even, and the integer is the sum's encoding
 // minus the constant's -- four instructions in place of the fourteen of a
 // float -> int64 conversion.
+__device__ __forceinline__ int64_t fx_from_small_f32(float v) {  // |v| < 2^18
+  const double d = (double)(v * 4294967296.0f) + 6755399441055744.0;
+  return (int64_t)((uint64_t)__double_as_longlong(d) - 0x4338000000000000ull);
+}
 __device__ __forceinline__ int64_t fx_from_f32(float v) {
-  if (__builtin_expect(__builtin_fabsf(v) < 262144.0f, 1)) {
-    const double d = (double)(v * 4294967296.0f) + 6755399441055744.0;
-    return (int64_t)((uint64_t)__double_as_longlong(d) - 0x4338000000000000ull);
-  }
+  if (__builtin_expect(__builtin_fabsf(v) < 262144.0f, 1)) return fx_from_small_f32(v);
   if (!(__builtin_fabsf(v) < 2147483648.0f)) return v != v ? 0 : (v < 0.0f ? INT64_MIN : INT64_MAX);
   return (int64_t)(v * 4294967296.0f);  // a float of 2^18 or more is a multiple of 2^-5
 }
@@ -39,6 +40,18 @@ __device__ __forceinline__ int64_t fx_from_f32(float v) {
 // rounds to nearest even, and the power-of-two scale is exact (|m| >= 1
 // keeps the result far from the denormal range).
 __device__ __forceinline__ float f32_from_fx(int64_t m) { return (float)m * 2.3283064365386963e-10f; }
+
+// The same for |m| < 2^47: the part above the lowest 24 bits and those 24
+// bits each convert exactly, and one fused multiply-add rounds their scaled
+// sum (six instructions, none 64-bit, for eleven).
+__device__ __forceinline__ float f32_from_small_fx(int64_t m) {
+  const float hi = (float)(int32_t)__builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, 24);
+  const float lo = (float)((uint32_t)m & 0xffffffu);
+  return __builtin_fmaf(hi, 0x1p-8f, lo * 0x1p-32f);
+}
+__device__ __forceinline__ bool small_fx(int64_t m) {  // -2^39 <= m < 2^39
+  return (uint32_t)((int32_t)(m >> 32) + 128) < 256u;
+}
 
 // exp for float32: Cody-Waite reduction with a two-part ln2, degree-7
 // Taylor polynomial in Horner form, exact power-of-two scaling (two steps,

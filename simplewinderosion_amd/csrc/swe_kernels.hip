@@ -246,7 +246,9 @@ __global__ __launch_bounds__(kRelaxThreads) void k_relax(RelaxArgs a) {
     const float sc = LAYERS == 2 ? shs[ic] : 0.0f;
     const auto sed_of = [&](int32_t k) { return shs[ic + off_x(k) * kHY + off_y(k)]; };
     cascade_cell_dev<LAYERS>(hn, sed_of, hc, sc, valid, settle_factor_dev(a.settling, v), a.maxdiff,
-                             [&](int32_t k, int64_t amt) { out[k] = amt; });
+                             [&](int32_t k, int64_t amt) {
+                               if (amt != 0) out[k] = amt;
+                             });
   }
   __syncthreads();
 

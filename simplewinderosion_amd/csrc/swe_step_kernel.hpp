@@ -88,6 +88,7 @@ __device__ __forceinline__ int32_t wrapt(int32_t v, int32_t n) {
 // phase takes the pointer through step_args, which the compiler cannot see
 // through, so its loads are not moved above it.
 typedef const __attribute__((address_space(4))) StepArgs* StepArgsPtr;
+typedef const __attribute__((address_space(4))) Terrain* TerrainPtr;
 __device__ __forceinline__ StepArgsPtr step_args(StepArgsPtr p) {
   asm volatile("" : "+s"(p));
   return p;
@@ -131,7 +132,8 @@ __device__ __forceinline__ void step_body() {
   __shared__ uint32_t s_ncas;        // cells whose cascade moves material
   __shared__ uint32_t s_ccnt[COLOUR ? 32 : 1];  // visited cells per colour class
   __shared__ uint32_t s_cpre[COLOUR ? 33 : 1];  // exclusive prefix of s_ccnt
-  __shared__ uint32_t s_more[2];                // a cell is still waiting (by round parity)
+  __shared__ uint32_t s_nready[2];              // cells listed in a round (by parity)
+  __shared__ uint32_t s_large;                  // the region holds a master of 2^39 or more
 
   // XCD-aware order (workgroup b runs on XCD b % 8).  tile_order 0: XCD k
   // takes a contiguous range of tiles, so neighbouring tiles share halo
@@ -149,9 +151,6 @@ __device__ __forceinline__ void step_body() {
   const uint32_t ls = RELAX_ONLY ? 0u : (uint32_t)ap->light_slots;
   const uint32_t nb = (uint32_t)ap->default_slots, b = blockIdx.x - (uint32_t)ap->heavy_slots;
   const uint32_t xcd = b % 8;
-  // a single map's terrain record does not depend on the tile: its load goes
-  // out with the slot's list or stamp loads below, not after them
-  const Terrain T1 = ap->terr[0];
   int32_t u;  // global tile
   bool listed = false;
   if (blockIdx.x < (uint32_t)ap->heavy_slots) {
@@ -194,16 +193,17 @@ __device__ __forceinline__ void step_body() {
   // before it loads anything
   if ((hs | ls) > 0 && !listed && ap->hstamp[u] > (uint32_t)ap->window) return;
   // the terrain this tile belongs to; all map indices below are terrain-local
-  Terrain T = T1;
-  if (ap->nterr != 1) T = ap->terr[ap->tile_terrain[u]];
-  const int32_t nx = T.nx, ny = T.ny;
-  const int32_t tiles_x = T.tiles_x, tiles_y = T.tiles_y;
-  const int32_t t0 = T.tile0;
+  // (a single map's record is among the arguments: no dependent load)
+  TerrainPtr tp = &ap->t0;
+  if (ap->nterr != 1) tp = (TerrainPtr)(uintptr_t)(ap->terr + ap->tile_terrain[u]);
+  const int32_t nx = tp->nx, ny = tp->ny;
+  const int32_t tiles_x = tp->tiles_x, tiles_y = tp->tiles_y;
+  const int32_t t0 = tp->tile0;
   const int32_t ul = u - t0;
   const int32_t tx = ul / tiles_y, ty = ul % tiles_y;
   const int32_t x0 = tx * kSX, y0 = ty * kSY;
-  const float rcp_nx = T.rcp_nx, rcp_ny = T.rcp_ny;
-  const int64_t c0 = T.cell0;
+  const float rcp_nx = tp->rcp_nx, rcp_ny = tp->rcp_ny;
+  const int64_t c0 = tp->cell0;
   const int64_t* zm_in = ap->zm_in + c0;
   const float* snap_in = ap->snap_in + c0;
   float* snap_out = ap->snap_out + c0;
@@ -239,6 +239,9 @@ __device__ __forceinline__ void step_body() {
     if (t < u) part_n = ap->nin_cur[t];
   }
   const uint32_t nin_u = RELAX_ONLY ? 0u : ap->nin_cur[u];
+  // read here, so that the particle phase does not start by waiting for them
+  const uint64_t cycle = RELAX_ONLY ? 0u : *ap->cycle;
+  const uint32_t far_n = RELAX_ONLY ? 0u : *ap->far_cnt_in;
 
   PRec rec0{};       // this thread's first arrival (loaded in the relax phase)
   uint32_t sr0 = 0;  // its sub-range
@@ -359,13 +362,14 @@ __device__ __forceinline__ void step_body() {
     uint32_t* v_r = (uint32_t*)(z_r + R * LAYERS);
     uint16_t* list = (uint16_t*)(v_r + R);
     // class of a visited cell whose cascade has not run yet (1 ..), else 0;
-    // one row and two cells of zeros before and after it, so that the 5 x 5
-    // neighbourhood of any listed cell can be read
-    uint8_t* cls = (uint8_t*)(list + R) + RY + 2;
+    // a row and eight cells of zeros before and after it, so that the 5 x 5
+    // neighbourhood of any listed cell can be read in eight-byte rows
+    uint8_t* cls = (uint8_t*)(list + R) + RY + 8;
     if (threadIdx.x < 32) s_ccnt[threadIdx.x] = 0;
-    if (threadIdx.x < 2) s_more[threadIdx.x] = 0;
-    for (int32_t e = threadIdx.x; e < RY + 2; e += kStepThreads) {
-      cls[e - RY - 2] = 0;
+    if (threadIdx.x < 2) s_nready[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_large = 0;
+    for (int32_t e = threadIdx.x; e < RY + 8; e += kStepThreads) {
+      cls[e - RY - 8] = 0;
       cls[R + e] = 0;
     }
     // region row of index e (e < 2^16: the product is within 1/2 of a step of exact)
@@ -380,7 +384,9 @@ __device__ __forceinline__ void step_body() {
     constexpr int kChunks = (kSY + kColourHaloMax.yl + kColourHaloMax.yh + 63) / 64;
     constexpr int kB = kRows < 8 ? kRows : 8;  // rows a wave has in flight
     const int32_t wv = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x >> 6), lane = (int32_t)threadIdx.x & 63;
-    uint32_t where[kChunks][kRows];  // class << 16 | rank within it; 0: not listed
+    uint32_t where[kChunks][kRows];  // class << 16 | rank in the wave's part of it; 0: not listed
+    uint32_t wcnt = 0;
+    bool large = false;  // a master the quick conversion below cannot take
     __syncthreads();
 #pragma unroll
     for (int cc = 0; cc < kChunks; cc++) {
@@ -431,26 +437,28 @@ __device__ __forceinline__ void step_body() {
             z_r[e] = zv[j];
             if (LAYERS == 2) s_r[e] = sv[j];
             v_r[e] = vv[j];
+            large = large || !small_fx(zv[j]) || (LAYERS == 2 && !small_fx(sv[j]));
             cls[e] = (uint8_t)(act ? cv : 0);
           }
-          // rank within the class: one counter update per wave and class
+          // rank within the wave's cells of the class (lane c of wcnt counts class c)
           uint64_t rem = __ballot(act);
           while (rem) {
-            const int32_t l = __builtin_ctzll(rem);
-            const int32_t c = __builtin_amdgcn_readlane(cv, l);
+            const int32_t c = __builtin_amdgcn_readlane(cv, __builtin_ctzll(rem));
             const bool in = act && cv == c;
             const uint64_t m = __ballot(in);
-            uint32_t base = 0;
-            if (lane == l) base = atomicAdd(&s_ccnt[c], (uint32_t)__popcll(m));
-            base = __builtin_amdgcn_readlane(base, l);
+            const uint32_t base = __builtin_amdgcn_readlane(wcnt, c);
             const uint32_t below =
                 __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
             if (in) where[cc][b0 + j] = (uint32_t)c << 16 | (base + below);
+            if (lane == c) wcnt += (uint32_t)__popcll(m);
             rem &= ~m;
           }
         }
       }
     }
+    // this wave's part of each class's list starts at wcnt
+    if (lane < 32) wcnt = wcnt ? atomicAdd(&s_ccnt[lane], wcnt) : 0u;
+    if (__ballot(large) && lane == 0) s_large = 1;
     __syncthreads();
     prefix_arrivals();
     if (threadIdx.x >= kStepThreads - 64) {  // the last wave: prefix over the classes
@@ -470,99 +478,154 @@ __device__ __forceinline__ void step_body() {
     for (int cc = 0; cc < kChunks; cc++)
 #pragma unroll
       for (int i = 0; i < kRows; i++)
-        if (where[cc][i])
-          list[s_cpre[where[cc][i] >> 16] + (where[cc][i] & 0xffffu)] =
-              (uint16_t)((wv + i * kWaves) * RY + 64 * cc + lane);
+        if (__ballot(where[cc][i] != 0)) {
+          const uint32_t w = where[cc][i], base = __shfl(wcnt, (int)(w >> 16), 64);
+          if (w)
+            list[s_cpre[w >> 16] + base + (w & 0xffffu)] = (uint16_t)((wv + i * kWaves) * RY + 64 * cc + lane);
+        }
     const uint32_t nvis = s_cpre[32];
     if (!RELAX_ONLY) first_arrival();
     __syncthreads();
 
+    // Masters below 2^39 at the start (heights below 128) stay below 2^47
+    // through the relax: with settling in [0, 1] a transfer is at most half
+    // the difference of the two heights, so heights stay within the region's
+    // range, and a cell's sediment sees at most 8 x 25 transfers.  Those take
+    // the short conversion.
+    const bool quick = s_large == 0 && ap->settling >= 0.0f && ap->settling <= 1.0f;
     // one cell's cascade on the LDS masters
     auto relax = [&](int32_t e) __attribute__((always_inline)) {
       const int32_t lx = row_of(e), ly = e - lx * RY;
       const int32_t gx = x0 - hl.xl + lx, gy = y0 - hl.yl + ly;
-      const float hc = f32_from_fx(z_r[e]);
+      int64_t zn[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) zn[k] = z_r[e + c_ox[k] * RY + c_oy[k]];
+      const int64_t zc = z_r[e];
+      float hc = f32_from_small_fx(zc);
       float hn[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) hn[k] = f32_from_small_fx(zn[k]);
+      if (!quick) {
+        hc = f32_from_fx(zc);
+#pragma unroll
+        for (int k = 0; k < 8; k++) hn[k] = f32_from_fx(zn[k]);
+      }
       uint32_t valid = 0;
-      bool act = false;
+      // no neighbour beyond the threshold: the walk moves nothing
+      float most = -1.0f;
       const float dd = __builtin_sqrtf(2.0f);
 #pragma unroll
       for (int k = 0; k < 8; k++) {
-        hn[k] = f32_from_fx(z_r[e + c_ox[k] * RY + c_oy[k]]);
         bool ok = true;
         if (!PERIODIC) {
           const int32_t qx = gx + c_ox[k], qy = gy + c_oy[k];
           ok = qx >= 0 && qy >= 0 && qx < nx && qy < ny;
         }
         valid |= (ok ? 1u : 0u) << k;
-        const float diff = hc - hn[k];
+        const float ad = __builtin_fabsf(hc - hn[k]);
         const float d = (c_ox[k] != 0 && c_oy[k] != 0) ? dd : 1.0f;
-        const float excess = __builtin_fabsf(diff) - (d * ap->maxdiff) * 1.0f;
-        act = act || (ok && diff != 0.0f && !(excess <= 0.0f));
+        const float m = __builtin_fminf(ad - (d * ap->maxdiff) * 1.0f, ad);
+        most = __builtin_fmaxf(most, ok ? m : -1.0f);
       }
-      if (!act) return;  // no neighbour beyond the threshold: the walk moves nothing
-      const auto sed_of = [&](int32_t k) { return f32_from_fx(s_r[e + off_x(k) * RY + off_y(k)]); };
+      if (!(most > 0.0f)) return;
+      const auto sed_at = [&](int32_t q) __attribute__((always_inline)) {
+        const int64_t m = s_r[q];
+        float f = f32_from_small_fx(m);
+        if (!quick) f = f32_from_fx(m);
+        return f;
+      };
+      const auto sed_of = [&](int32_t k) { return sed_at(e + off_x(k) * RY + off_y(k)); };
       int64_t centre = 0;
-      cascade_cell_dev<LAYERS>(hn, sed_of, hc, LAYERS == 2 ? f32_from_fx(s_r[e]) : 0.0f, valid,
-                               settle_factor_dev(ap->settling, v_r[e]), ap->maxdiff, [&](int32_t k, int64_t amt) {
+      cascade_cell_dev<LAYERS>(hn, sed_of, hc, LAYERS == 2 ? sed_at(e) : 0.0f, valid,
+                               u2f(v_r[e]), ap->maxdiff, [&](int32_t k, int64_t amt) {
                                  centre -= amt;
                                  const int32_t q = e + off_x(k) * RY + off_y(k);
-                                 z_r[q] += amt;
-                                 if (LAYERS == 2) s_r[q] += amt;
+                                 // no other cell in flight touches q: the atomics only save the reads' wait
+                                 if (amt != 0) {
+                                   atomicAdd((unsigned long long*)&z_r[q], (unsigned long long)amt);
+                                   if (LAYERS == 2) atomicAdd((unsigned long long*)&s_r[q], (unsigned long long)amt);
+                                 }
                                });
-      z_r[e] += centre;
-      if (LAYERS == 2) s_r[e] += centre;
+      atomicAdd((unsigned long long*)&z_r[e], (unsigned long long)centre);
+      if (LAYERS == 2) atomicAdd((unsigned long long*)&s_r[e], (unsigned long long)centre);
     };
-    // Few visited cells (at most one a thread): each thread holds one and runs
-    // its cascade as soon as no visited cell of an earlier class within two
-    // cells is waiting (cells further apart share no neighbour, and of two
-    // closer ones the earlier class goes first).  Dependences run down the
-    // classes, so at most as many rounds as classes; scattered cells need
-    // two or three.  Many: one class after another, a thread a cell.
-    const bool few = nvis <= (uint32_t)kStepThreads;
-    bool pend = few && threadIdx.x < nvis;
-    const int32_t own = pend ? list[threadIdx.x] : 0;
-    const uint8_t own_cls = pend ? cls[own] : 0;
-    int32_t c = 0;               // class of the current chunk (many)
-    uint32_t pos = 0, end = 0;   // its unread part of the list
-    for (int32_t round = 0; !few || round < kColourAxisMax * kColourAxisMax; round++) {
-      int32_t e = -1;
+    // Up to two visited cells a thread: in rounds, every cell that no visited
+    // cell of an earlier class within two cells still precedes is listed
+    // (cells further apart share no neighbour, and of two closer ones the
+    // earlier class goes first), and the listed cells run on packed waves.
+    // Dependences run down the classes, so there are at most as many rounds as
+    // classes; scattered cells need two or three.  More cells: one class after
+    // another.
+    constexpr int kClasses = kColourAxisMax * kColourAxisMax;
+    const bool few = nvis <= 2u * kStepThreads;
+    const bool have0 = threadIdx.x < nvis, have1 = threadIdx.x + kStepThreads < nvis;
+    const int32_t own0 = few && have0 ? list[threadIdx.x] : 0;
+    const int32_t own1 = few && have1 ? list[threadIdx.x + kStepThreads] : 0;
+    uint32_t pend = few ? (have0 ? 1u : 0u) | (have1 ? 2u : 0u) : 0u;
+    uint32_t done = 0;
+    // the visited cells' settling factors, in place of their events
+    for (uint32_t i = threadIdx.x; i < nvis; i += kStepThreads) {
+      const int32_t e = list[i];
+      v_r[e] = f2u(settle_factor_dev(ap->settling, v_r[e]));
+    }
+    __syncthreads();  // (the list is in registers too: its storage takes the rounds' cells)
+    for (int32_t round = 0; round < kClasses; round++) {
+      const uint16_t* run = list;
+      uint32_t n;
       if (few) {
-        if (pend) {
-          const uint8_t* p = cls + own;
-          bool ready = true;
+        for (int q = 0; q < 2; q++) {
+          bool ready = false;
+          const int32_t e = q == 0 ? own0 : own1;
+          if (pend & (1u << q)) {
+            // the five rows of its neighbourhood, five cells each: no byte o
+            // with 0 < o < mine (bytes are below 128, so per-byte sums and
+            // differences do not carry)
+            const uint8_t* p = cls + e - 2;
+            const uint32_t mine = p[2] * 0x01010101u;
+            uint32_t w[5], x[5];
 #pragma unroll
-          for (int dx = -2; dx <= 2; dx++)
-#pragma unroll
-            for (int dy = -2; dy <= 2; dy++) {
-              if (dx == 0 && dy == 0) continue;
-              const uint8_t o = p[dx * RY + dy];
-              ready = ready && (o == 0 || o >= own_cls);
+            for (int dx = 0; dx < 5; dx++) {
+              __builtin_memcpy(&w[dx], p + (dx - 2) * RY, 4);
+              x[dx] = p[(dx - 2) * RY + 4];
             }
-          if (ready) e = own;
+            const uint32_t xs = x[0] | x[1] << 8 | x[3] << 16 | x[4] << 24;
+            uint32_t before = 0;
+#pragma unroll
+            for (int i = 0; i < 7; i++) {
+              const uint32_t o = i < 5 ? w[i] : (i == 5 ? xs : x[2]);
+              before |= ~((o | 0x80808080u) - mine) & (o + 0x7f7f7f7fu);
+            }
+            ready = (before & 0x80808080u) == 0;
+          }
+          const uint64_t m = __ballot(ready);
+          if (m) {
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&s_nready[round & 1], (uint32_t)__popcll(m));
+            base = __builtin_amdgcn_readfirstlane(base);
+            if (ready) {
+              list[base + below] = (uint16_t)e;
+              pend &= ~(1u << q);
+            }
+          }
+          if (nvis <= (uint32_t)kStepThreads) break;
         }
-        if (threadIdx.x == 0) s_more[round & 1] = 0;
         __syncthreads();
+        n = s_nready[round & 1];
+        if (threadIdx.x == 0) s_nready[(round & 1) ^ 1] = 0;
       } else {
-        while (pos >= end && c < kColourAxisMax * kColourAxisMax) {
-          c++;
-          pos = s_cpre[c];
-          end = pos + s_ccnt[c];
-        }
-        if (pos >= end) break;
-        if (pos + threadIdx.x < end) e = list[pos + threadIdx.x];
-        pos += kStepThreads;
+        n = s_ccnt[round + 1];
+        if (n == 0) continue;
+        run = list + s_cpre[round + 1];
       }
-      if (e >= 0) relax(e);
-      if (few) {
-        if (e >= 0) {
-          cls[e] = 0;
-          pend = false;
-        }
-        if (pend) s_more[round & 1] = 1;
+      for (uint32_t i = threadIdx.x; i < n; i += kStepThreads) {
+        const int32_t e = run[i];
+        relax(e);
+        cls[e] = 0;
       }
       __syncthreads();
-      if (few && s_more[round & 1] == 0) break;
+      done += n;
+      if (done >= nvis) break;
     }
 
     // the relaxed masters of the tile and its one-cell halo; the sediment
@@ -822,6 +885,7 @@ __device__ __forceinline__ void step_body() {
 
   // ---------------- 2. particles of the tile ----------------
   ap = step_args(ap);
+  asm volatile("" : "+s"(tp));
   int64_t* acc_d = (int64_t*)s_work;
   int64_t* acc_ds = acc_d + kCell;  // LAYERS == 2
   uint32_t* acc_v = (uint32_t*)(acc_d + kCell * (LAYERS == 2 ? 2 : 1));
@@ -851,12 +915,11 @@ __device__ __forceinline__ void step_body() {
     k.suspension = ap->suspension;
     k.gravity = ap->gravity;
     k.abrasion = ap->abrasion;
-    k.ps = mk(T.ps[0], T.ps[1], T.ps[2]);
-    k.nps = mk(T.nps[0], T.nps[1], T.nps[2]);
-    const uint64_t ck = cycle_key(T.seed, *ap->cycle);
-    const int64_t p0 = T.part0;
+    k.ps = mk(tp->ps[0], tp->ps[1], tp->ps[2]);
+    k.nps = mk(tp->nps[0], tp->nps[1], tp->nps[2]);
+    const uint64_t ck = cycle_key(tp->seed, cycle);
+    const int64_t p0 = tp->part0;
     const int64_t out_base = s_base;  // 9 x the input counts of tiles 0 .. u-1
-    const uint32_t far_n = *ap->far_cnt_in;
 
     // one input record
     using Rec = PRec;
@@ -970,7 +1033,7 @@ __device__ __forceinline__ void step_body() {
     }
     for (int64_t j = threadIdx.x; j < (int64_t)far_n; j += kStepThreads) {
       const int64_t fp = (int64_t)f2u(ap->far_in[j].q1.w);
-      if (fp < p0 || fp >= p0 + T.npart) continue;  // another terrain's particle
+      if (fp < p0 || fp >= p0 + tp->npart) continue;  // another terrain's particle
       int32_t cx, cy;
       const f4a8 q0 = ap->far_in[j].q0;
       int32_t ctx, cty;
@@ -1136,9 +1199,10 @@ __device__ __forceinline__ void step_body() {
 // particles, write-out) and by vector issue within them.  Phase-wise argument
 // reads, one address per halo cell and branch-free primitives took the
 // kernel from 10,470 to 7,000 instructions (70 to 46 KB of code, past and
-// within the instruction cache) and from 18.8 to 16.2 us a window on 256^2
-// (2,000 particles), 17.2 to 13.9 us on 75 x 101 (300), 73.0 to 70.9 us on
-// 1024^2 (a million).
+// within the instruction cache); with the lists of a one-round launch dropped
+// and the cascade walk's chain shortened a window takes 14.6 us (18.8 before)
+// on 256^2 with 2,000 particles, 13.2 (17.2) on 75 x 101 with 300, and 71
+// (73) on 1024^2 with a million, where vector issue is half the time.
 template <int SX, int SY, int NT, int WPE, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_step(StepArgs) {
   step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
@@ -1150,10 +1214,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 // (9 to 25 launches, each two memory round trips: 7.5 us apiece on 512^2).
 // Redundant work is 3.4 regions per tile, but a window pays one launch and
 // one load of the region; its time is the most crowded tile's rounds of
-// dependent cascades.  Measured against the class launches: 512^2 bounded,
-// 4096 particles 46.2 -> 17.5 ms a cycle; 400 x 301 periodic, two layers,
-// 30,000 particles 85.5 -> 35.9 ms; 1024^2 with a million particles, where a
-// class launch fills the chip, 110 -> 111 ms.
+// dependent cascades (1,500 to 5,000 cycles each).  Measured against the
+// class launches: 512^2 bounded, 4096 particles 46.2 -> 12.8 ms a cycle; 400 x
+// 301 periodic, two layers, 30,000 particles 85.4 -> 28.7 ms; 1024^2 with a
+// million particles, where a class launch fills the chip, 110 -> 95 ms.
 template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colour_step(StepArgs) {
   step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
@@ -1164,7 +1228,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 template <int SX, int SY>
 inline size_t colour_lds(const ColourHalo& h, bool track, int layers) {
   const size_t ry = (size_t)(SY + h.yl + h.yh), r = (size_t)(SX + h.xl + h.xh) * ry;
-  const size_t relax = r * (8 * (size_t)layers + 4 + 2 + 1) + 2 * (ry + 2);
+  const size_t relax = r * (8 * (size_t)layers + 4 + 2 + 1) + 2 * (ry + 8);
   const size_t march = (size_t)SX * SY * (8 * (size_t)layers + 4 + (track ? 32 : 0));
   return ((relax > march ? relax : march) + 15) & ~(size_t)15;
 }
