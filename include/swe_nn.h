@@ -28,11 +28,11 @@ int swe_nn_conv3x3(const void* x, int32_t N, int32_t H, int32_t W, int32_t Cin, 
 int swe_nn_conv3x3_masked(const void* x, int32_t N, int32_t H, int32_t W, int32_t Cin, const void* w,
                           const float* bias, int32_t Cout, const void* mask, void* y16, void* stream);
 /* The same convolution with a caller's workspace: act 0 none, 1 ReLU, 2
- * zero where mask <= 0.  Layers with few pixel blocks and a long reduction
- * (low resolutions, many channels) split the reduction over up to 8
- * workgroups per block, whose partial sums (work: swe_nn_conv3x3_work
- * floats, 0 when the layer is not split) are added in a fixed order; with
- * less work than that the layer runs unsplit. */
+ * zero where mask <= 0.  Layers with few
+ * pixel blocks and a long reduction (low resolutions, many channels) sum it
+ * in up to 8 slices that are added in a fixed order when `work` holds
+ * swe_nn_conv3x3_work floats (0 when the layer is not split), and in one
+ * chain with less; nothing is written to `work`. */
 int64_t swe_nn_conv3x3_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout);
 int swe_nn_conv3x3_ws(const void* x, int32_t N, int32_t H, int32_t W, int32_t Cin, const void* w, const float* bias,
                       int32_t Cout, int32_t act, const void* mask, void* y16, float* y32, float* work,

@@ -26,361 +26,467 @@ __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }  // round to n
 
 __device__ __forceinline__ int32_t wrapi(int32_t v, int32_t n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
-// three offsets picked by a wave-uniform index in 0..2
-struct Off3 {
-  uint32_t v0, v1, v2;
-  __device__ __forceinline__ uint32_t at(int32_t i) const { return i == 0 ? v0 : (i == 1 ? v1 : v2); }
-};
+// Epilogue of the tile kernels: bias, ACT (0 none, 1 ReLU, 2 zero where mask
+// <= 0) and the stores of a wave's PF x CF result fragments for the tile at
+// (y0, x0) of image n.
+template <int PF, int CF, int S, int ACT>
+__device__ __forceinline__ void conv_store(const f32x4 (&acc)[PF][CF], const float* s_bias,
+                                           const bf16* __restrict__ mask, bf16* __restrict__ y16,
+                                           float* __restrict__ y32, int32_t n, int32_t y0, int32_t x0, int32_t H,
+                                           int32_t W, int32_t Cout, int32_t co0, int32_t vec) {
+  constexpr int CP = CF == 1 ? 1 : CF / 2;  // output vectors a lane holds per pixel
+  constexpr int CV = CF == 1 ? 4 : 8;       // channels of one
+  const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rl = lane & 15, g = lane >> 4;
+  // output positions of this lane: pixel rl of each fragment
+  int32_t po[PF];
+#pragma unroll
+  for (int f = 0; f < PF; f++) {
+    const int32_t idx = wave * PF + f, yy = y0 + idx / S, xx = x0 + 16 * (idx % S) + rl;
+    po[f] = yy < H && xx < W ? (n * H + yy) * W + xx : -1;
+  }
+  typedef bf16 bf16v __attribute__((ext_vector_type(CV)));
+  bf16v mk[ACT == 2 ? PF : 1][ACT == 2 ? CP : 1];
+  if (ACT == 2 && vec) {  // every mask load in flight at once
+#pragma unroll
+    for (int f = 0; f < PF; f++)
+#pragma unroll
+      for (int q = 0; q < CP; q++) {
+        const int32_t co = co0 + 32 * q + CV * g;
+        if (po[f] >= 0 && co < Cout) mk[f][q] = *(const bf16v*)(mask + (int64_t)po[f] * Cout + co);
+      }
+  }
+#pragma unroll
+  for (int f = 0; f < PF; f++) {
+    if (po[f] < 0) continue;
+#pragma unroll
+    for (int q = 0; q < CP; q++) {
+      const int32_t co = co0 + 32 * q + CV * g;
+      if (co >= Cout) continue;
+      float v[CV];
+#pragma unroll
+      for (int e = 0; e < CV; e++) {
+        v[e] = acc[f][CF == 1 ? 0 : 2 * q + e / 4][e % 4] + s_bias[32 * q + CV * g + e];
+        if (ACT == 1) v[e] = v[e] > 0.0f ? v[e] : 0.0f;
+      }
+      const int64_t o = (int64_t)po[f] * Cout + co;
+      if (vec) {
+        // all CV channels lie below Cout and the vectors are aligned
+        if (ACT == 2) {
+#pragma unroll
+          for (int e = 0; e < CV; e++) v[e] = bf2f(mk[f][q][e]) > 0.0f ? v[e] : 0.0f;
+        }
+        if (y16) {
+          bf16v r;
+#pragma unroll
+          for (int e = 0; e < CV; e++) r[e] = f2bf(v[e]);
+          *(bf16v*)(y16 + o) = r;
+        }
+        if (y32) {
+#pragma unroll
+          for (int e = 0; e < CV; e += 4) *(f32x4*)(y32 + o + e) = (f32x4){v[e], v[e + 1], v[e + 2], v[e + 3]};
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < CV; e++) {
+          if (co + e >= Cout) continue;
+          if (ACT == 2) v[e] = bf2f(mask[o + e]) > 0.0f ? v[e] : 0.0f;
+          if (y16) y16[o + e] = f2bf(v[e]);
+          if (y32) y32[o + e] = v[e];
+        }
+      }
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------
-// 3x3 convolution, implicit GEMM: rows = pixels (the batch's pixels
-// flattened, n-major), columns = output channels, reduction k = tap * Cin +
-// ci in steps of 32 (one tap, 32 input channels; channels at or beyond Cin
-// read as zero, so any Cin % 8 == 0 works).  A workgroup (4 waves) owns 128
-// pixels x NT output channels.  Each step's A block [128][32] (the pixels
-// shifted by the tap, periodic) and B block [NT][32] are staged in LDS,
-// double buffered with rows padded to 40 elements: every thread loads its
-// 16-byte runs of the next step into registers while the waves run the
-// current step's MFMAs, then stores them into the other buffer (one barrier
-// per step).  Waves tile the block 2 x 2 (NT >= 64) or 4 x 1; per
-// v_mfma_f32_16x16x32_bf16, lane l supplies A row l%16 and B row l%16, both
-// at k = 8*(l/16) .. +7, and holds D rows 4*(l/16) .. +3 of column l%16.
-// A step issues only 8 MFMAs a wave, so its loop, address and barrier work
-// is what the step costs: no step divides, and addresses are 32-bit.
+// 3x3 convolution over rectangular tiles: a workgroup (4 waves) owns 64 PF
+// pixels (4 PF / S rows of 16 S columns of one image) x 16 CF output
+// channels.  This kernel takes up to 32 input channels: the weights of all
+// nine taps are staged in LDS once, then for each of the workgroup's `per`
+// consecutive tiles the input patch (the tile and its one-pixel periodic
+// halo, read once for all nine taps); the next tile's loads are in flight
+// while the waves compute.
+// LDS rows are one pixel (one output channel of one tap) of 32 channels, 64
+// bytes at a stride of 80, so that the 16 rows a fragment read touches fall
+// in different banks and a tap is an immediate offset.
+//
+// The weights are the MFMA's A operand and the pixels its B operand, so a
+// lane's four results are four output channels of one pixel.  Two fragments
+// interleave their rows (row r of fragment j is channel 8 (r / 4) + 4 j +
+// r % 4 of their 32), which leaves a lane with eight consecutive channels:
+// one 16-byte store (and mask load) where a pixel-major result takes eight
+// two-byte ones.  Each wave takes PF fragments of 16 pixels and all CF of
+// channels: PF + CF reads of 1 KB for PF CF MFMAs.
+//
+// Tiles are dealt so that each XCD (workgroup b runs on XCD b % 8) gets a
+// contiguous range with all its channel blocks.
+//
+// Bound: memory at full resolution (32 -> 32 moves 67 MB, 100 with a mask).
+// Against a row-streamed kernel with pixel-major results (us, batch 8): 32 ->
+// 32 at 256^2 25.3 -> 20.6, its masked data gradient 31.0 -> 24.3; 8 -> 32
+// 25.2 -> 19.9; 32 -> 16 20.6 -> 13.5; 32 -> 32 at 200 x 230, batch 3, 13.0 ->
+// 10.1.
 // ---------------------------------------------------------------------------
-// ACT 0: none, 1: ReLU, 2: zero where mask <= 0 (the ReLU gradient of a
-// data gradient through the layer below, mask = that layer's output).
-// With part, workgroup z of gridDim.z takes the k-steps [z K / Z, (z + 1) K /
-// Z) and stores its raw sums in part[z][pixel][channel] (k_conv_reduce adds
-// the Z partials in order and applies the epilogue): split-K for layers with
-// few pixel blocks, whose workgroups would otherwise each walk every k-step.
-template <int NT, int ACT>
-__global__ __launch_bounds__(256) void k_conv3x3(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                 const float* __restrict__ bias, const bf16* __restrict__ mask,
-                                                 bf16* __restrict__ y16, float* __restrict__ y32, int32_t N,
-                                                 int32_t H, int32_t W, int32_t Cin, int32_t Cout,
-                                                 float* __restrict__ part) {
-  constexpr int WM = NT >= 64 ? 2 : 4;  // waves along the pixels
-  constexpr int WN = 4 / WM;            // ... and the channels
-  constexpr int TM = 128 / WM, TN = NT / WN;
-  constexpr int BM = TM / 16, BN = TN / 16;
-  constexpr int KC = 32, LD = KC + 8;
-  __shared__ __attribute__((aligned(16))) bf16 sA[2][128 * LD];
-  __shared__ __attribute__((aligned(16))) bf16 sB[2][NT * LD];
+// waves per SIMD that the LDS of a shape leaves room for, and its register budget
+// (the 16-channel shape fits four waves' registers but for two)
+constexpr int conv_tile_waves(int pf, int cf) { return cf == 4 ? 2 : (pf == 4 && cf == 2 ? 3 : 4); }
+constexpr int conv_tile_budget(int pf, int cf) { return cf == 1 ? 3 : conv_tile_waves(pf, cf); }
+
+template <int PF, int CF, int S, int ACT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_tile_budget(PF, CF)))) void k_conv_tile(
+    const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ bias,
+    const bf16* __restrict__ mask, bf16* __restrict__ y16, float* __restrict__ y32, int32_t N, int32_t H, int32_t W,
+    int32_t Cin, int32_t Cout, int32_t per, int32_t vec) {
+  constexpr int TW = 16 * S, TH = 4 * PF / S;  // tile columns, rows
+  constexpr int PW = TW + 2, PH = TH + 2;      // patch
+  constexpr int LD = 40;                       // LDS row stride (elements)
+  constexpr int AI = PW * PH * 4, AP = (AI + 255) / 256;    // 16-byte items of the patch, per thread
+  constexpr int BR = 9 * 16 * CF, BP = (BR * 4 + 255) / 256;  // weight rows; items per thread
+  __shared__ __attribute__((aligned(16))) bf16 s_a[PW * PH * LD];
+  __shared__ __attribute__((aligned(16))) bf16 s_b[BR * LD];
+  __shared__ __attribute__((aligned(16))) float s_bias[16 * CF];
   const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int32_t wm = wave / WN, wn = wave % WN;
-  const int64_t P = (int64_t)N * H * W;
-  const int64_t p0 = (int64_t)blockIdx.x * 128;
-  const int32_t co0 = blockIdx.y * NT;
-  const int32_t cchunks = (Cin + KC - 1) / KC, ksteps = 9 * cchunks;
-  const int32_t g = tid & 3, r0 = tid >> 2;  // loader: row r0 (+64), channel group g
+  const int32_t rl = lane & 15, g = lane >> 4, gg = tid & 3;
+  const int32_t tx = (W + TW - 1) / TW, ty = (H + TH - 1) / TH, tiles = N * ty * tx;
+  const int32_t ncob = (Cout + 16 * CF - 1) / (16 * CF);
+  const int32_t groups = (tiles + per - 1) / per;
+  // this workgroup's (tile group, channel block): XCD k takes the groups from
+  // k q + min(k, r) on
+  const uint32_t nb = gridDim.x, b = blockIdx.x, q8 = nb / 8, r8 = nb % 8, xcd = b % 8;
+  const int32_t lin = (int32_t)(xcd * q8 + (xcd < r8 ? xcd : r8) + b / 8);
+  const int32_t grp = lin / ncob, co0 = (lin - grp * ncob) * 16 * CF;
+  if (grp >= groups) return;
+  const int32_t t_first = grp * per, t_end = t_first + per < tiles ? t_first + per : tiles;
 
-  // Loads are raw buffer loads at 32-bit byte offsets (the host keeps x and
-  // w under 2 GiB): an offset at or above kBad lies beyond the buffer and
-  // reads zero, which stands for pixels past P, output channels past Cout and
-  // input channels past Cin.  Each thread keeps the byte offsets of its two
-  // A pixels' three (periodic) rows and three columns, so a step's address
-  // is two selects and an add rather than 64-bit index arithmetic.
-  // Descriptors: stride 0 (raw: offsets are bytes, checked against
-  // num_records = the buffer's size), flags word 0x00020000 = the 32-bit
-  // data format the gfx9 family's untyped buffer loads need.
+  constexpr uint32_t kBad = 0x80000000u;  // past both buffers: reads zero
+  constexpr int kRawFlags = 0x00020000;
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, (int)((int64_t)N * H * W * Cin * 2), kRawFlags);
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, (int)((int64_t)Cout * 9 * Cin * 2), kRawFlags);
+  // weight items: LDS row (tap, fragment, row) <- the channel it stands for
+  bf16x8 rb[BP];
+#pragma unroll
+  for (int h = 0; h < BP; h++) {
+    const int32_t rho = (tid + 256 * h) >> 2, t = rho / (16 * CF), jr = rho % (16 * CF), j = jr >> 4, r = jr & 15;
+    const int32_t co = co0 + (CF == 1 ? r : 32 * (j >> 1) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3));
+    const uint32_t o = rho < BR && co < Cout && 8 * gg < Cin ? (uint32_t)(((co * 9 + t) * Cin + 8 * gg) * 2) : kBad;
+    rb[h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)o, 0, 0));
+  }
+  uint32_t io[AP];  // byte offsets of the patch items of the tile being loaded
+  // on maps of at least a patch a row or column wraps at most once: an
+  // item's offset in the patch is fixed and its wraps are two compares
+  const bool big = H >= PH && W >= PW;
+  const uint32_t rowb = (uint32_t)(W * Cin * 2), imgb = (uint32_t)H * rowb;
+  auto place = [&](int32_t tile) __attribute__((always_inline)) {
+    // (the items' rows and columns are recomputed each time: held over the
+    // tiles they would take 30 registers)
+    int32_t it = tid;
+    asm volatile("" : "+v"(it));
+    const int32_t cx = tile % tx, cy = (tile / tx) % ty, n = tile / (tx * ty);
+    // (H and W may be smaller than a patch)
+    const int32_t by = (cy * TH + H - 1) % H, bx = (cx * TW + W - 1) % W;
+    if (big) {
+      const uint32_t base = (uint32_t)n * imgb + (uint32_t)by * rowb + (uint32_t)(bx * Cin * 2);
+#pragma unroll
+      for (int h = 0; h < AP; h++) {
+        const int32_t p = (it + 256 * h) >> 2, r = p / PW, c = p - r * PW;
+        uint32_t o = base + (uint32_t)r * rowb + (uint32_t)(c * Cin * 2 + 16 * gg);
+        if (r >= H - by) o -= imgb;
+        if (c >= W - bx) o -= rowb;
+        io[h] = p < PW * PH ? o : kBad;
+      }
+      return;
+    }
+#pragma unroll
+    for (int h = 0; h < AP; h++) {
+      const int32_t p = (it + 256 * h) >> 2, r = p / PW, c = p - r * PW;
+      int32_t yy = by + r, xx = bx + c;
+      if (yy >= H) yy = yy < 2 * H ? yy - H : yy % H;
+      if (xx >= W) xx = xx < 2 * W ? xx - W : xx % W;
+      io[h] = p < PW * PH ? (uint32_t)((((n * H + yy) * W + xx) * Cin + 8 * gg) * 2) : kBad;
+    }
+  };
+  bf16x8 ra[AP];
+  const bool gok = 8 * gg < Cin;
+  auto load_a = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < AP; h++)
+      ra[h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(gok ? io[h] : kBad), 0, 0));
+  };
+  auto store_a = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < AP; h++) {
+      const int32_t p = (tid + 256 * h) >> 2;
+      if (AI % 256 == 0 || p < PW * PH) *(bf16x8*)&s_a[p * LD + 8 * gg] = ra[h];
+    }
+  };
+  if (tid < 16 * CF) s_bias[tid] = bias && co0 + tid < Cout ? bias[co0 + tid] : 0.0f;
+
+  place(t_first);
+  load_a();
+#pragma unroll
+  for (int h = 0; h < BP; h++) {
+    const int32_t rho = (tid + 256 * h) >> 2;
+    if (BR * 4 % 256 == 0 || rho < BR) *(bf16x8*)&s_b[rho * LD + 8 * gg] = rb[h];
+  }
+  store_a();
+  __syncthreads();
+  // fragment addresses: pixel (row, segment) of fragment f of this wave
+  const bf16* ap[PF];
+#pragma unroll
+  for (int f = 0; f < PF; f++) {
+    const int32_t idx = wave * PF + f;
+    ap[f] = s_a + ((idx / S) * PW + 16 * (idx % S) + rl) * LD + 8 * g;
+  }
+  const bf16* bp = s_b + rl * LD + 8 * g;
+
+  for (int32_t tile = t_first; tile < t_end; tile++) {
+    f32x4 acc[PF][CF];
+#pragma unroll
+    for (int f = 0; f < PF; f++)
+#pragma unroll
+      for (int j = 0; j < CF; j++) acc[f][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    const bool more = tile + 1 < t_end;
+    if (more) {
+      place(tile + 1);
+      load_a();
+    }
+    // a row of taps at a time: unrolled over all nine, the scheduler reads
+    // fragments so far ahead that they spill
+#pragma unroll 1
+    for (int dy = 0; dy < 3; dy++) {
+      const bf16* bt = bp + dy * 3 * CF * 16 * LD;
+      const int32_t at = dy * PW * LD;
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++) {
+        bf16x8 fa[CF], fb[PF];
+#pragma unroll
+        for (int j = 0; j < CF; j++) fa[j] = *(const bf16x8*)(bt + (dx * CF + j) * 16 * LD);
+#pragma unroll
+        for (int f = 0; f < PF; f++) fb[f] = *(const bf16x8*)(ap[f] + at + dx * LD);
+#pragma unroll
+        for (int f = 0; f < PF; f++)
+#pragma unroll
+          for (int j = 0; j < CF; j++)
+            acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[j], fb[f], acc[f][j], 0, 0, 0);
+      }
+    }
+    if (more) {
+      __syncthreads();
+      store_a();
+      __syncthreads();
+    }
+    conv_store<PF, CF, S, ACT>(acc, s_bias, mask, y16, y32, tile / (tx * ty), (tile / tx) % ty * TH, tile % tx * TW, H, W,
+                               Cout, co0, vec);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same convolution for more than 32 input channels.  The tile's whole
+// patch (up to KC = 256 channels; more run as blocks of KC) stays in LDS, and
+// the weights stream through it tap by tap, two taps ahead in registers: so
+// the reduction runs tap by tap and within a tap over the 32-channel chunks,
+// the order of the implicit GEMM's k = tap Cin + channel.  With kz > 1 the
+// k-steps are summed in kz slices [z K / kz, (z + 1) K / kz) whose sums are
+// added in order (a layer given the workspace of a split reduction).
+// LDS rows are KC channels at a stride of KC + 8 elements (16 m + 4 dwords:
+// the 16 rows of a fragment read fall in different banks).
+//
+// Bound: LDS reads and the barrier a tap (PF + CF reads of 1 KB feed PF CF
+// MFMAs, two chunks' reads ahead of them; 38% of the MFMA rate a large product
+// reaches at 128 -> 128).  Against a flattened-pixel kernel that staged every
+// tap's pixels anew, with the split reduction's partial sums through memory
+// (us, batch 8, forward / masked data gradient): 64 -> 64 at 128^2 28.4 / 33.5
+// -> 20.4 / 23.7; 128 -> 128 at 64^2 27.6 / 32.2 -> 18.3 / 18.9; 192 -> 192 at
+// 32^2 28.4 / 28.0 -> 17.8 / 18.5; 256 -> 192 at 16^2 18.6 / 17.1 -> 14.0 /
+// 11.9; 64 -> 64 at 512^2, batch 1, 50.9 / 63.9 -> 40.3 / 42.9.  Reading one
+// chunk ahead across the taps' barriers took 10% longer (spills at 4 x 4).
+// ---------------------------------------------------------------------------
+// 32-channel chunks of a block at most: KC <= 256, for the largest workgroups
+// 192 (their patch of more would not fit the LDS)
+constexpr int conv_wide_chunks(int pf, int cf) { return pf * cf > 8 ? 6 : 8; }
+
+template <int PF, int CF, int S, int ACT, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT && PF * CF > 4 ? 1 : 2))) void k_conv_wide(
+    const bf16* __restrict__ x, const bf16* __restrict__ w, const float* __restrict__ bias,
+    const bf16* __restrict__ mask, bf16* __restrict__ y16, float* __restrict__ y32, int32_t N, int32_t H, int32_t W,
+    int32_t Cin, int32_t Cout, int32_t KC, int32_t kz, int32_t two, int32_t vec) {
+  constexpr int TW = 16 * S, TH = 4 * PF / S, PW = TW + 2, PH = TH + 2, NP = PW * PH;
+  constexpr int AP = (NP + 63) / 64;                // patch pixels per thread quad
+  constexpr int RB = 16 * CF;                       // weight rows of a tap
+  constexpr int QB = 64 / RB;                       // chunks the 64 quads load at once
+  constexpr int BP = (conv_wide_chunks(PF, CF) + QB - 1) / QB;  // weight loads a thread holds of one tap
+  extern __shared__ __attribute__((aligned(16))) bf16 s_wide[];
+  const int32_t LD = KC + 8, nc = KC / 32;
+  bf16* s_a = s_wide;
+  bf16* s_b = s_wide + NP * LD;
+  float* s_bias = (float*)(s_b + (two ? 2 : 1) * RB * LD);
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t rl = lane & 15, g = lane >> 4, gg = tid & 3, quad = tid >> 2;
+  const int32_t tx = (W + TW - 1) / TW, ty = (H + TH - 1) / TH;
+  const int32_t ncob = (Cout + RB - 1) / RB;
+  const uint32_t nb = gridDim.x, b = blockIdx.x, q8 = nb / 8, r8 = nb % 8, xcd = b % 8;
+  const int32_t lin = (int32_t)(xcd * q8 + (xcd < r8 ? xcd : r8) + b / 8);
+  const int32_t tile = lin / ncob, co0 = (lin - tile * ncob) * RB;
+  const int32_t cx = tile % tx, cy = (tile / tx) % ty, n = tile / (tx * ty);
+
   constexpr uint32_t kBad = 0x80000000u;
   constexpr int kRawFlags = 0x00020000;
   const __amdgpu_buffer_rsrc_t xr =
-      __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, (int)(P * Cin * 2), kRawFlags);
+      __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, (int)((int64_t)N * H * W * Cin * 2), kRawFlags);
   const __amdgpu_buffer_rsrc_t wr =
       __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, (int)((int64_t)Cout * 9 * Cin * 2), kRawFlags);
-  Off3 rowo[2], colo[2];  // named fields, not arrays: a select between them stays in registers
-  uint32_t wo[2];
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const int64_t p = p0 + r0 + 64 * h;
-    const bool ok = p < P;
-    const int64_t pc = ok ? p : 0;
-    const int32_t ax = (int32_t)(pc % W), ay = (int32_t)((pc / W) % H), ai = (int32_t)(pc / ((int64_t)W * H));
-    auto row = [&](int32_t d) { return ok ? (uint32_t)(((int64_t)ai * H + wrapi(ay + d, H)) * W * Cin * 2) : kBad; };
-    auto col = [&](int32_t d) { return (uint32_t)(wrapi(ax + d, W) * Cin * 2 + 16 * g); };
-    rowo[h] = Off3{row(-1), row(0), row(1)};
-    colo[h] = Off3{col(-1), col(0), col(1)};
-    const int32_t co = co0 + r0 + 64 * h;
-    wo[h] = co < Cout ? (uint32_t)((int64_t)co * 9 * Cin * 2 + 16 * g) : kBad;
-  }
-  const int32_t kz = (int32_t)gridDim.z, z = (int32_t)blockIdx.z;
-  const int32_t s0 = (int32_t)((int64_t)z * ksteps / kz), s1 = (int32_t)((int64_t)(z + 1) * ksteps / kz);
-  // the next step to load, kept as tap (row ty, column tx) and chunk c so
-  // that no step divides; abase: the A byte offsets of that tap, recomputed
-  // only when the tap changes, so a step adds the chunk and selects kBad for
-  // channels past Cin
-  int32_t ltap = s0 / cchunks, lc = s0 - ltap * cchunks;
-  int32_t lty = ltap / 3, ltx = ltap - 3 * lty;
-  uint32_t abase[2];
-  auto settap = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) abase[h] = rowo[h].at(lty) + colo[h].at(ltx);
-  };
-  settap();
-  const int32_t cin_g = Cin - 8 * g;  // a lane's channels at k are valid while k < cin_g
-  bf16x8 ra[2], rb[2];
-  auto load = [&]() __attribute__((always_inline)) {
-    const int32_t k = lc * KC;
-    const bool cok = k < cin_g;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t o = abase[h] + (uint32_t)(k * 2);
-      ra[h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(cok ? o : kBad), 0, 0));
-    }
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int32_t row = r0 + 64 * h;
-      if (row < NT && (h == 0 || NT > 64)) {
-        const uint32_t o = wo[h] + (uint32_t)((ltap * Cin + k) * 2);
-        rb[h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(cok ? o : kBad), 0, 0));
-      }
-    }
-    if (++lc == cchunks) {
-      lc = 0;
-      ++ltap;
-      if (++ltx == 3) {
-        ltx = 0;
-        ++lty;
-      }
-      settap();
-    }
-  };
-  auto store = [&](int32_t buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) *(bf16x8*)&sA[buf][(r0 + 64 * h) * LD + 8 * g] = ra[h];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const int32_t row = r0 + 64 * h;
-      if (row < NT && (h == 0 || NT > 64)) *(bf16x8*)&sB[buf][row * LD + 8 * g] = rb[h];
-    }
-  };
-
-  f32x4 acc[BM][BN];
-#pragma unroll
-  for (int i = 0; i < BM; i++)
-#pragma unroll
-    for (int j = 0; j < BN; j++) acc[i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-
-  load();
-  store(0);
-  __syncthreads();
-  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
-  for (int32_t s = s0; s < s1; s++) {
-    const int32_t buf = (s - s0) & 1;
-    if (s + 1 < s1) load();
-    bf16x8 a[BM], b[BN];
-#pragma unroll
-    for (int i = 0; i < BM; i++) a[i] = *(const bf16x8*)&sA[buf][(wm * TM + 16 * i + rl) * LD + kq];
-#pragma unroll
-    for (int j = 0; j < BN; j++) b[j] = *(const bf16x8*)&sB[buf][(wn * TN + 16 * j + rl) * LD + kq];
-#pragma unroll
-    for (int i = 0; i < BM; i++)
-#pragma unroll
-      for (int j = 0; j < BN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    if (s + 1 < s1) store(buf ^ 1);
-    __syncthreads();
-  }
-  if (part) {
-    float* pz = part + (int64_t)z * P * Cout;
-#pragma unroll
-    for (int j = 0; j < BN; j++) {
-      const int32_t co = co0 + wn * TN + 16 * j + rl;
-      if (co >= Cout) continue;
-#pragma unroll
-      for (int i = 0; i < BM; i++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int64_t p = p0 + wm * TM + 16 * i + 4 * (lane >> 4) + e;
-          if (p < P) pz[p * Cout + co] = acc[i][j][e];
-        }
-    }
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < BN; j++) {
-    const int32_t co = co0 + wn * TN + 16 * j + rl;
-    if (co >= Cout) continue;
-    const float bv = bias ? bias[co] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < BM; i++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int64_t p = p0 + wm * TM + 16 * i + 4 * (lane >> 4) + e;
-        if (p >= P) continue;
-        float v = acc[i][j][e] + bv;
-        if (ACT == 1) v = v > 0.0f ? v : 0.0f;
-        if (ACT == 2) v = bf2f(mask[p * Cout + co]) > 0.0f ? v : 0.0f;
-        if (y16) y16[p * Cout + co] = f2bf(v);
-        if (y32) y32[p * Cout + co] = v;
-      }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 3x3 convolution over row strips (W % 32 == 0, Cin <= CI, CI = 32 or 64):
-// a workgroup owns 32 output channels and walks R rows of one 32-pixel
-// column strip of one image.  Its weights [32][9][CI] stay in LDS for the
-// whole strip; input rows y - 1, y, y + 1 (34 pixels with the periodic
-// halo, all input channels) sit in a four-row LDS ring, the next row loaded
-// while the current one is computed, so every input value is read from
-// memory once per strip and serves all nine taps.  NHWC rows are the MFMA's
-// A layout (lane: one pixel, 8 consecutive channels) and the weights' its B
-// layout, so both are copied as 16-byte runs; the tap's shift is the ring
-// row and the pixel row within it.  Waves tile the 32 x 32 output block of a
-// row 2 x 2 (16 pixels x 16 channels each) and write it before the next row.
-// Epilogue as k_conv3x3 (bias; ACT 0 none, 1 ReLU, 2 mask).
-// ---------------------------------------------------------------------------
-template <int CI, int ACT>
-__global__ __launch_bounds__(256) void k_conv_rows(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                   const float* __restrict__ bias, const bf16* __restrict__ mask,
-                                                   bf16* __restrict__ y16, float* __restrict__ y32, int32_t N,
-                                                   int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t R) {
-  constexpr int LDX = CI + 8;          // ring row stride (elements): 16-byte aligned, shifted banks
-  constexpr int LDW = 9 * CI + 8;      // weight row stride
-  constexpr int XG = CI / 8;           // 16-byte groups of a pixel
-  constexpr int XITEMS = 34 * XG;      // loads of one input row
-  constexpr int XPER = (XITEMS + 255) / 256;
-  __shared__ __attribute__((aligned(16))) bf16 s_w[32 * LDW];
-  __shared__ __attribute__((aligned(16))) bf16 s_x[4][34 * LDX];
-  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int32_t segs = W / 32, cps = (H + R - 1) / R;
-  const int32_t chunk = blockIdx.x;
-  const int32_t rc = chunk % cps, sg = (chunk / cps) % segs, n = chunk / (cps * segs);
-  const int32_t co0 = blockIdx.y * 32;
-  const int32_t y0 = rc * R, rows = R < H - y0 ? R : H - y0, x0 = sg * 32;
-  const int64_t img = (int64_t)n * H;
-  const bf16x8 zero = {};
-
-  // weights of the 32 output channels: [co][tap][ci], channels >= Cin zero
-  for (int32_t u = tid; u < 32 * 9 * XG; u += 256) {
-    const int32_t g = u % XG, t = (u / XG) % 9, col = u / (9 * XG);
-    const int32_t co = co0 + col, ci = 8 * g;
-    bf16x8 v = zero;
-    if (co < Cout && ci < Cin) v = *(const bf16x8*)(w + ((int64_t)co * 9 + t) * Cin + ci);
-    *(bf16x8*)&s_w[col * LDW + t * CI + ci] = v;
-  }
-  // input row loads: items (pixel column c = 0 .. 33, group g)
-  int32_t xc[XPER], xg[XPER];
-  bool xitem[XPER], xok[XPER];
-  int64_t xcol[XPER];
-#pragma unroll
-  for (int h = 0; h < XPER; h++) {
-    const int32_t u = tid + 256 * h;
-    xitem[h] = u < XITEMS;
-    xc[h] = u / XG;
-    xg[h] = u % XG;
-    xok[h] = xitem[h] && 8 * xg[h] < Cin;
-    xcol[h] = (int64_t)wrapi(x0 + xc[h] - 1, W) * Cin + 8 * xg[h];
-  }
-  struct Row {
-    bf16x8 v[XPER];
-  };
-  auto load = [&](int32_t k) __attribute__((always_inline)) {  // image row y0 - 1 + k
-    Row r;
-    const int64_t xrow = (img + wrapi(y0 - 1 + k, H)) * W * Cin;
-#pragma unroll
-    for (int h = 0; h < XPER; h++) r.v[h] = xok[h] ? *(const bf16x8*)(x + xrow + xcol[h]) : zero;
-    return r;
-  };
-  auto store = [&](const Row& r, int32_t slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int h = 0; h < XPER; h++)
-      if (xitem[h]) *(bf16x8*)&s_x[slot][xc[h] * LDX + 8 * xg[h]] = r.v[h];
-  };
-  // ring rows k = 0, 1, 2 in LDS; row k = 3 in registers (two rows ahead
-  // of the first step's need)
-  Row ra, rb;
+  uint32_t io[AP];
   {
-    const Row r0 = load(0), r1 = load(1), r2 = load(2);
-    if (rows > 1) ra = load(3);
-    store(r0, 0);
-    store(r1, 1);
-    store(r2, 2);
-  }
-  __syncthreads();
-
-  const int32_t pt = wave & 1, ct = wave >> 1;  // 16 pixels x 16 channels of the 32 x 32 block
-  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
-  const int32_t co_b = 16 * ct + rl;            // B row (output channel within the block)
-  const int32_t co = co0 + co_b;
-  const float bv = (bias && co < Cout) ? bias[co] : 0.0f;
-  // A wave's B fragments (its 16 output channels, every tap and 32-channel
-  // slice: 9 or 18) stay in registers for the whole strip, so a row step
-  // reads only A from LDS (measured faster than reading B per row also at
-  // 64 input channels, where they take 72 registers)
-  constexpr int BREG = 9 * (CI / 32);
-  bf16x8 breg[BREG];
+    const int32_t by = (cy * TH + H - 1) % H, bx = (cx * TW + W - 1) % W;
 #pragma unroll
-  for (int u = 0; u < BREG; u++)
-    breg[u] = *(const bf16x8*)(s_w + co_b * LDW + (u / (CI / 32)) * CI + 32 * (u % (CI / 32)) + kq);
-  // step s: LDS holds rows s .. s + 2, `held` row s + 3 (needed from step
-  // s + 1 on); row s + 4 is loaded into `next`, and `held` is stored into
-  // the slot of row s - 1, free since the barrier that ended step s - 1
-  auto step = [&](int32_t s, Row& held, Row& next) __attribute__((always_inline)) {
-    if (s + 2 < rows) next = load(s + 4);
-    // D rows (pixels) 4 (lane / 16) + e of the wave's 16, column = channel co
-    const int64_t prow = (img + y0 + s) * W + x0 + 16 * pt + 4 * (lane >> 4);
-    float mk[4] = {1.0f, 1.0f, 1.0f, 1.0f};  // the mask is requested before the MFMAs
-    if (ACT == 2 && co < Cout) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) mk[e] = bf2f(mask[(prow + e) * Cout + co]);
+    for (int h = 0; h < AP; h++) {
+      const int32_t p = quad + 64 * h, r = p / PW, c = p - r * PW;
+      int32_t yy = by + r, xx = bx + c;
+      if (yy >= H) yy = yy < 2 * H ? yy - H : yy % H;
+      if (xx >= W) xx = xx < 2 * W ? xx - W : xx % W;
+      io[h] = p < NP ? (uint32_t)((((n * H + yy) * W + xx) * Cin + 8 * gg) * 2) : kBad;
     }
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // weights: quad -> (row of the tap's block, chunk within a group of QB)
+  const int32_t brow = quad % RB, bq = quad / RB;
+  uint32_t wo;
+  {
+    const int32_t j = brow >> 4, r = brow & 15;
+    const int32_t co = co0 + 32 * (j >> 1) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3);
+    wo = co < Cout ? (uint32_t)((co * 9 * Cin + 8 * gg) * 2) : kBad;
+  }
+  // the weights of tap t of channel block k0 (zero past Cin and Cout)
+  struct Tap {
+    bf16x8 v[BP];
+  };
+  auto load_b = [&](Tap& r, int32_t t, int32_t k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int dyi = 0; dyi < 3; dyi++) {
-      const bf16* xr = s_x[(s + dyi) & 3];
+    for (int i = 0; i < BP; i++) {
+      if (QB * i >= nc) continue;
+      const int32_t k = k0 + 32 * (QB * i + bq);
+      const bool ok = wo != kBad && k + 8 * gg < Cin;
+      r.v[i] = __builtin_bit_cast(
+          bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(ok ? wo + (uint32_t)((t * Cin + k) * 2) : kBad), 0, 0));
+    }
+  };
+  auto store_b = [&](const Tap& r, int32_t buf) __attribute__((always_inline)) {
 #pragma unroll
-      for (int dxi = 0; dxi < 3; dxi++) {
-        const int32_t t = 3 * dyi + dxi;
-        // A: pixel 16 pt + rl of the row, shifted by dx (column + dxi)
-        const bf16* ap = xr + (16 * pt + rl + dxi) * LDX + kq;
+    for (int i = 0; i < BP; i++) {
+      if (QB * i >= nc) continue;
+      const int32_t c = QB * i + bq;
+      if (c < nc) *(bf16x8*)&s_b[(buf * RB + brow) * LD + 32 * c + 8 * gg] = r.v[i];
+    }
+  };
+  if (tid < RB) s_bias[tid] = bias && co0 + tid < Cout ? bias[co0 + tid] : 0.0f;
+
+  const bf16* ap[PF];
 #pragma unroll
-        for (int kc = 0; kc < CI / 32; kc++) {
-          const bf16x8 a = *(const bf16x8*)(ap + 32 * kc);
-          const bf16x8 b = breg[t * (CI / 32) + kc];
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+  for (int f = 0; f < PF; f++) {
+    const int32_t idx = wave * PF + f;
+    ap[f] = s_a + ((idx / S) * PW + 16 * (idx % S) + rl) * LD + 8 * g;
+  }
+  const bf16* bp = s_b + rl * LD + 8 * g;
+  f32x4 acc[PF][CF], tot[SPLIT ? PF : 1][SPLIT ? CF : 1];
+#pragma unroll
+  for (int f = 0; f < PF; f++)
+#pragma unroll
+    for (int j = 0; j < CF; j++) acc[f][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  // split reduction: the slice that ends before step `cut`
+  const int32_t ksteps = 9 * ((Cin + 31) / 32);
+  int32_t z = 0, step = 0, cut = SPLIT && kz > 1 ? ksteps / kz : ksteps;
+  auto slice_end = [&]() __attribute__((always_inline)) {
+    if (SPLIT && step == cut && step < ksteps) {
+#pragma unroll
+      for (int f = 0; f < PF; f++)
+#pragma unroll
+        for (int j = 0; j < CF; j++) {
+          tot[f][j] = z == 0 ? acc[f][j] : tot[f][j] + acc[f][j];
+          acc[f][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      z++;
+      cut = (int32_t)((int64_t)(z + 1) * ksteps / kz);
+    }
+  };
+
+  for (int32_t k0 = 0; k0 < Cin; k0 += KC) {
+    Tap w0, w1;
+    load_b(w0, 0, k0);
+    // the patch, two or four chunks of loads in flight at a time
+    constexpr int AB = PF == 4 ? 2 : 4;
+    if (k0 > 0) __syncthreads();  // the previous block's reads are done
+    for (int32_t c0 = 0; c0 < nc; c0 += AB) {
+      bf16x8 ra[AB][AP];
+#pragma unroll
+      for (int c = 0; c < AB; c++) {
+        const bool ok = c0 + c < nc && k0 + 32 * (c0 + c) + 8 * gg < Cin;
+#pragma unroll
+        for (int h = 0; h < AP; h++)
+          ra[c][h] = __builtin_bit_cast(
+              bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                          xr, (int)(ok && io[h] != kBad ? io[h] + (uint32_t)(2 * k0 + 64 * (c0 + c)) : kBad), 0, 0));
+      }
+#pragma unroll
+      for (int c = 0; c < AB; c++) {
+        if (c0 + c >= nc) continue;
+#pragma unroll
+        for (int h = 0; h < AP; h++) {
+          const int32_t p = quad + 64 * h;
+          if (NP % 64 == 0 || p < NP) *(bf16x8*)&s_a[p * LD + 32 * (c0 + c) + 8 * gg] = ra[c][h];
         }
       }
     }
-    if (co < Cout) {
+    store_b(w0, 0);
+    load_b(w1, 1, k0);
+    __syncthreads();
+    // chunks of this block that hold channels (the steps of the GEMM)
+    const int32_t ncb = (Cin - k0 + 31) / 32 < nc ? (Cin - k0 + 31) / 32 : nc;
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int64_t p = prow + e;
-        float v = acc[e] + bv;
-        if (ACT == 1) v = v > 0.0f ? v : 0.0f;
-        if (ACT == 2) v = mk[e] > 0.0f ? v : 0.0f;
-        if (y16) y16[p * Cout + co] = f2bf(v);
-        if (y32) y32[p * Cout + co] = v;
+    for (int t = 0; t < 9; t++) {
+      // with two weight buffers the next tap's go to the other one here
+      if (two && t + 1 < 9) store_b(t % 2 == 0 ? w1 : w0, (t + 1) & 1);
+      if (t + 2 < 9) load_b(t % 2 == 0 ? w0 : w1, t + 2, k0);
+      const bf16* bt = bp + (two ? (t & 1) * RB * LD : 0);
+      const int32_t at = ((t / 3) * PW + t % 3) * LD;
+      for (int32_t c = 0; c < ncb; c += 2) {
+        bf16x8 fa[2][CF], fb[2][PF];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          if (u == 1 && c + 1 >= ncb) continue;
+#pragma unroll
+          for (int j = 0; j < CF; j++) fa[u][j] = *(const bf16x8*)(bt + j * 16 * LD + 32 * (c + u));
+#pragma unroll
+          for (int f = 0; f < PF; f++) fb[u][f] = *(const bf16x8*)(ap[f] + at + 32 * (c + u));
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          if (u == 1 && c + 1 >= ncb) continue;
+#pragma unroll
+          for (int f = 0; f < PF; f++)
+#pragma unroll
+            for (int j = 0; j < CF; j++)
+              acc[f][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[u][j], fb[u][f], acc[f][j], 0, 0, 0);
+          step++;
+          slice_end();
+        }
+      }
+      if (t + 1 < 9) {
+        __syncthreads();
+        if (!two) {
+          store_b(t % 2 == 0 ? w1 : w0, 0);
+          __syncthreads();
+        }
       }
     }
-    if (s + 1 < rows) store(held, (s + 3) & 3);
-    __syncthreads();
-  };
-  for (int32_t s = 0; s < rows; s += 2) {
-    step(s, ra, rb);
-    if (s + 1 < rows) step(s + 1, rb, ra);
   }
-}
-
-// y = the Z split-K partials added in order + bias, then ACT (as k_conv3x3's
-// epilogue); n = pixels x Cout
-template <int ACT>
-__global__ void k_conv_reduce(const float* __restrict__ part, int32_t kz, int64_t n, int32_t Cout,
-                              const float* __restrict__ bias, const bf16* __restrict__ mask, bf16* __restrict__ y16,
-                              float* __restrict__ y32) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  float a = part[i];
-  for (int32_t z = 1; z < kz; z++) a += part[(int64_t)z * n + i];
-  // 32-bit remainder where n allows (a 64-bit one per element is slower than the loads)
-  const int32_t co = n <= 0x7fffffffLL ? (int32_t)((uint32_t)i % (uint32_t)Cout) : (int32_t)(i % Cout);
-  float v = a + (bias ? bias[co] : 0.0f);
-  if (ACT == 1) v = v > 0.0f ? v : 0.0f;
-  if (ACT == 2) v = bf2f(mask[i]) > 0.0f ? v : 0.0f;
-  if (y16) y16[i] = f2bf(v);
-  if (y32) y32[i] = v;
+  if (SPLIT && z > 0) {
+#pragma unroll
+    for (int f = 0; f < PF; f++)
+#pragma unroll
+      for (int j = 0; j < CF; j++) acc[f][j] = tot[f][j] + acc[f][j];
+  }
+  conv_store<PF, CF, S, ACT>(acc, s_bias, mask, y16, y32, n, cy * TH, cx * TW, H, W, Cout, co0, vec);
 }
 
 // wt[ci][t'][co] = w[co][8 - t][ci]: the data gradient of a periodic 3x3
@@ -1121,32 +1227,17 @@ static inline unsigned G(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 extern "C" {
 
-// Maps whose rows are whole 32-pixel strips take k_conv_rows for layers of
-// at most 32 input channels, and of at most 64 when the output has at most
-// 2^SWENN_CONV_ROWS64_LOG2 values (measured on the surrogate's layers,
-// MI355X: 32-channel layers at 256^2 45 -> 30 us; with 64 input channels
-// the 57 KB of LDS leave two workgroups per CU and every 32-channel output
-// block re-reads the rows, which the register-held weights now outweigh up
-// to the 64 -> 64 layers at 128^2, 2^23 values): 32 output channels a
-// workgroup, each strip cut into chunks of R rows, enough chunks for
-// ~SWENN_CONV_WGS workgroups but at most ceil(H / SWENN_CONV_MINROWS) a
-// strip.  Others take k_conv3x3, whose output channels per workgroup are the
-// layer's (up to 64), 128 where that still leaves two workgroups per CU of
-// the chip's 256.
-#ifndef SWENN_CONV_ROWS
-#define SWENN_CONV_ROWS 1
-#endif
-#ifndef SWENN_CONV_WGS
-#define SWENN_CONV_WGS 2048
-#endif
-#ifndef SWENN_CONV_MINROWS
-#define SWENN_CONV_MINROWS 8
-#endif
-// split-K factor of k_conv3x3 for a grid of mt x ncob workgroups: layers
-// with fewer workgroups than the chip has CUs and a long reduction are split
-// so that ~768 workgroups take >= 8 k-steps each (at most 8 parts)
-static int32_t conv_split(int64_t mt, int64_t ncob, int32_t ksteps) {
-  const int64_t wgs = mt * ncob;
+// Slices of a split reduction: layers whose grid of 128-pixel blocks has fewer
+// workgroups than the chip has CUs, ~768 over the slices, >= 8 steps of 32
+// channels each, at most 8.  The tile kernels sum the slices in one workgroup
+// (they need no workspace), but a layer given the workspace keeps the slices'
+// order of additions.
+static int32_t conv_slices(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
+  const int64_t P = (int64_t)N * H * W;
+  if (W % 32 == 0 && (Cin <= 32 || (Cin <= 64 && (int64_t)Cout * P <= ((int64_t)1 << 23)))) return 1;
+  const int64_t mt = (P + 127) / 128;
+  const int32_t nt = Cout <= 16 ? 16 : (Cout <= 32 ? 32 : (Cout <= 64 || mt * ((Cout + 127) / 128) < 512 ? 64 : 128));
+  const int64_t wgs = mt * ((Cout + nt - 1) / nt), ksteps = 9 * ((Cin + 31) / 32);
   if (wgs >= 256 || ksteps < 24) return 1;
   int64_t z = (768 + wgs - 1) / wgs;
   if (z > ksteps / 8) z = ksteps / 8;
@@ -1154,101 +1245,145 @@ static int32_t conv_split(int64_t mt, int64_t ncob, int32_t ksteps) {
   return z < 2 ? 1 : (int32_t)z;
 }
 
-static bool conv_rows_ok(int32_t W, int32_t Cin, int32_t Cout, int64_t P);
-
-// k_conv3x3's grid: pixel blocks, output-channel blocks of nt, split parts
-static void conv_grid(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int64_t* mt, int32_t* nt,
-                      int32_t* kz) {
-  const int64_t P = (int64_t)N * H * W;
-  *mt = (P + 127) / 128;
-  *nt = Cout <= 16 ? 16 : (Cout <= 32 ? 32 : (Cout <= 64 || *mt * ((Cout + 127) / 128) < 512 ? 64 : 128));
-  *kz = conv_split(*mt, (Cout + *nt - 1) / *nt, 9 * ((Cin + 31) / 32));
+// The shape of a layer's workgroups (k_conv_tile up to 32 input channels,
+// k_conv_wide above)
+struct ConvTile {
+  int32_t pf, cf, s, per;
+  int64_t wgs;
+  int32_t kc, two;
+  size_t lds;
+};
+static bool conv_tile(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t kz, ConvTile* t) {
+  const int32_t segs = (W + 15) / 16;
+  t->s = segs % 2 == 0 ? 2 : 1;
+  auto tiles = [&](int32_t pf) {
+    const int32_t th = 4 * pf / t->s;
+    return (int64_t)N * ((H + th - 1) / th) * (segs / t->s);
+  };
+  auto wgs = [&](int32_t pf, int32_t cf) { return tiles(pf) * ((Cout + 16 * cf - 1) / (16 * cf)); };
+  t->kc = t->two = 0;
+  t->lds = 0;
+  const bool wide = Cin > 32;
+  if (!wide) {
+    // the largest workgroups that still make enough of them for the chip's 256
+    // CUs, which hold two to four each (32 -> 64 at 128^2, batch 8: (4, 4)
+    // 11.4 us, (2, 4) 11.9, (2, 2) 11.7; 32 -> 32 at 256^2, batch 1, (4, 2)
+    // 9.5, (2, 2) 9.7, (1, 2) 10.1)
+    struct Shape {
+      int32_t pf, cf, wgs;
+    };
+    static const Shape k16[] = {{4, 1, 0}};
+    static const Shape k32[] = {{4, 2, 512}, {2, 2, 192}, {1, 2, 0}};
+    static const Shape k64[] = {{4, 4, 512}, {2, 4, 400}, {2, 2, 192}, {1, 2, 0}};
+    const Shape* sh = Cout <= 16 ? k16 : (Cout <= 32 ? k32 : k64);
+    while (wgs(sh->pf, sh->cf) < sh->wgs) sh++;
+    t->pf = sh->pf;
+    t->cf = sh->cf;
+  } else {
+    // The shape of least estimated time: rounds of workgroups (one or two to a
+    // CU, by LDS) times a workgroup's fragment reads, PF + CF a k-step; two on
+    // a CU take 1.3 times as long as one alone.  Measured (us) at batch 8: 192
+    // -> 192 at 32^2, (4, 2) 17.7 (one round), (2, 4) 19.7 (one), (1, 2) 23.1
+    // (two rounds of two), (2, 2) 25.5 (two); 128 -> 192 there, (2, 2) 13.3,
+    // (4, 2) 14.8, (2, 4) 15.9; 128 -> 128 at 64^2, (2, 4) 18.2, (2, 2) 22.5,
+    // (4, 2) 24.7; 256 -> 192 at 16^2, (1, 2) 13.9, (2, 2) 16.0, (2, 4) 23.8.
+    static const int32_t kShape[][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {1, 2}};
+    double best = 0.0;
+    for (const auto& sh : kShape) {
+      const int32_t pf = sh[0], cf = sh[1], kmax = 32 * conv_wide_chunks(pf, cf);
+      if ((cf > 2 && Cout <= 32) || (kz > 1 && pf * cf > 8)) continue;
+      const int32_t kc = Cin > kmax ? kmax : (Cin + 31) / 32 * 32;
+      const size_t rows = (size_t)(4 * pf / t->s + 2) * (16 * t->s + 2), row = (size_t)(kc + 8) * 2;
+      const size_t one = (rows + 16 * cf) * row + 64 * cf, two = one + 16 * cf * row;
+      if (one > 163840) continue;
+      const int64_t w = wgs(pf, cf), per_cu = one <= 81920 ? 2 : 1;
+      const double est = (double)((w + 256 * per_cu - 1) / (256 * per_cu)) * (pf + cf) * (per_cu == 2 && w > 256 ? 1.3 : 1.0);
+      if (best > 0.0 && est >= best) continue;
+      best = est;
+      t->pf = pf;
+      t->cf = cf;
+      t->kc = kc;
+      // a second weight buffer saves a barrier a tap; not at the price of the
+      // second workgroup on a CU
+      t->two = two <= 81920 || (per_cu == 1 && two <= 163840);
+      t->lds = t->two ? two : one;
+    }
+    if (best == 0.0) return false;
+  }
+  const int64_t n = tiles(t->pf), ncob = (Cout + 16 * t->cf - 1) / (16 * t->cf);
+  // one chunk: a workgroup keeps its weights over several tiles, one round of
+  // workgroups in all
+  const int64_t round = 256 * conv_tile_waves(t->pf, t->cf);
+  t->per = !wide ? (int32_t)((n * ncob + round - 1) / round) : 1;
+  t->wgs = (n + t->per - 1) / t->per * ncob;
+  return t->wgs <= 0x7fffffffLL && n <= 0x3fffffffLL;
 }
 
 static int conv_launch(const void* x, int32_t N, int32_t H, int32_t W, int32_t Cin, const void* w, const float* bias,
                        int32_t Cout, int act, const void* mask, void* y16, float* y32, void* stream,
-                       float* work = nullptr, int64_t work_len = 0) {
+                       const float* work = nullptr, int64_t work_len = 0) {
   if (!x || !w || N < 1 || H < 1 || W < 1 || Cin < 8 || Cin % 8 || Cout < 1 || (!y16 && !y32)) return -1;
   const int64_t P = (int64_t)N * H * W;
-  // k_conv3x3's buffer loads take 32-bit byte offsets below 2^31
+  // the kernels' buffer loads take 32-bit byte offsets below 2^31
   if (P * Cin * 2 >= ((int64_t)1 << 31) || (int64_t)Cout * 9 * Cin * 2 >= ((int64_t)1 << 31)) return -1;
   const bf16* xx = (const bf16*)x;
   const bf16* ww = (const bf16*)w;
   const bf16* mm = (const bf16*)mask;
   bf16* yy = (bf16*)y16;
-  if (conv_rows_ok(W, Cin, Cout, P)) {
-    const int64_t strips = (int64_t)N * (W / 32), cob = (Cout + 31) / 32;
-    int64_t cps = (SWENN_CONV_WGS + strips * cob - 1) / (strips * cob);
-    const int64_t cmax = (H + SWENN_CONV_MINROWS - 1) / SWENN_CONV_MINROWS;
-    if (cps > cmax) cps = cmax;
-    if (cps < 1) cps = 1;
-    const int32_t R = (int32_t)((H + cps - 1) / cps);
-    const int64_t chunks = strips * ((H + R - 1) / R);
-    if (chunks > 0x7fffffffLL || cob > 65535) return -1;
-    const dim3 g((unsigned)chunks, (unsigned)cob);
-#define SWENN_CONV_R(CI_, AC)                                                                                   \
-  hipLaunchKernelGGL((k_conv_rows<CI_, AC>), g, dim3(256), 0, S(stream), xx, ww, bias, mm, yy, y32, N, H, W, Cin, \
-                     Cout, R)
-#define SWENN_CONV_R_CI(CI_)                \
-  if (act == 1) SWENN_CONV_R(CI_, 1);      \
-  else if (act == 2) SWENN_CONV_R(CI_, 2); \
-  else SWENN_CONV_R(CI_, 0)
-    if (Cin <= 32) { SWENN_CONV_R_CI(32); }
-    else { SWENN_CONV_R_CI(64); }
-#undef SWENN_CONV_R_CI
-#undef SWENN_CONV_R
-    SWENN_LAUNCH_CHECK();
+  int32_t kz = conv_slices(N, H, W, Cin, Cout);
+  if (!work || work_len < (int64_t)kz * P * Cout) kz = 1;
+  ConvTile ct;
+  if (!conv_tile(N, H, W, Cin, Cout, kz, &ct)) return -1;
+  // 16-byte stores and mask loads where every row of channels is aligned to them
+  const int32_t vec = Cout % 8 == 0 && !(((uintptr_t)y16 | (uintptr_t)y32 | (uintptr_t)mask) & 15);
+  const dim3 g((unsigned)ct.wgs);
+#define SWENN_CT(PF_, CF_, S_, AC)                                                                               \
+  hipLaunchKernelGGL((k_conv_tile<PF_, CF_, S_, AC>), g, dim3(256), 0, S(stream), xx, ww, bias, mm, yy, y32, N, H, \
+                     W, Cin, Cout, ct.per, vec)
+#define SWENN_CW_(PF_, CF_, S_, AC, SP_)                                                                          \
+  hipLaunchKernelGGL((k_conv_wide<PF_, CF_, S_, AC, SP_>), g, dim3(256), ct.lds, S(stream), xx, ww, bias, mm, yy, \
+                     y32, N, H, W, Cin, Cout, ct.kc, kz, ct.two, vec)
+#define SWENN_CW(PF_, CF_, S_, AC) SWENN_CW_(PF_, CF_, S_, AC, false)
+#define SWENN_CWS(PF_, CF_, S_, AC) SWENN_CW_(PF_, CF_, S_, AC, true)
+#define SWENN_CT_ACT(K_, PF_, CF_, S_)    \
+  if (act == 1) K_(PF_, CF_, S_, 1);      \
+  else if (act == 2) K_(PF_, CF_, S_, 2); \
+  else K_(PF_, CF_, S_, 0)
+#define SWENN_CT_S(K_, PF_, CF_)                    \
+  if (ct.s == 2) { SWENN_CT_ACT(K_, PF_, CF_, 2); } \
+  else { SWENN_CT_ACT(K_, PF_, CF_, 1); }
+  if (Cin > 32 && kz > 1) {
+    if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CWS, 2, 4); }
+    else if (ct.pf == 4 && ct.cf == 2) { SWENN_CT_S(SWENN_CWS, 4, 2); }
+    else if (ct.pf == 2 && ct.cf == 2) { SWENN_CT_S(SWENN_CWS, 2, 2); }
+    else { SWENN_CT_S(SWENN_CWS, 1, 2); }
+  } else if (Cin > 32) {
+    if (ct.pf == 4 && ct.cf == 4) { SWENN_CT_S(SWENN_CW, 4, 4); }
+    else if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CW, 2, 4); }
+    else if (ct.pf == 4 && ct.cf == 2) { SWENN_CT_S(SWENN_CW, 4, 2); }
+    else if (ct.pf == 2 && ct.cf == 2) { SWENN_CT_S(SWENN_CW, 2, 2); }
+    else { SWENN_CT_S(SWENN_CW, 1, 2); }
+  } else {
+    if (ct.pf == 4 && ct.cf == 4) { SWENN_CT_S(SWENN_CT, 4, 4); }
+    else if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CT, 2, 4); }
+    else if (ct.pf == 4 && ct.cf == 2) { SWENN_CT_S(SWENN_CT, 4, 2); }
+    else if (ct.pf == 2 && ct.cf == 2) { SWENN_CT_S(SWENN_CT, 2, 2); }
+    else if (ct.pf == 1 && ct.cf == 2) { SWENN_CT_S(SWENN_CT, 1, 2); }
+    else { SWENN_CT_S(SWENN_CT, 4, 1); }
   }
-  int64_t mt;
-  int32_t nt, kz;
-  conv_grid(N, H, W, Cin, Cout, &mt, &nt, &kz);
-  if (mt > 0x7fffffffLL) return -1;
-  if (kz > 1 && (!work || work_len < (int64_t)kz * P * Cout)) kz = 1;  // no room for the partials: unsplit
-  float* part = kz > 1 ? work : nullptr;
-  const dim3 grid((unsigned)mt, (unsigned)((Cout + nt - 1) / nt), (unsigned)kz);
-  // split: the parts hold raw sums (the kernel's epilogue is not run)
-  const int ka = kz > 1 ? 0 : act;
-#define SWENN_CONV(NT_, AC)                                                                                       \
-  hipLaunchKernelGGL((k_conv3x3<NT_, AC>), grid, dim3(256), 0, S(stream), xx, ww, bias, mm, yy, y32, N, H, W, Cin, \
-                     Cout, part)
-#define SWENN_CONV_NT(NT_)            \
-  if (ka == 1) SWENN_CONV(NT_, 1);  \
-  else if (ka == 2) SWENN_CONV(NT_, 2); \
-  else SWENN_CONV(NT_, 0)
-  if (nt == 16) { SWENN_CONV_NT(16); }
-  else if (nt == 32) { SWENN_CONV_NT(32); }
-  else if (nt == 64) { SWENN_CONV_NT(64); }
-  else { SWENN_CONV_NT(128); }
-#undef SWENN_CONV_NT
-#undef SWENN_CONV
-  if (kz > 1) {
-    const int64_t n = P * Cout;
-    if (act == 1)
-      hipLaunchKernelGGL(k_conv_reduce<1>, dim3(G(n)), dim3(256), 0, S(stream), part, kz, n, Cout, bias, mm, yy, y32);
-    else if (act == 2)
-      hipLaunchKernelGGL(k_conv_reduce<2>, dim3(G(n)), dim3(256), 0, S(stream), part, kz, n, Cout, bias, mm, yy, y32);
-    else
-      hipLaunchKernelGGL(k_conv_reduce<0>, dim3(G(n)), dim3(256), 0, S(stream), part, kz, n, Cout, bias, mm, yy, y32);
-  }
+#undef SWENN_CT_S
+#undef SWENN_CT_ACT
+#undef SWENN_CWS
+#undef SWENN_CW
+#undef SWENN_CW_
+#undef SWENN_CT
   SWENN_LAUNCH_CHECK();
-}
-
-#ifndef SWENN_CONV_ROWS64_LOG2
-#define SWENN_CONV_ROWS64_LOG2 23
-#endif
-static bool conv_rows_ok(int32_t W, int32_t Cin, int32_t Cout, int64_t P) {
-  return SWENN_CONV_ROWS && W % 32 == 0 &&
-         (Cin <= 32 || (Cin <= 64 && (int64_t)Cout * P <= ((int64_t)1 << SWENN_CONV_ROWS64_LOG2)));
 }
 
 int64_t swe_nn_conv3x3_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   if (N < 1 || H < 1 || W < 1 || Cin < 1 || Cout < 1) return 0;
-  const int64_t P = (int64_t)N * H * W;
-  if (conv_rows_ok(W, Cin, Cout, P)) return 0;
-  int64_t mt;
-  int32_t nt, kz;
-  conv_grid(N, H, W, Cin, Cout, &mt, &nt, &kz);
-  return kz > 1 ? (int64_t)kz * P * Cout : 0;
+  const int32_t z = conv_slices(N, H, W, Cin, Cout);
+  return z > 1 ? (int64_t)z * N * H * W * Cout : 0;
 }
 
 int swe_nn_conv3x3_ws(const void* x, int32_t N, int32_t H, int32_t W, int32_t Cin, const void* w, const float* bias,

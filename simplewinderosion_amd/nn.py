@@ -99,7 +99,7 @@ def conv3x3(x, w, bias=None, relu=False, out16=None, out32=None, work=None):
     """x [N,H,W,Cin] bf16, w [Cout,9,Cin] bf16, bias [Cout] float -> out16
     [N,H,W,Cout] bf16 and/or out32 float (allocated when neither is given).
     With `work` (float device tensor of conv_work(...) floats), layers with
-    few pixel blocks split their reduction over several workgroups."""
+    few pixel blocks sum their reduction in slices added in a fixed order."""
     import torch
 
     _dense(x, torch.bfloat16, "x")

@@ -94,7 +94,7 @@ class Surrogate:
         self.step = 0
         self._work = None
         self._adam = None  # swe_nn_adam_multi table over every parameter tensor
-        self._cw = None    # split-K partials of the low-resolution convolutions
+        self._cw = None    # sums the low-resolution convolutions in slices
 
     # -- bookkeeping ----------------------------------------------------------
     def n_params(self):
