@@ -501,356 +501,342 @@ __global__ void k_flip(const bf16* __restrict__ w, bf16* __restrict__ wt, int32_
 // ---------------------------------------------------------------------------
 // Weight and bias gradients: dW[co][t][ci] = sum_p dY[p][co] X[p + s_t][ci],
 // db[co] = sum_p dY[p][co].  Rows = output channels, columns = input
-// channels of one tap, reduction over pixels.  A workgroup (4 waves) owns a
-// 64 (co) x 64 (ci) block of one tap and a chunk of the flattened batch's
-// pixels; per step of 32 pixels every thread loads one 16-byte run of dY
-// (8 channels of a pixel) and one of the tap-shifted X, and stores them
-// channel-major into LDS (double buffered: the next step's runs are loaded
-// while the waves run the current MFMAs); each wave accumulates a 32 x 32
-// sub-block.  The workgroups of tap 4 (no shift) and the first ci block
-// also sum their dY runs for the bias.  Each chunk writes its partial
-// block to `part` ([chunk][Cout * 9 * Cin + Cout]); k_reduce_parts adds the
-// chunks in a fixed order, so the result is deterministic.  Cin % 8 == Cout % 8 == 0.
+// channels of one tap, reduction over pixels, 32 of a row at a time
+// (v_mfma_f32_32x32x16_bf16: a wave alone on its SIMD issues them at the full
+// rate, 32 clocks each; of the 16x16x32 form one every 27 clocks, not 16).
+//
+// A wave owns a 32 (co) x 32 (ci) block of all nine taps and walks units: R
+// rows of one 32-pixel column strip of one image (the last strip of a row may
+// be narrower).  Per dY row y it needs the X rows y - 1, y, y + 1, whose
+// fragments at the three column shifts stay in registers, so every X and dY
+// value is loaded once per strip and passes through LDS once.  Both lie there
+// as loaded (a pixel's 32 channels, 64 bytes) and ds_read_b64_tr_b16 hands
+// each lane four pixels of one channel: a shift is a row offset, and the 32
+// lanes that are served together read 256 consecutive bytes.
+//
+// The four waves of a workgroup take different units of one block and share
+// nothing until the end, where their sums are added through LDS: no barrier in
+// the loop, and a quarter of the partials.  A wave has its SIMD to itself: the
+// accumulators, four rows of loads in flight and the next row's fragments,
+// read while this one's MFMAs run, take ~370 registers.  Partials go to
+// `part`, [chunk][block][tap, quarter][lane][4] and the block's 32 bias sums;
+// k_wgrad_sum adds the chunks in a fixed order.  With one chunk (`dw` given)
+// the sums are the result.  Cin % 8 == Cout % 8 == 0.
+//
+// Bound: MFMA and LDS, 0.5 us a row of 32 pixels in short launches (the MFMAs
+// alone 0.34), memory for 32 channels at 256^2 (67 MB at 8 TB/s from the
+// last-level cache).  With k_wgrad_sum, against a kernel whose workgroups
+// shared 32 x 32 blocks over a barrier a row and transposed in two-byte stores
+// (1024 of them, 38 MB of partials), and one tap a workgroup for rows that are
+// not whole strips (us, batch 8): 64 -> 64 at 128^2 28.1 -> 19.6; 32 -> 32 at
+// 256^2 31.6 -> 21.0; 128 -> 128 at 64^2 30.5 -> 21.6; 256 -> 192 at 16^2 30.6
+// -> 16.0; 128 -> 128 at 50 x 60 68.0 -> 20.7; 32 -> 32 at 200 x 230, batch 3,
+// 110.6 -> 17.0.  Eight rows of loads in flight took 1 to 3 us longer.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ x, const bf16* __restrict__ dy,
-                                               float* __restrict__ part, int32_t N, int32_t H, int32_t W,
-                                               int32_t Cin, int32_t Cout, int32_t chunk) {
-  constexpr int LD = 40;
-  __shared__ __attribute__((aligned(16))) bf16 s_dy[2][64 * LD];  // [co][pixel]
-  __shared__ __attribute__((aligned(16))) bf16 s_x[2][64 * LD];   // [ci][pixel]
-  __shared__ float s_b[32][65];                                    // bias partials [pixel lane][co]
-  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int32_t cit = (Cin + 63) / 64;
-  int32_t bq = blockIdx.y;
-  const int32_t t = bq % 9;
-  bq /= 9;
-  const int32_t ciB = (bq % cit) * 64, coB = (bq / cit) * 64;
-  const bool do_bias = t == 4 && ciB == 0;
-  const int64_t npix = (int64_t)N * H * W;
-  const int64_t p0 = (int64_t)blockIdx.x * chunk;
-  const int64_t pend = p0 + chunk < npix ? p0 + chunk : npix;
-  const int32_t dyo = t / 3 - 1, dxo = t % 3 - 1;
-  // loader: pixel q of the step, channel group gg (8 channels)
-  const int32_t q = tid >> 3, gg = tid & 7;
-  const int32_t co_ld = coB + 8 * gg, ci_ld = ciB + 8 * gg;
-  const bool co_ok = co_ld < Cout, ci_ok = ci_ld < Cin;
-  const bf16x8 zero = {};
-  bf16x8 rdy, rx;
-  float bsum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto load = [&](int64_t q0) __attribute__((always_inline)) {
-    const int64_t p = q0 + q;
-    rdy = zero;
-    rx = zero;
-    if (p < pend) {
-      if (co_ok) rdy = *(const bf16x8*)(dy + p * Cout + co_ld);
-      if (ci_ok) {
-        const int32_t xx = (int32_t)(p % W);
-        const int64_t r = p / W;
-        const int32_t yy = (int32_t)(r % H);
-        const int64_t im = r / H;
-        const int32_t sy = wrapi(yy + dyo, H), sx = wrapi(xx + dxo, W);
-        rx = *(const bf16x8*)(x + ((im * H + sy) * W + sx) * Cin + ci_ld);
-      }
-    }
-  };
-  auto store = [&](int32_t buf) __attribute__((always_inline)) {
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kWgradPart = 9 * 32 * 32 + 32;      // floats of a block's partials
+constexpr int kWgradWave = (48 + 32) * 32;        // LDS elements of a wave: X row (34 pixels of 48), dY row
+constexpr int kWgradRed = 4 * 9 * 4 * 64 * 16;    // LDS bytes: the waves' sums, which overlay the rows
+constexpr int kWgradLds = kWgradRed + 4 * 32 * 4; // and their bias sums
+
+// four results of a lane to dw: D rows (co) = 8 quarter + 4 (lane / 32) + e,
+// column (ci) = lane % 32
+__device__ __forceinline__ void wgrad_put(float* __restrict__ dw, f32x4 v, int32_t t, int32_t quarter, int32_t lane,
+                                          int32_t coB, int32_t ciB, int32_t Cin, int32_t Cout) {
+  const int32_t co = coB + 8 * quarter + 4 * (lane >> 5), ci = ciB + (lane & 31);
+  if (ci >= Cin) return;
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      s_dy[buf][(8 * gg + e) * LD + q] = rdy[e];
-      s_x[buf][(8 * gg + e) * LD + q] = rx[e];
-    }
-    if (do_bias) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) bsum[e] += bf2f(rdy[e]);
-    }
-  };
-  // consumer: wave (wave / 2, wave % 2) owns co rows 32 * (wave / 2) .., ci 32 * (wave % 2) ..
-  const int32_t wr = 32 * (wave >> 1), wc = 32 * (wave & 1);
-  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++) acc[i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-  load(p0);
-  store(0);
-  __syncthreads();
-  int32_t buf = 0;
-  for (int64_t q0 = p0; q0 < pend; q0 += 32) {
-    const bool more = q0 + 32 < pend;
-    if (more) load(q0 + 32);
-    bf16x8 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) a[i] = *(const bf16x8*)&s_dy[buf][(wr + 16 * i + rl) * LD + kq];
-#pragma unroll
-    for (int j = 0; j < 2; j++) b[j] = *(const bf16x8*)&s_x[buf][(wc + 16 * j + rl) * LD + kq];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    if (more) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  const int64_t nw = (int64_t)Cout * 9 * Cin;
-  float* out = part + (int64_t)blockIdx.x * (nw + Cout);
-  // D rows (co) = wr + 16 i + 4 (lane / 16) + e, column (ci) = wc + 16 j + lane % 16
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int32_t ci = ciB + wc + 16 * j + rl;
-    if (ci >= Cin) continue;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int32_t co = coB + wr + 16 * i + 4 * (lane >> 4) + e;
-        if (co < Cout) out[((int64_t)co * 9 + t) * Cin + ci] = acc[i][j][e];
-      }
-  }
-  if (do_bias) {  // the 32 pixel lanes' sums per channel, added in a fixed order
-#pragma unroll
-    for (int e = 0; e < 8; e++) s_b[q][8 * gg + e] = bsum[e];
-    __syncthreads();
-    if (tid < 64) {
-      float sb = 0.0f;
-      for (int k = 0; k < 32; k++) sb += s_b[k][tid];
-      if (coB + tid < Cout) out[nw + coB + tid] = sb;
-    }
-  }
+  for (int e = 0; e < 4; e++)
+    if (co + e < Cout) dw[((int64_t)(co + e) * 9 + t) * Cin + ci] = v[e];
 }
 
-// ---------------------------------------------------------------------------
-// Weight and bias gradients over row strips (W % 32 == 0): a workgroup owns a
-// CB (co) x IB (ci) block of all nine taps and walks R rows of one 32-pixel
-// column strip of one image.  Per row y it loads the dY row (32 pixels x CB)
-// and the X row y + 1 (34 pixels, x0 - 1 .. x0 + 32, periodic); X rows y - 1,
-// y, y + 1 stay in a four-row LDS ring, so every X and dY value is loaded
-// once per strip and serves all nine taps.  LDS rows are channel-major
-// (pixels contiguous, the MFMA's k), 40 elements a row, with the 8-pixel
-// blocks of columns 0..31 permuted per row (block ^ (row / 8) % 4) so that
-// the transposing two-byte stores of eight channel rows fall in different
-// banks.  The tap shift dx = -1, 0, +1 is a B operand read at column
-// offset 0, 1, 2: one aligned 16-byte read plus the next dword, shifted by
-// one element with v_alignbit for the odd offset.  Waves tile the block
-// 2 x 2; each holds 9 x (CB/32) x (IB/32) accumulators.  The workgroups of
-// the first ci block also sum the dY rows for the bias.  Partials go to
-// `part` ([chunk][Cout * 9 * Cin + Cout]) like k_wgrad's.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int32_t wg_col(int32_t row, int32_t c) { return c < 32 ? c ^ (8 * ((row >> 3) & 3)) : c; }
+template <bool RAG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_wgrad(
+    const bf16* __restrict__ x, const bf16* __restrict__ dy, float* __restrict__ part, float* __restrict__ dw,
+    float* __restrict__ db, int32_t H, int32_t W, int32_t Cin, int32_t Cout, int32_t R, uint32_t units, uint32_t per,
+    int32_t nblk) {
+  constexpr int D = 4;  // rows of loads in flight
+  extern __shared__ __attribute__((aligned(16))) char s_wg[];
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // this workgroup's (chunk, block): each XCD (workgroup b runs on XCD b % 8)
+  // takes a contiguous range, so that the blocks of one chunk share its L2
+  const uint32_t nb = gridDim.x, b = blockIdx.x, q8 = nb / 8, r8 = nb % 8, xcd = b % 8;
+  const uint32_t lin = xcd * q8 + (xcd < r8 ? xcd : r8) + b / 8;
+  const int32_t chunk = (int32_t)(lin / (uint32_t)nblk), blk = (int32_t)lin - chunk * nblk;
+  const int32_t nci = (Cin + 31) / 32;
+  const int32_t ciB = (blk % nci) * 32, coB = (blk / nci) * 32;
+  const uint32_t segs = (uint32_t)(W + 31) / 32, cps = (uint32_t)(H + R - 1) / (uint32_t)R;
 
-template <int CB, int IB>
-__global__ __launch_bounds__(256) void k_wgrad_rows(const bf16* __restrict__ x, const bf16* __restrict__ dy,
-                                                    float* __restrict__ part, int32_t N, int32_t H, int32_t W,
-                                                    int32_t Cin, int32_t Cout, int32_t R) {
-  constexpr int LD = 40;
-  constexpr int TI = CB / 32, TJ = IB / 32;  // 16 x 16 tiles per wave along co and ci
-  constexpr int DG = CB / 8, XG = IB / 8;    // 16-byte channel groups of a pixel
-  constexpr int XITEMS = 34 * XG;            // X row loads (pixel, group)
-  __shared__ __attribute__((aligned(16))) bf16 s_x[4][IB * LD];
-  __shared__ __attribute__((aligned(16))) bf16 s_dy[2][CB * LD];
-  __shared__ float s_b[32][CB + 1];
-  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int32_t segs = W / 32, cps = (H + R - 1) / R;
-  const int32_t chunk = blockIdx.x;
-  const int32_t rc = chunk % cps, sg = (chunk / cps) % segs, n = chunk / (cps * segs);
-  const int32_t nci = (Cin + IB - 1) / IB;
-  const int32_t ciB = (int32_t)(blockIdx.y % nci) * IB, coB = (int32_t)(blockIdx.y / nci) * CB;
-  const int32_t y0 = rc * R, rows = R < H - y0 ? R : H - y0, x0 = sg * 32;
-  const bool do_bias = ciB == 0;
-  const bf16x8 zero = {};
+  bf16* s_x = (bf16*)s_wg + wave * kWgradWave;
+  bf16* s_d = s_x + 48 * 32;
+  const int32_t at = 8 * lane;  // item lane + 64 h of a row: pixel, channel group
+  // a lane's part of a transposing read: pixel 8 (lane / 32) + lane % 16 / 4
+  // (+ 4, + 16), channels 16 (lane / 16 % 2) + 4 (lane % 4) ..
+  const int32_t tr = (8 * (lane >> 5) + ((lane & 15) >> 2)) * 32 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  auto frag = [&](const bf16* p) __attribute__((always_inline)) {
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(p + 4 * 32));
+    return __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // orders a wave's own LDS accesses (other lanes') for the compiler; the
+  // hardware keeps a wave's LDS accesses in order
+  auto fence = [&]() __attribute__((always_inline)) { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  const int64_t xrow = (int64_t)W * Cin, drow = (int64_t)W * Cout;
+  constexpr uint32_t kBad = 0xffffffffu;  // past any row: reads zero
+  auto fetch = [&](const bf16* row, uint32_t off) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)row, (short)0, (int)0xffffffff, 0x00020000);
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+  };
 
-  // dY loads: thread -> (pixel dpx, group dg), groups fastest (coalesced)
-  const bool dy_item = tid < 32 * DG;
-  const int32_t dpx = tid / DG, dg = tid % DG;
-  const bool dy_ok = dy_item && coB + 8 * dg < Cout;
-  const int64_t dy_col = (int64_t)(x0 + dpx) * Cout + coB + 8 * dg;
-  // X loads: items tid and tid + 256 -> (column c, group g)
-  int32_t xc[2], xg[2];
-  bool xok[2], xitem[2];
-  int64_t xcol[2];
+  // a unit: its loads' offsets in a row (what lies outside the strip or the
+  // channels reads as zero), its rows, and the first rows' loads
+  uint32_t xo[3], dof[2], keep[2][4];
+  int32_t rows = 0, yx = 0, yd = 0;
+  const bf16 *xim = x, *dim = dy, *xp = x, *dp = dy;
+  struct Row {
+    u32x4 x[3], d[2];
+  } ring[D], first, second;
+  // the next X and dY rows; both run on past the unit's last row (around the
+  // image: in bounds, and not used)
+  auto load_x = [&](Row& r) __attribute__((always_inline)) {
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const int32_t u = tid + 256 * h;
-    xitem[h] = u < XITEMS;
-    xc[h] = u / XG;
-    xg[h] = u % XG;
-    xok[h] = xitem[h] && ciB + 8 * xg[h] < Cin;
-    xcol[h] = (int64_t)wrapi(x0 + xc[h] - 1, W) * Cin + ciB + 8 * xg[h];
-  }
-  const int64_t img = (int64_t)n * H;
-
-  struct Regs {
-    bf16x8 d, xa, xb;
+    for (int h = 0; h < 3; h++) r.x[h] = fetch(xp, xo[h]);
+    yx = yx + 1 == H ? 0 : yx + 1;
+    xp = yx ? xp + xrow : xim;
   };
-  // the loads of X row k (image row y0 - 1 + k) and dY row y
-  auto load = [&](int32_t k, int32_t y, bool with_dy) __attribute__((always_inline)) {
-    Regs r;
-    const int64_t xrow = (img + wrapi(y0 - 1 + k, H)) * W * Cin;
-    r.xa = xok[0] ? *(const bf16x8*)(x + xrow + xcol[0]) : zero;
-    r.xb = xok[1] ? *(const bf16x8*)(x + xrow + xcol[1]) : zero;
-    r.d = (with_dy && dy_ok) ? *(const bf16x8*)(dy + (img + y) * W * Cout + dy_col) : zero;
-    return r;
+  auto load_d = [&](Row& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) r.d[h] = fetch(dp, dof[h]);
+    yd = yd + 1 == H ? 0 : yd + 1;
+    dp = yd ? dp + drow : dim;
   };
-  float bsum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto store_x = [&](const Regs& r, int32_t slot) __attribute__((always_inline)) {
+  auto begin = [&](uint32_t u) __attribute__((always_inline)) {
+    const uint32_t rest = u / cps, n = rest / segs;
+    const int32_t y0 = (int32_t)(u - rest * cps) * R, x0 = (int32_t)(rest - n * segs) * 32;
+    const int32_t w = W - x0 < 32 ? W - x0 : 32;
+    rows = R < H - y0 ? R : H - y0;
+#pragma unroll
+    for (int h = 0; h < 3; h++) {
+      const int32_t c = (lane >> 2) + 16 * h, ch = ciB + 8 * (lane & 3);
+      xo[h] = c <= w + 1 && ch < Cin ? (uint32_t)(wrapi(x0 + c - 1, W) * (int64_t)Cin + ch) * 2 : kBad;
+    }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      if (!xitem[h]) continue;
-      const bf16x8 v = h == 0 ? r.xa : r.xb;
+      const int32_t c = (lane >> 2) + 16 * h, ch = coB + 8 * (lane & 3);
+      dof[h] = c < w && ch < Cout ? (uint32_t)((x0 + c) * (int64_t)Cout + ch) * 2 : kBad;
+      // the strip's pixels among a lane's fragment elements
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int32_t row = 8 * xg[h] + e;
-        s_x[slot][row * LD + wg_col(row, xc[h])] = v[e];
+      for (int e = 0; e < 4; e++) {
+        const int32_t p = 16 * h + 8 * (lane >> 5) + 2 * e;
+        keep[h][e] = (p < w ? 0xffffu : 0u) | (p + 1 < w ? 0xffff0000u : 0u);
+      }
+    }
+    xim = x + (int64_t)n * H * xrow;
+    dim = dy + (int64_t)n * H * drow;
+    yx = y0 > 0 ? y0 - 1 : H - 1;
+    yd = y0;
+    xp = xim + yx * xrow;
+    dp = dim + yd * drow;
+    load_x(first);
+    load_x(second);
+    load_x(ring[0]);
+    load_d(ring[0]);
+#pragma unroll
+    for (int k = 1; k < D; k++) {
+      load_x(ring[k]);
+      load_d(ring[k]);
+    }
+  };
+  auto store_x = [&](const Row& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 3; h++) *(u32x4*)&s_x[at + 512 * h] = r.x[h];
+  };
+  // bias sums: channels 8 (lane % 4) .. of this lane's pixels
+  float bsum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  auto store_d = [&](const Row& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      *(u32x4*)&s_d[at + 512 * h] = r.d[h];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        bsum[2 * e] += __builtin_bit_cast(float, r.d[h][e] << 16);
+        bsum[2 * e + 1] += __builtin_bit_cast(float, r.d[h][e] & 0xffff0000u);
       }
     }
   };
-  auto store_dy = [&](const Regs& r, int32_t slot) __attribute__((always_inline)) {
-    if (!dy_item) return;
+  // fragments (16 pixels each): dY rows s, s + 1; X rows s .. s + 3 at the
+  // three column shifts
+  u32x4 fa[2][2], fb[4][3][2];
+  auto read_x = [&](u32x4 (*bb)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int32_t row = 8 * dg + e;
-      s_dy[slot][row * LD + wg_col(row, dpx)] = r.d[e];
-    }
-    if (do_bias) {
+    for (int d = 0; d < 3; d++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) bsum[e] += bf2f(r.d[e]);
+      for (int h = 0; h < 2; h++) bb[d][h] = frag(s_x + tr + (16 * h + d) * 32);
+  };
+  auto read_d = [&](u32x4* a) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) a[h] = frag(s_d + tr + 16 * h * 32);
+  };
+  // a narrow strip: zero against zero past its last pixel, whatever X holds
+  auto clip = [&](u32x4 (*bb)[2]) __attribute__((always_inline)) {
+    if (!RAG) return;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) bb[d][h][e] &= keep[h][e];
+  };
+  f32x16 acc[9];
+  // dY row s against X rows s, s + 1, s + 2, while the next rows go from
+  // registers through LDS to fragments
+  auto step = [&](int v, bool more) __attribute__((always_inline)) {
+    if (more) {
+      fence();
+      store_x(ring[(v + 1) % D]);
+      store_d(ring[(v + 1) % D]);
+      fence();
+      load_x(ring[(v + 1) % D]);
+      load_d(ring[(v + 1) % D]);
     }
+    clip(fb[(v + 2) & 3]);
+    if (more) {
+      read_x(fb[(v + 3) & 3]);
+      read_d(fa[(v + 1) & 1]);
+    }
+#pragma unroll
+    for (int t = 0; t < 9; t++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[v & 1][h]),
+                                                         __builtin_bit_cast(bf16x8, fb[(v + t / 3) & 3][t % 3][h]),
+                                                         acc[t], 0, 0, 0);
   };
 
-  const int32_t wr = (CB / 2) * (wave >> 1), wc = (IB / 2) * (wave & 1);
-  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
-  f32x4 acc[9][TI][TJ];
+  uint32_t u = ((uint32_t)chunk * 4 + wave) * per;
+  const uint32_t u1 = u + per < units ? u + per : units;
+  if (u < u1) begin(u);
 #pragma unroll
   for (int t = 0; t < 9; t++)
 #pragma unroll
-    for (int i = 0; i < TI; i++)
+    for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
+  while (u < u1) {
+    fence();
+    store_x(first);
+    fence();
+    read_x(fb[0]);
+    fence();
+    store_x(second);
+    fence();
+    read_x(fb[1]);
+    fence();
+    store_x(ring[0]);
+    store_d(ring[0]);
+    fence();
+    load_x(ring[0]);
+    load_d(ring[0]);
+    read_x(fb[2]);
+    read_d(fa[0]);
+    clip(fb[0]);
+    clip(fb[1]);
+    int32_t s = 0;
+    for (; s + D < rows; s += D) {
 #pragma unroll
-      for (int j = 0; j < TJ; j++) acc[t][i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+      for (int v = 0; v < D; v++) step(v, true);
+    }
+    const int32_t left = rows - s;  // 1 .. D
+#pragma unroll
+    for (int v = 0; v < D; v++)
+      if (v < left) step(v, v + 1 < left);
+    if (++u < u1) begin(u);
+  }
 
-  // prologue: X rows y0 - 1, y0, y0 + 1 and dY row y0, all loads in flight together
-  {
-    const Regs r0 = load(0, y0, true), r1 = load(1, y0, false), r2 = load(2, y0, false);
-    store_x(r0, 0);
-    store_x(r1, 1);
-    store_x(r2, 2);
-    store_dy(r0, 0);
+  // the four waves' sums, added in wave order
+  float* out = part + ((int64_t)chunk * nblk + blk) * kWgradPart;
+  f32x4* red = (f32x4*)s_wg;
+  float* s_bias = (float*)(s_wg + kWgradRed);
+#pragma unroll
+  for (int e = 0; e < 8; e++) {  // over the 16 lanes of a channel group
+#pragma unroll
+    for (int m = 4; m < 64; m *= 2) bsum[e] += __shfl_xor(bsum[e], m);
+  }
+  if (lane < 4) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) s_bias[wave * 32 + 8 * lane + e] = bsum[e];
   }
   __syncthreads();
-  for (int32_t s = 0; s < rows; s++) {
-    const bool more = s + 1 < rows;
-    Regs nx;
-    if (more) nx = load(s + 3, y0 + s + 1, true);
-    const int32_t ds = s & 1;
-    bf16x8 a[TI];
 #pragma unroll
-    for (int i = 0; i < TI; i++) {
-      const int32_t row = wr + 16 * i + rl;
-      a[i] = *(const bf16x8*)&s_dy[ds][row * LD + wg_col(row, kq)];
+  for (int t = 0; t < 9; t++)
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      red[(wave * 36 + t * 4 + q) * 64 + lane] =
+          (f32x4){acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const int32_t f = 4 * k + wave;
+    f32x4 v = red[f * 64 + lane];
+#pragma unroll
+    for (int j = 1; j < 4; j++) v += red[(j * 36 + f) * 64 + lane];
+    if (dw) {
+      wgrad_put(dw, v, k, wave, lane, coB, ciB, Cin, Cout);
+    } else {
+      *(f32x4*)(out + (f * 64 + lane) * 4) = v;
     }
-#pragma unroll
-    for (int dyi = 0; dyi < 3; dyi++) {
-      const bf16* xr = s_x[(s + dyi) & 3];
-#pragma unroll
-      for (int j = 0; j < TJ; j++) {
-        const int32_t row = wc + 16 * j + rl;
-        const u32x4 v0 = *(const u32x4*)&xr[row * LD + wg_col(row, kq)];
-        const uint32_t v1 = *(const uint32_t*)&xr[row * LD + wg_col(row, kq + 8)];
-        const u32x4 vm = v0;  // columns kq .. kq + 7: pixel x + dx for dx = -1
-        const u32x4 vz = {__builtin_amdgcn_alignbit(v0[1], v0[0], 16), __builtin_amdgcn_alignbit(v0[2], v0[1], 16),
-                          __builtin_amdgcn_alignbit(v0[3], v0[2], 16), __builtin_amdgcn_alignbit(v1, v0[3], 16)};
-        const u32x4 vp = {v0[1], v0[2], v0[3], v1};
-        const bf16x8 bm = __builtin_bit_cast(bf16x8, vm), bz = __builtin_bit_cast(bf16x8, vz),
-                     bp = __builtin_bit_cast(bf16x8, vp);
-#pragma unroll
-        for (int i = 0; i < TI; i++) {
-          acc[3 * dyi + 0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bm, acc[3 * dyi + 0][i][j], 0, 0, 0);
-          acc[3 * dyi + 1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bz, acc[3 * dyi + 1][i][j], 0, 0, 0);
-          acc[3 * dyi + 2][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bp, acc[3 * dyi + 2][i][j], 0, 0, 0);
-        }
-      }
-    }
-    if (more) {
-      store_x(nx, (s + 3) & 3);
-      store_dy(nx, ds ^ 1);
-    }
-    __syncthreads();
   }
-
-  const int64_t nw = (int64_t)Cout * 9 * Cin;
-  float* out = part + (int64_t)chunk * (nw + Cout);
-  // D rows (co) = wr + 16 i + 4 (lane / 16) + e, column (ci) = wc + 16 j + lane % 16
-#pragma unroll
-  for (int j = 0; j < TJ; j++) {
-    const int32_t ci = ciB + wc + 16 * j + rl;
-    if (ci >= Cin) continue;
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int32_t co = coB + wr + 16 * i + 4 * (lane >> 4) + e;
-        if (co >= Cout) continue;
-#pragma unroll
-        for (int t = 0; t < 9; t++) out[((int64_t)co * 9 + t) * Cin + ci] = acc[t][i][j][e];
-      }
-  }
-  if (do_bias) {  // the 32 pixel columns' sums per channel, added in a fixed order
-    if (dy_item) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) s_b[dpx][8 * dg + e] = bsum[e];
-    }
-    __syncthreads();
-    if (tid < CB) {
-      float sb = 0.0f;
-      for (int k = 0; k < 32; k++) sb += s_b[k][tid];
-      if (coB + tid < Cout) out[nw + coB + tid] = sb;
-    }
+  if (tid < 32) {
+    const float v = s_bias[tid] + s_bias[32 + tid] + s_bias[64 + tid] + s_bias[96 + tid];
+    if (!dw) out[9 * 32 * 32 + tid] = v;
+    else if (db && ciB == 0 && coB + tid < Cout) db[coB + tid] = v;
   }
 }
 
-// dw[i] (i < nw) and db[i - nw] (nw <= i < nw + Cout, when db is given):
-// the chunks' partials added in a fixed order.  A workgroup takes 64
-// consecutive entries; its 16 groups of 16 threads read them as float4 runs
-// from every 16th chunk (group g: chunks g, g + 16, ...), and the groups'
-// sums are added in group order.  Rows are nw + Cout floats, a multiple of
-// 8 (Cin % 8 == Cout % 8 == 0), so the runs are aligned.
-__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, float* __restrict__ dw,
-                                                      float* __restrict__ db, int64_t nw, int32_t Cout,
-                                                      int32_t nparts) {
-  __shared__ float s_sum[16][65];
-  const int32_t tid = threadIdx.x, c4 = tid & 15, g = tid >> 4;
-  const int64_t stride = nw + Cout;
-  const int64_t n = db ? stride : nw;
-  const int64_t i0 = (int64_t)blockIdx.x * 64 + 4 * c4;
+// dw and db (optional) from k_wgrad's partials, the chunks added in a fixed
+// order: a workgroup takes 1024 / NG consecutive floats of a block; its NG
+// groups of threads read them as 16-byte runs from every NG-th chunk (group q:
+// chunks q, q + NG, ...), and the groups' sums are added in group order.
+template <int NG>
+__global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ part, float* __restrict__ dw,
+                                                   float* __restrict__ db, int32_t Cin, int32_t Cout, int32_t nblk,
+                                                   int32_t nparts) {
+  constexpr int TG = 256 / NG, kTiles = (kWgradPart / 4 + TG - 1) / TG;
+  __shared__ f32x4 s_sum[NG][TG];
+  const int32_t tid = threadIdx.x, c = tid % TG, q = tid / TG;
+  const int32_t blk = (int32_t)blockIdx.x / kTiles, at = ((int32_t)blockIdx.x % kTiles) * TG + c;
+  const int64_t stride = (int64_t)nblk * kWgradPart;
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (i0 < n) {
-    const float* p = part + i0;
-    int32_t k = g;
-    // four chunks' loads in flight per step; the adds stay in chunk order
-    for (; k + 48 < nparts; k += 64) {
-      const f32x4 v0 = *(const f32x4*)(p + (int64_t)k * stride);
-      const f32x4 v1 = *(const f32x4*)(p + (int64_t)(k + 16) * stride);
-      const f32x4 v2 = *(const f32x4*)(p + (int64_t)(k + 32) * stride);
-      const f32x4 v3 = *(const f32x4*)(p + (int64_t)(k + 48) * stride);
-      acc += v0;
-      acc += v1;
-      acc += v2;
-      acc += v3;
-    }
-    for (; k < nparts; k += 16) acc += *(const f32x4*)(p + (int64_t)k * stride);
-  }
+  if (4 * at < kWgradPart) {
+    const float* p = part + (int64_t)blk * kWgradPart + 4 * at;
+    int32_t k = q;
+    // eight chunks' loads in flight per step; the adds stay in chunk order
+    for (; k + 7 * NG < nparts; k += 8 * NG) {
+      f32x4 v[8];
 #pragma unroll
-  for (int e = 0; e < 4; e++) s_sum[g][4 * c4 + e] = acc[e];
+      for (int i = 0; i < 8; i++) v[i] = *(const f32x4*)(p + (int64_t)(k + i * NG) * stride);
+#pragma unroll
+      for (int i = 0; i < 8; i++) acc += v[i];
+    }
+    for (; k < nparts; k += NG) acc += *(const f32x4*)(p + (int64_t)k * stride);
+  }
+  s_sum[q][c] = acc;
   __syncthreads();
-  if (tid < 64) {
-    const int64_t i = (int64_t)blockIdx.x * 64 + tid;
-    if (i < n) {
-      float s = 0.0f;
+  if (q != 0 || 4 * at >= kWgradPart) return;
 #pragma unroll
-      for (int q = 0; q < 16; q++) s += s_sum[q][tid];
-      if (i < nw) dw[i] = s;
-      else db[i - nw] = s;
+  for (int i = 1; i < NG; i++) acc += s_sum[i][c];
+  const int32_t nci = (Cin + 31) / 32, ciB = (blk % nci) * 32, coB = (blk / nci) * 32;
+  if (at >= 9 * 256) {
+    const int32_t co = coB + 4 * at - 9 * 32 * 32;
+    if (db && ciB == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (co + e < Cout) db[co + e] = acc[e];
     }
+    return;
   }
+  wgrad_put(dw, acc, at / 256, at / 64 % 4, at % 64, coB, ciB, Cin, Cout);
 }
 
 // ---------------------------------------------------------------------------
@@ -1411,87 +1397,78 @@ int swe_nn_flip(const void* w, int32_t Cin, int32_t Cout, void* wt, void* stream
   SWENN_LAUNCH_CHECK();
 }
 
-// How a weight gradient is split.  Maps whose rows are whole 32-pixel
-// strips take k_wgrad_rows: CB x IB channel blocks (32; 64 where the layer
-// has that many channels when SWENN_WGRAD_BLOCK is 64), each strip cut into
-// chunks of R rows, enough chunks for ~SWENN_WGRAD_WGS workgroups but at
-// most ceil(H / 8) a strip.  Measured on the surrogate's training layers
-// (MI355X, batch 8 at 256^2): 32 x 32 blocks and 1024 workgroups are the
-// fastest (64 x 64 blocks hold 356 registers a lane, one wave per SIMD).  Others take k_wgrad: 64 x 64 blocks of
-// one tap over chunks of `chunk` pixels (~1024 workgroups, >= 256 pixels, a
-// multiple of 32).  Either way the partials are [chunks][Cout*9*Cin + Cout].
-#ifndef SWENN_WGRAD_BLOCK
-#define SWENN_WGRAD_BLOCK 32
-#endif
-#ifndef SWENN_WGRAD_WGS
-#define SWENN_WGRAD_WGS 1024
-#endif
-#ifndef SWENN_WGRAD_ROWS
-#define SWENN_WGRAD_ROWS 1
-#endif
+// How a weight gradient is split: 32 x 32 channel blocks, each over `chunks`
+// workgroups of four waves with `per` units a wave.  One round of workgroups
+// (a CU holds one), units as long as that allows (a unit loads two X rows more
+// than it has), but of at least six rows: below, a wave's ~5 us outside its
+// rows and the partials outweigh the 0.5 us a row.  Measured (us, with the pass
+// over the partials) for a least of four / six / eight rows: 128 -> 192 at
+// 32^2, batch 8, 16.8 / 16.6 / 15.9; 32 -> 32 at 200 x 230, batch 3, 17.8 /
+// 17.0 / 16.1; 192 -> 256 at 12 x 16, batch 2, 11.9 / 10.1 / 9.8; the other
+// way 32 -> 32 at 256^2, batch 1, 12.9 / 13.7 / 13.8; 64 -> 64 at 300 x 9,
+// 14.2 / 15.0 / 15.2.  Chunks of at most eight rows in all become one, whose
+// workgroups write the result: 256 -> 192 at 4^2, batch 2, 12.7 -> 9.5; to
+// sixteen rows it loses (192 -> 256 at 8^2, batch 8, 14.6 -> 19.0).
+constexpr int32_t kWgradMinRows = 6, kWgradOneChunk = 8;
 struct WgradPlan {
-  bool rows;
-  int32_t cb, ib, R;
-  int64_t chunk, chunks, blocks;
+  int32_t R;
+  int64_t blocks, units, per, chunks;
 };
 
 static WgradPlan wgrad_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   WgradPlan p{};
-  const int64_t npix = (int64_t)N * H * W;
-  if (SWENN_WGRAD_ROWS && W % 32 == 0) {
-    p.rows = true;
-    p.cb = Cout >= 64 && SWENN_WGRAD_BLOCK >= 64 ? 64 : 32;
-    p.ib = Cin >= 64 && SWENN_WGRAD_BLOCK >= 64 ? 64 : 32;
-    p.blocks = (int64_t)((Cout + p.cb - 1) / p.cb) * ((Cin + p.ib - 1) / p.ib);
-    const int64_t strips = (int64_t)N * (W / 32);
-    int64_t cps = (SWENN_WGRAD_WGS + strips * p.blocks - 1) / (strips * p.blocks);
-    const int64_t cmax = (H + 7) / 8;
-    if (cps > cmax) cps = cmax;
-    if (cps < 1) cps = 1;
-    p.R = (int32_t)((H + cps - 1) / cps);
-    p.chunks = strips * ((H + p.R - 1) / p.R);
-  } else {
-    p.blocks = (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64);
-    int64_t c = (npix * p.blocks + 1023) / 1024;
-    c = (c + 31) / 32 * 32;
-    p.chunk = c < 256 ? 256 : c;
-    p.chunks = (npix + p.chunk - 1) / p.chunk;
+  p.blocks = (int64_t)((Cout + 31) / 32) * ((Cin + 31) / 32);
+  const int64_t strips = (int64_t)N * ((W + 31) / 32), waves = p.blocks >= 256 ? 4 : 4 * (256 / p.blocks);
+  int64_t cps = waves / strips;
+  const int64_t cmax = (H + kWgradMinRows - 1) / kWgradMinRows;
+  if (cps > cmax) cps = cmax;
+  if (cps < 1) cps = 1;
+  p.R = (int32_t)((H + cps - 1) / cps);
+  p.units = strips * ((H + p.R - 1) / p.R);
+  p.per = (p.units + waves - 1) / waves;
+  p.chunks = (p.units + 4 * p.per - 1) / (4 * p.per);
+  // a few rows more a wave cost less than the pass that adds the chunks
+  if (p.chunks * p.per * p.R <= kWgradOneChunk) {
+    p.per *= p.chunks;
+    p.chunks = 1;
   }
   return p;
 }
 
 int64_t swe_nn_wgrad_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   if (N < 1 || H < 1 || W < 1 || Cin < 1 || Cout < 1) return 0;
-  return wgrad_plan(N, H, W, Cin, Cout).chunks * ((int64_t)Cout * 9 * Cin + Cout);
+  const WgradPlan p = wgrad_plan(N, H, W, Cin, Cout);
+  return p.chunks * p.blocks * kWgradPart;
 }
-
 int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout,
                  float* dw, float* db, float* work, int64_t work_len, void* stream) {
   if (!x || !dy || !dw || !work || (uintptr_t)work % 16) return -1;
   if (N < 1 || H < 1 || W < 1 || Cin < 8 || Cout < 8 || Cin % 8 || Cout % 8) return -1;
   if (work_len < swe_nn_wgrad_work(N, H, W, Cin, Cout)) return -1;
   const WgradPlan p = wgrad_plan(N, H, W, Cin, Cout);
-  if (p.chunks > 0x7fffffffLL || p.chunk > 0x7fffffffLL || p.blocks > 65535) return -1;
-  const int64_t nw = (int64_t)Cout * 9 * Cin;
-  const dim3 grid((unsigned)p.chunks, (unsigned)p.blocks);
+  // what a grid's second axis once held: 64 x 64 blocks of one tap where a row
+  // is not whole strips
+  const int64_t tall = W % 32 ? (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64) : 0;
+  if (p.blocks > 65535 || tall > 65535 || p.chunks * p.blocks > 0x7fffffffLL) return -1;
+  if (p.units + 4 * p.per > 0xffffffffLL || (int64_t)W * (Cin > Cout ? Cin : Cout) * 2 >= 0xffffffffLL) return -1;
+  const dim3 grid((unsigned)(p.chunks * p.blocks));
   const bf16* xx = (const bf16*)x;
   const bf16* dd = (const bf16*)dy;
-  if (p.rows) {
-#define SWENN_ROWS_KERNEL(CB_, IB_)                                                                         \
-  hipLaunchKernelGGL((k_wgrad_rows<CB_, IB_>), grid, dim3(256), 0, S(stream), xx, dd, work, N, H, W, Cin, Cout, \
-                     p.R)
-    if (p.cb == 64 && p.ib == 64) SWENN_ROWS_KERNEL(64, 64);
-    else if (p.cb == 64) SWENN_ROWS_KERNEL(64, 32);
-    else if (p.ib == 64) SWENN_ROWS_KERNEL(32, 64);
-    else SWENN_ROWS_KERNEL(32, 32);
-#undef SWENN_ROWS_KERNEL
-  } else {
-    hipLaunchKernelGGL(k_wgrad, grid, dim3(256), 0, S(stream), xx, dd, work, N, H, W, Cin, Cout, (int32_t)p.chunk);
-  }
-  // one pass adds the chunks' weight and bias partials (contiguous per chunk)
-  const int64_t nred = db ? nw + Cout : nw;
-  hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((nred + 63) / 64)), dim3(256), 0, S(stream), work, dw, db, nw,
-                     Cout, (int32_t)p.chunks);
+  float* dw1 = p.chunks == 1 ? dw : nullptr;
+  if (W % 32)
+    hipLaunchKernelGGL(k_wgrad<true>, grid, dim3(256), kWgradLds, S(stream), xx, dd, work, dw1, db, H, W, Cin, Cout,
+                       p.R, (uint32_t)p.units, (uint32_t)p.per, (int32_t)p.blocks);
+  else
+    hipLaunchKernelGGL(k_wgrad<false>, grid, dim3(256), kWgradLds, S(stream), xx, dd, work, dw1, db, H, W, Cin, Cout,
+                       p.R, (uint32_t)p.units, (uint32_t)p.per, (int32_t)p.blocks);
+  // one pass adds the chunks' weight and bias partials
+  const int32_t nq = kWgradPart / 4;
+  if (p.chunks >= 32)
+    hipLaunchKernelGGL(k_wgrad_sum<16>, dim3((unsigned)(p.blocks * ((nq + 15) / 16))), dim3(256), 0, S(stream), work,
+                       dw, db, Cin, Cout, (int32_t)p.blocks, (int32_t)p.chunks);
+  else if (p.chunks > 1)
+    hipLaunchKernelGGL(k_wgrad_sum<4>, dim3((unsigned)(p.blocks * ((nq + 63) / 64))), dim3(256), 0, S(stream), work,
+                       dw, db, Cin, Cout, (int32_t)p.blocks, (int32_t)p.chunks);
   SWENN_LAUNCH_CHECK();
 }
 

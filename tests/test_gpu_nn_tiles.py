@@ -74,3 +74,33 @@ def test_conv_tile(N, H, W, Cin, Cout):
         torch.cuda.synchronize()
         assert torch.allclose(y32, ref.clamp_min(0), atol=1e-4 * (9 * Cin) ** 0.5, rtol=1e-4)
         assert torch.equal(y16, y32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("N,H,W,Cin,Cout", [
+    (1, 1, 1, 8, 8),         # one pixel: every tap is it
+    (2, 4, 4, 96, 40),       # one chunk: no pass over the partials
+    (1, 2, 33, 40, 24), (3, 3, 31, 32, 32), (1, 7, 95, 8, 72),  # 1 .. 7 rows, strips of 1, 31, 32 columns
+    (5, 13, 50, 64, 64),     # the last chunk of a strip one row shorter
+    (1, 260, 70, 32, 64),    # over 32 chunks
+    (3, 9, 70, 512, 520),    # three units a wave, a wave without one
+])
+def test_wgrad_units(N, H, W, Cin, Cout):
+    """k_wgrad's strips, rows and units against float64; columns past a strip's
+    end count for nothing even where the map holds infinities there."""
+    print("case wgrad units", N, H, W, Cin, Cout, flush=True)
+    x = rnd((N, H, W, Cin), seed=41)
+    dy = rnd((N, H, W, Cout), seed=42)
+    x[0, 0, min(32, W - 1), 3] = float("inf")
+    dw = torch.empty((Cout, 9, Cin), device=DEV)
+    db = torch.empty((Cout,), device=DEV)
+    work = nn.wgrad(x, dy, dw, db)
+    again = torch.empty_like(dw)
+    nn.wgrad(x, dy, again, None, work)
+    torch.cuda.synchronize()
+    xd, dd = x.cpu().double(), dy.cpu().double().reshape(-1, Cout)
+    taps = [torch.roll(xd, (1 - t // 3, 1 - t % 3), (1, 2)).reshape(-1, Cin) for t in range(9)]
+    ref = torch.stack([dd.T @ v for v in taps], 1)
+    tol = 1e-5 * (N * H * W) ** 0.5 + 1e-3
+    assert torch.allclose(dw.cpu().double(), ref, atol=tol, rtol=1e-4, equal_nan=True)
+    assert torch.allclose(db.cpu().double(), dd.sum(0), atol=tol, rtol=1e-4)
+    assert torch.equal(dw.view(torch.int32), again.view(torch.int32))
