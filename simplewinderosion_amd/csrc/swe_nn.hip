@@ -301,7 +301,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_tile_b
 // -> 20.4 / 23.7; 128 -> 128 at 64^2 27.6 / 32.2 -> 18.3 / 18.9; 192 -> 192 at
 // 32^2 28.4 / 28.0 -> 17.8 / 18.5; 256 -> 192 at 16^2 18.6 / 17.1 -> 14.0 /
 // 11.9; 64 -> 64 at 512^2, batch 1, 50.9 / 63.9 -> 40.3 / 42.9.  Reading one
-// chunk ahead across the taps' barriers took 10% longer (spills at 4 x 4).
+// chunk ahead across the taps' barriers took 10% longer (spills at 4 x 4), four
+// chunks at once 10% longer in the smallest shapes; the weights' loads a tap
+// earlier 7% longer at 4 x 4.
 // ---------------------------------------------------------------------------
 // 32-channel chunks of a block at most: KC <= 256, for the largest workgroups
 // 192 (their patch of more would not fit the LDS)
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT && PF
   uint32_t wo;
   {
     const int32_t j = brow >> 4, r = brow & 15;
-    const int32_t co = co0 + 32 * (j >> 1) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3);
+    const int32_t co = co0 + (CF == 1 ? r : 32 * (j >> 1) + 8 * (r >> 2) + 4 * (j & 1) + (r & 3));
     wo = co < Cout ? (uint32_t)((co * 9 * Cin + 8 * gg) * 2) : kBad;
   }
   // the weights of tap t of channel block k0 (zero past Cin and Cout)
@@ -1272,8 +1274,10 @@ static bool conv_tile(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout
     // -> 192 at 32^2, (4, 2) 17.7 (one round), (2, 4) 19.7 (one), (1, 2) 23.1
     // (two rounds of two), (2, 2) 25.5 (two); 128 -> 192 there, (2, 2) 13.3,
     // (4, 2) 14.8, (2, 4) 15.9; 128 -> 128 at 64^2, (2, 4) 18.2, (2, 2) 22.5,
-    // (4, 2) 24.7; 256 -> 192 at 16^2, (1, 2) 13.9, (2, 2) 16.0, (2, 4) 23.8.
-    static const int32_t kShape[][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {1, 2}};
+    // (4, 2) 24.7; 256 -> 192 at 16^2, (1, 2) 13.9, (2, 2) 16.0, (2, 4) 23.8;
+    // at batch 1 256 -> 256 at 16^2, (1, 1) 11.4, (1, 2) 13.4 (slices over
+    // workgroups and a pass that adds them: 13.3).
+    static const int32_t kShape[][2] = {{4, 4}, {4, 2}, {2, 4}, {2, 2}, {1, 2}, {1, 1}};
     double best = 0.0;
     for (const auto& sh : kShape) {
       const int32_t pf = sh[0], cf = sh[1], kmax = 32 * conv_wide_chunks(pf, cf);
@@ -1342,13 +1346,15 @@ static int conv_launch(const void* x, int32_t N, int32_t H, int32_t W, int32_t C
     if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CWS, 2, 4); }
     else if (ct.pf == 4 && ct.cf == 2) { SWENN_CT_S(SWENN_CWS, 4, 2); }
     else if (ct.pf == 2 && ct.cf == 2) { SWENN_CT_S(SWENN_CWS, 2, 2); }
-    else { SWENN_CT_S(SWENN_CWS, 1, 2); }
+    else if (ct.cf == 2) { SWENN_CT_S(SWENN_CWS, 1, 2); }
+    else { SWENN_CT_S(SWENN_CWS, 1, 1); }
   } else if (Cin > 32) {
     if (ct.pf == 4 && ct.cf == 4) { SWENN_CT_S(SWENN_CW, 4, 4); }
     else if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CW, 2, 4); }
     else if (ct.pf == 4 && ct.cf == 2) { SWENN_CT_S(SWENN_CW, 4, 2); }
     else if (ct.pf == 2 && ct.cf == 2) { SWENN_CT_S(SWENN_CW, 2, 2); }
-    else { SWENN_CT_S(SWENN_CW, 1, 2); }
+    else if (ct.cf == 2) { SWENN_CT_S(SWENN_CW, 1, 2); }
+    else { SWENN_CT_S(SWENN_CW, 1, 1); }
   } else {
     if (ct.pf == 4 && ct.cf == 4) { SWENN_CT_S(SWENN_CT, 4, 4); }
     else if (ct.pf == 2 && ct.cf == 4) { SWENN_CT_S(SWENN_CT, 2, 4); }

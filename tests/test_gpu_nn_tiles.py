@@ -26,8 +26,9 @@ CASES = [
     (8, 64, 64, 16, 136),     # (2, 4), a partial channel block
     (9, 64, 48, 16, 320),     # (2, 4), 16 columns
     # above 32 input channels; `2` is two weight buffers, `k` several blocks of channels
-    (1, 9, 16, 264, 24), (1, 9, 16, 72, 24),        # (1, 2), 16 columns: k, 2
-    (1, 9, 21, 264, 24), (2, 19, 21, 72, 24),       # (1, 2): 2 k, 2
+    (1, 9, 21, 264, 24), (1, 9, 16, 72, 24), (2, 19, 21, 72, 24),  # (1, 1): k; 16 columns 2; 2
+    (5, 9, 45, 264, 200), (5, 9, 45, 72, 200),      # (1, 2), 16 columns: k, 2
+    (8, 9, 21, 72, 200), (8, 9, 21, 40, 200),       # (1, 2): 2
     (5, 17, 45, 136, 200), (5, 17, 45, 72, 200),    # (2, 2), 16 columns: -, 2
     (5, 32, 21, 136, 200), (8, 33, 21, 264, 40),    # (2, 2): -, 2 k
     (5, 33, 45, 104, 200), (5, 17, 45, 264, 200),   # (2, 4), 16 columns: -, 2 k
