@@ -95,7 +95,7 @@ typedef struct swe_params {
                              window's snapshot; settling <= 0.25 only); 1 = colour-ordered (cells in
                              3x3 colour classes, one class after another, each reading the map the
                              earlier classes left: the reference's sequential cascades in class
-                             order; global path, single maps) */
+                             order) */
   int32_t reserved;       /* 0 */
 } swe_params;
 
@@ -192,7 +192,8 @@ int swe_set_path(swe_ctx* ctx, int32_t path);
  *     launch's tail; 0 = every tile in the SWE_TUNE_TILE_ORDER order.
  *     Default: 2 for contexts of up to 4096 tiles (16x32 cells each), 1
  *     above (measured best on a 1024^2 map and on a 64-terrain batch).
- *     Contexts of fewer than 64 tiles always use 0.
+ *     Contexts of fewer than 64 tiles always use 0, and by default so do
+ *     launches whose workgroups all fit the chip at once.
  *   SWE_TUNE_SHAPE: the step kernel's tile shape, an index into the
  *     compiled shapes 0 = 16x32 cells / 256 threads / 5 waves per SIMD
  *     (default), 1 = 32x16 / 256 / 5, 2 = 16x16 / 128 / 5, 3 = 16x32 / 256 / 4,

@@ -67,7 +67,7 @@ struct swe_ctx {
   int32_t path = 0;  // 0 auto, 1 global-atomic march, 2 tile-owned step
   int32_t tile_order = 0;  // SWE_TUNE_TILE_ORDER
   int32_t use_graph = 1;   // SWE_TUNE_GRAPH
-  int32_t heavy_first = -1;  // SWE_TUNE_HEAVY_FIRST; -1 = default (2 up to 4096 tiles, else 1)
+  int32_t heavy_first = -1;  // SWE_TUNE_HEAVY_FIRST; -1 = default (0 where one round holds every tile, 2 up to 4096 tiles, else 1)
   int32_t shape = 0;         // SWE_TUNE_SHAPE: index into swe::kStepShape
   // one captured map-cycle of the tile path per starting window parity, and
   // the launch configuration it was captured for
