@@ -489,11 +489,12 @@ __device__ __forceinline__ void step_body() {
     __syncthreads();
 
     // Masters below 2^39 at the start (heights below 128) stay below 2^47
-    // through the relax: with settling in [0, 1] a transfer is at most half
-    // the difference of the two heights, so heights stay within the region's
-    // range, and a cell's sediment sees at most 8 x 25 transfers.  Those take
-    // the short conversion.
-    const bool quick = s_large == 0 && ap->settling >= 0.0f && ap->settling <= 1.0f;
+    // through the relax: with settling in [0, 1] and a threshold of zero or
+    // more a transfer is at most half the difference of the two heights, so
+    // heights stay within the region's range, and a cell's sediment sees at
+    // most 8 x 25 transfers.  Those take the short conversion.
+    const bool quick =
+        s_large == 0 && ap->settling >= 0.0f && ap->settling <= 1.0f && ap->maxdiff >= 0.0f;
     // one cell's cascade on the LDS masters
     auto relax = [&](int32_t e) __attribute__((always_inline)) {
       const int32_t lx = row_of(e), ly = e - lx * RY;
