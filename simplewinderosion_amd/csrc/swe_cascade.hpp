@@ -114,9 +114,15 @@ __device__ __forceinline__ void cascade_cell_dev(const float hn[8], const SedOf&
   int64_t amt[8];
 #pragma unroll
   for (int r = 0; r < 8; r++) amt[r] = fx_from_small_f32(ts[r]);
+  // an amount that may saturate is rounded before its direction is applied:
+  // what the loser gives is what the taker gets, also at -2^63.  (The sign of
+  // ts is the direction, reversed by a negative settling factor.)
   if (__builtin_expect(big, 0)) {
 #pragma unroll
-    for (int r = 0; r < 8; r++) amt[r] = fx_from_f32(ts[r]);
+    for (int r = 0; r < 8; r++) {
+      const uint64_t m = (uint64_t)fx_from_f32(__builtin_copysignf(ts[r], settling));
+      amt[r] = (int64_t)((ts[r] < 0.0f) != (settling < 0.0f) ? 0 - m : m);
+    }
   }
 #pragma unroll
   for (int r = 0; r < 8; r++) emit(kk[r], amt[r]);
