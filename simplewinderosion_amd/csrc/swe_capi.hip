@@ -256,15 +256,29 @@ int32_t heavy_first_mode(const swe_ctx* c) {
   return c->heavy_first >= 0 ? c->heavy_first : (c->ntiles <= 4096 ? 2 : 1);
 }
 
+// widest halo of the colour-ordered relax over a context's terrains
+swe::ColourHalo colour_halo_of(const swe_ctx* c) {
+  swe::ColourHalo w = swe::kColourHalo;
+  for (int32_t k = 0; k < c->nterr; k++) {
+    const swe::ColourHalo h = swe::colour_halo(c->tnx[(size_t)k], c->tny[(size_t)k], c->p.periodic != 0);
+    w.xl = std::max(w.xl, h.xl);
+    w.xh = std::max(w.xh, h.xh);
+    w.yl = std::max(w.yl, h.yl);
+    w.yh = std::max(w.yh, h.yh);
+  }
+  return w;
+}
+
 // Tiles whose workgroups are all resident at once: the chip's 256 CUs times
-// the workgroups a CU holds (the shape's waves per SIMD; three of the
-// colour-ordered kernel's, by its LDS).  A launch of no more has no order to
+// the workgroups a CU holds (the shape's waves per SIMD; of the
+// colour-ordered kernel's also its LDS).  A launch of no more has no order to
 // choose, so by default it lists no tiles: the lists cost a dependent load
 // before the halo and a returning atomic at the end (256^2 map, 128 tiles:
 // 25.7 ms for three cycles with them, 24.0 ms without).
 int64_t resident_tiles(const swe_ctx* c) {
   const swe::StepShape sh = swe::kStepShape[c->shape];
-  return 256 * (colour_mode(c->p) ? 3 : 4 * sh.waves / (sh.threads / 64));
+  if (colour_mode(c->p)) return swe::colour_resident(sh, colour_halo_of(c), c->p.track != 0, c->p.layers);
+  return 256 * (4 * sh.waves / (sh.threads / 64));
 }
 
 // light-tile slots of a launch: half the tiles, a multiple of 8
@@ -583,15 +597,8 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   // kernel only moves the particles (MODE 2), and its relax follows at once
   // as one launch per colour class, with no closing relax-only window.
   bool alias = false;
-  sa.chalo = swe::kColourHalo;
-  for (int32_t k = 0; k < c->nterr; k++) {
-    alias = alias || c->tnx[(size_t)k] < 3 || c->tny[(size_t)k] < 3;
-    const swe::ColourHalo h = swe::colour_halo(c->tnx[(size_t)k], c->tny[(size_t)k], c->p.periodic != 0);
-    sa.chalo.xl = std::max(sa.chalo.xl, h.xl);
-    sa.chalo.xh = std::max(sa.chalo.xh, h.xh);
-    sa.chalo.yl = std::max(sa.chalo.yl, h.yl);
-    sa.chalo.yh = std::max(sa.chalo.yh, h.yh);
-  }
+  for (int32_t k = 0; k < c->nterr; k++) alias = alias || c->tnx[(size_t)k] < 3 || c->tny[(size_t)k] < 3;
+  sa.chalo = colour_halo_of(c);
   const bool colour = colour_mode(c->p) && alias, fused = colour_mode(c->p) && !alias;
   swe::RelaxArgs ra{};
   ra.nx = c->nx;

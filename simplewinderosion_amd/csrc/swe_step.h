@@ -44,6 +44,26 @@ inline ColourHalo colour_halo(int32_t nx, int32_t ny, bool periodic) {
   return nx % 3 <= 1 && ny % 3 <= 1 && nx >= 16 && ny >= 16 ? kColourHaloSeam : kColourHaloMax;
 }
 
+// Dynamic LDS of k_colour_step: the region's masters, events, list and
+// classes, or the march's accumulators
+inline int64_t colour_lds(const StepShape& sh, const ColourHalo& h, bool track, int32_t layers) {
+  const int64_t ry = sh.sy + h.yl + h.yh, r = (sh.sx + h.xl + h.xh) * ry;
+  const int64_t relax = r * (8 * layers + 4 + 2 + 1) + 2 * (ry + 8);
+  const int64_t march = (int64_t)sh.sx * sh.sy * (8 * layers + 4 + (track ? 32 : 0));
+  return ((relax > march ? relax : march) + 15) / 16 * 16;
+}
+
+// Workgroups of k_colour_step that the chip's 256 CUs hold at once: four waves
+// a SIMD, and in 160 KB of LDS a CU (taken in steps of 1280 bytes) what
+// colour_lds gives, the tile's new snapshots and up to 512 bytes of counters.
+// 1024 tiles of 16 x 32 cells with one layer, 768 with two; 768 and 512 near
+// the widest halo.
+inline int64_t colour_resident(const StepShape& sh, const ColourHalo& h, bool track, int32_t layers) {
+  const int64_t lds = colour_lds(sh, h, track, layers) + 4 * (int64_t)(sh.sx + 2) * (sh.sy + 2) * layers + 512;
+  const int64_t by_lds = 163840 / ((lds + 1279) / 1280 * 1280), by_waves = 16 / (sh.threads / 64);
+  return 256 * (by_lds < by_waves ? by_lds : by_waves);
+}
+
 // One terrain of a context: its cells, tiles and particles are contiguous
 // ranges of the context's buffers
 struct Terrain {

@@ -1225,16 +1225,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
 }
 
-// dynamic LDS of k_colour_step: the region's masters, events, list and
-// classes, or the march's accumulators
-template <int SX, int SY>
-inline size_t colour_lds(const ColourHalo& h, bool track, int layers) {
-  const size_t ry = (size_t)(SY + h.yl + h.yh), r = (size_t)(SX + h.xl + h.xh) * ry;
-  const size_t relax = r * (8 * (size_t)layers + 4 + 2 + 1) + 2 * (ry + 8);
-  const size_t march = (size_t)SX * SY * (8 * (size_t)layers + 4 + (track ? 32 : 0));
-  return ((relax > march ? relax : march) + 15) & ~(size_t)15;
-}
-
 // ---------------------------------------------------------------------------
 // Launchers of one shape (instantiated per shape in swe_step_shapes.hip)
 // ---------------------------------------------------------------------------
@@ -1249,7 +1239,7 @@ struct StepLauncher {
       h.xh = a.chalo.xh > h.xh ? a.chalo.xh : h.xh;
       h.yl = a.chalo.yl > h.yl ? a.chalo.yl : h.yl;
       h.yh = a.chalo.yh > h.yh ? a.chalo.yh : h.yh;
-      const unsigned lds = (unsigned)colour_lds<SX, SY>(h, T, L);
+      const unsigned lds = (unsigned)colour_lds(StepShape{SX, SY, NT, WPE}, h, T, L);
       if (mode == 3)
         hipLaunchKernelGGL((k_colour_step<SX, SY, NT, P, T, L, D, 3>), dim3(g), dim3(NT), lds, s, a);
       else

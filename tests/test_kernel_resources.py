@@ -71,3 +71,38 @@ def test_step_kernel_budget(metadata, shape):
         assert f["vgpr_count"] <= vgpr_max, (name, f["vgpr_count"])
         assert f.get("vgpr_spill_count", 0) == 0, name
         assert groups_per_cu * f["group_segment_fixed_size"] <= LDS_PER_CU, (name, f["group_segment_fixed_size"])
+
+
+def test_colour_residency(metadata, tmp_path):
+    """The workgroups that colour_resident (csrc/swe_step.h) says the chip
+    holds of k_colour_step: what the compiled kernels' static LDS and registers
+    leave room for, for every shape, halo and number of layers."""
+    src = tmp_path / "resident.cpp"
+    src.write_text('''#include <cstdio>
+#include "%s/swe_step.h"
+using namespace swe;
+int main() {
+  const ColourHalo hs[] = {kColourHalo, kColourHaloSeam, kColourHaloMax};
+  for (int i = 0; i < kStepShapes; i++)
+    for (int h = 0; h < 3; h++)
+      for (int t = 0; t < 2; t++)
+        for (int l = 1; l <= 2; l++)
+          printf("%%d %%d %%d %%d %%ld %%ld\\n", i, h, t, l, (long)colour_lds(kStepShape[i], hs[h], t, l),
+                 (long)colour_resident(kStepShape[i], hs[h], t, l));
+}
+''' % B.CSRC)
+    exe = str(tmp_path / "resident")
+    subprocess.run([B.hipcc(), "-std=c++17", "--offload-arch=gfx950", "-x", "hip", str(src), "-o", exe], check=True,
+                   capture_output=True)
+    rows = [tuple(int(v) for v in line.split()) for line in
+            subprocess.run([exe], check=True, capture_output=True, text=True).stdout.splitlines()]
+    assert len(rows) == 60
+    for i, h, t, layers, lds, resident in rows:
+        _, _, threads, _ = SHAPES[i]
+        mine = [f for k, f in metadata[i].items() if "k_colour_step" in k and "ELi%dE" % layers in k.split("Lb")[2]]
+        assert len(mine) == 16
+        static = max(f["group_segment_fixed_size"] for f in mine)
+        regs = max(f["vgpr_count"] for f in mine)
+        by_lds = LDS_PER_CU // (-(-(static + lds) // 1280) * 1280)
+        by_waves = 4 * min(512 // (-(-regs // 8) * 8), 8) // (threads // 64)
+        assert resident == 256 * min(by_lds, by_waves), (i, h, t, layers)
