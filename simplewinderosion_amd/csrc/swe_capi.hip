@@ -269,15 +269,32 @@ swe::ColourHalo colour_halo_of(const swe_ctx* c) {
   return w;
 }
 
+// Whether a window's colour-ordered relax runs inside the step kernel
+// (colour_fused), not as class launches after it.  On maps under three cells
+// along an axis a cell's neighbours alias across the wrap: class launches.
+bool fused_colour(const swe_ctx* c, int64_t particles) {
+  if (!colour_mode(c->p)) return false;
+  int32_t cx = 0, cy = 0;
+  for (int32_t k = 0; k < c->nterr; k++) {
+    const int32_t nx = c->tnx[(size_t)k], ny = c->tny[(size_t)k];
+    if (nx < 3 || ny < 3) return false;
+    cx = std::max(cx, 3 + (c->p.periodic ? nx % 3 : 0));
+    cy = std::max(cy, 3 + (c->p.periodic ? ny % 3 : 0));
+  }
+  const int64_t res =
+      swe::colour_resident(swe::kStepShape[c->shape], colour_halo_of(c), c->p.track != 0, c->p.layers);
+  return swe::colour_fused(c->ntiles, res, cx * cy, c->p.layers, (double)particles / (double)c->ncell);
+}
+
 // Tiles whose workgroups are all resident at once: the chip's 256 CUs times
 // the workgroups a CU holds (the shape's waves per SIMD; of the
 // colour-ordered kernel's also its LDS).  A launch of no more has no order to
 // choose, so by default it lists no tiles: the lists cost a dependent load
 // before the halo and a returning atomic at the end (256^2 map, 128 tiles:
 // 25.7 ms for three cycles with them, 24.0 ms without).
-int64_t resident_tiles(const swe_ctx* c) {
+int64_t resident_tiles(const swe_ctx* c, bool fused) {
   const swe::StepShape sh = swe::kStepShape[c->shape];
-  if (colour_mode(c->p)) return swe::colour_resident(sh, colour_halo_of(c), c->p.track != 0, c->p.layers);
+  if (fused) return swe::colour_resident(sh, colour_halo_of(c), c->p.track != 0, c->p.layers);
   return 256 * (4 * sh.waves / (sh.threads / 64));
 }
 
@@ -564,7 +581,8 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   sa.tile_order = c->tile_order;
   // listed crowded tiles get the first workgroups of a launch; at most one
   // slot per 8 tiles, a multiple of 8 (none on maps under 64 tiles)
-  const int32_t hf = c->ntiles <= resident_tiles(c) && c->heavy_first < 0 ? 0 : heavy_first_mode(c);
+  const bool fused = fused_colour(c, total), colour = colour_mode(c->p) && !fused;
+  const int32_t hf = c->ntiles <= resident_tiles(c, fused) && c->heavy_first < 0 ? 0 : heavy_first_mode(c);
   sa.heavy_slots = hf ? (int32_t)std::min<int64_t>(swe::kHeavySlotsMax, (c->ntiles / 8) & ~7LL) : 0;
   // light tiles last (heavy-first mode 2, maps of 64 tiles or more): the
   // usual order is padded to a multiple of 8 so that slot b runs on XCD b % 8
@@ -592,14 +610,10 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   sp.tile_sy = swe::kStepShape[c->shape].sy;
 
   // colour-ordered cascade: inside the step kernel (k_colour_step), with the
-  // same windows as the synchronous one.  On maps under three cells along an
-  // axis a cell's neighbours alias across the wrap; there every window's step
-  // kernel only moves the particles (MODE 2), and its relax follows at once
-  // as one launch per colour class, with no closing relax-only window.
-  bool alias = false;
-  for (int32_t k = 0; k < c->nterr; k++) alias = alias || c->tnx[(size_t)k] < 3 || c->tny[(size_t)k] < 3;
+  // same windows as the synchronous one, or as class launches: then every
+  // window's step kernel only moves the particles (MODE 2) and its relax
+  // follows at once, with no closing relax-only window
   sa.chalo = colour_halo_of(c);
-  const bool colour = colour_mode(c->p) && alias, fused = colour_mode(c->p) && !alias;
   swe::RelaxArgs ra{};
   ra.nx = c->nx;
   ra.ny = c->ny;

@@ -64,6 +64,35 @@ inline int64_t colour_resident(const StepShape& sh, const ColourHalo& h, bool tr
   return 256 * (by_lds < by_waves ? by_lds : by_waves);
 }
 
+// Whether a window of the colour-ordered cascade runs as one launch
+// (k_colour_step) or as a step launch and one launch per colour class.  Fused,
+// a window costs its rounds of workgroups (tiles / resident), each running 3
+// to 5 regions' cascades a tile; the classes cost `classes` launches, which
+// past a few rounds fill the chip too.  So the line is a number of rounds that
+// grows with the classes, and moves out where few cells are visited (a tile's
+// cascades are then few) or, with one layer, nearly all are (their events
+// shrink to the steep cells).  Measured, ms a 66-window cycle fused / classes:
+// 1024^2 periodic (16 classes, 2.7 rounds), two layers, 0.25 particles a cell
+// 10.8 / 12.3; 726^2 (9, 1.4) 6.9 / 6.9; 900^2 (9, 2.2) 9.4 / 8.6; 1025^2
+// (25, 4.2) 15.8 / 15.8; 2048^2 (25, 16) 45.2 / 27.3; one layer there (10.7)
+// 26.2 / 19.7, at one particle a cell 1281^2 (9, 3.2) 10.4 / 10.3; at 0.08
+// 2050^2 (16, 10.9), two layers, 19.9 / 20.2; at 0.02 always fused up to 10
+// rounds (2048^2, 16 rounds, 22.2 / 22.0).  Over 322 maps, densities and
+// layers the choice costs 0.3% more than the better of the two.
+inline bool colour_fused(int64_t tiles, int64_t resident, int32_t classes, int32_t layers, double per_cell) {
+  double rounds;
+  if (per_cell < 0.2) {
+    rounds = classes * (0.04 + 0.04 / (per_cell > 0.033 ? per_cell : 0.033)) * (layers == 1 ? 1.3 : 1.0);
+  } else if (layers == 1) {
+    rounds = per_cell < 0.5 ? 0.225 * classes : 0.46 * classes;
+    if (rounds > 10.0) rounds = 10.0;
+  } else {
+    rounds = 0.2 * classes - 0.5;
+    if (rounds > 4.0) rounds = 4.0;
+  }
+  return (double)tiles <= rounds * (double)resident;
+}
+
 // One terrain of a context: its cells, tiles and particles are contiguous
 // ranges of the context's buffers
 struct Terrain {

@@ -100,8 +100,8 @@ __device__ __forceinline__ StepArgsPtr step_args(StepArgsPtr p) {
 // call per particle; MODE 1: the relax only (the cycle's last window);
 // MODE 2: the fly() calls only -- the previous window was relaxed before the
 // launch by the colour-ordered cascade (one launch per colour class, on maps
-// of fewer than three cells along an axis), so the tile reads the snapshot and
-// masters as they are.
+// under three cells along an axis and where colour_fused prefers it), so the
+// tile reads the snapshot and masters as they are.
 // MODE 3, 4 (k_colour_step below): as 0 and 1 with the colour-ordered
 // cascade run inside the tile.
 template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
