@@ -191,9 +191,11 @@ int swe_set_path(swe_ctx* ctx, int32_t path);
  *     the last workgroups (on its own XCD), so short workgroups fill the
  *     launch's tail; 0 = every tile in the SWE_TUNE_TILE_ORDER order.
  *     Default: 2 for contexts of up to 4096 tiles (16x32 cells each), 1
- *     above (measured best on a 1024^2 map and on a 64-terrain batch).
- *     Contexts of fewer than 64 tiles always use 0, and by default so do
- *     launches whose workgroups all fit the chip at once.
+ *     above (measured best on a 1024^2 map and on a 64-terrain batch); by
+ *     default a call whose tiles hold at most 384 particles on average runs 1
+ *     in place of 2, and one whose workgroups all fit the chip at once 0
+ *     (swe_get_tune returns the setting, not what a call made of it).
+ *     Contexts of fewer than 64 tiles always use 0.
  *   SWE_TUNE_SHAPE: the step kernel's tile shape, an index into the
  *     compiled shapes 0 = 16x32 cells / 256 threads / 5 waves per SIMD
  *     (default), 1 = 32x16 / 256 / 5, 2 = 16x16 / 128 / 5, 3 = 16x32 / 256 / 4,

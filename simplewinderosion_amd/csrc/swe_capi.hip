@@ -67,7 +67,7 @@ struct swe_ctx {
   int32_t path = 0;  // 0 auto, 1 global-atomic march, 2 tile-owned step
   int32_t tile_order = 0;  // SWE_TUNE_TILE_ORDER
   int32_t use_graph = 1;   // SWE_TUNE_GRAPH
-  int32_t heavy_first = -1;  // SWE_TUNE_HEAVY_FIRST; -1 = default (0 where one round holds every tile, 2 up to 4096 tiles, else 1)
+  int32_t heavy_first = -1;  // SWE_TUNE_HEAVY_FIRST; -1 = default (heavy_first_launch)
   int32_t shape = 0;         // SWE_TUNE_SHAPE: index into swe::kStepShape
   // one captured map-cycle of the tile path per starting window parity, and
   // the launch configuration it was captured for
@@ -247,7 +247,8 @@ int ensure_particles(swe_ctx* c, int64_t n) {
   return 0;
 }
 
-// SWE_TUNE_HEAVY_FIRST in effect.  By default light tiles also go last when
+// SWE_TUNE_HEAVY_FIRST as set, or its default for well filled tiles
+// (heavy_first_launch: what a launch runs).  Light tiles also go last when
 // a launch is a few rounds of workgroups (up to 4096 tiles: 3.2 rounds at
 // five 16x32 tiles per CU), where the order of the last round sets the
 // launch's tail; with many rounds the tail matters little and moving tiles
@@ -296,6 +297,19 @@ int64_t resident_tiles(const swe_ctx* c, bool fused) {
   const swe::StepShape sh = swe::kStepShape[c->shape];
   if (fused) return swe::colour_resident(sh, colour_halo_of(c), c->p.track != 0, c->p.layers);
   return 256 * (4 * sh.waves / (sh.threads / 64));
+}
+
+// The mode a call's launches run: the setting, or by default none where one
+// round holds every tile, and no light lists where the mean load of a tile is
+// below 1.5 times kLightMax.  Most tiles are light then, and half of them wait
+// for the light slots, away from the tiles whose halo lines they share
+// (1537x1024, two layers, 0.2 particles a cell: 84 us a window with the light
+// lists, 61 without; 1200x1100, 0.7: 80, 75; 1024^2 with a million, 512 a tile,
+// 68.3 with them, 68.8 without).
+int32_t heavy_first_launch(const swe_ctx* c, int64_t particles) {
+  if (c->heavy_first >= 0) return c->heavy_first;
+  if (c->ntiles <= resident_tiles(c, fused_colour(c, particles))) return 0;
+  return particles <= (int64_t)c->ntiles * (swe::kLightMax + swe::kLightMax / 2) ? 1 : heavy_first_mode(c);
 }
 
 // light-tile slots of a launch: half the tiles, a multiple of 8
@@ -582,7 +596,7 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   // listed crowded tiles get the first workgroups of a launch; at most one
   // slot per 8 tiles, a multiple of 8 (none on maps under 64 tiles)
   const bool fused = fused_colour(c, total), colour = colour_mode(c->p) && !fused;
-  const int32_t hf = c->ntiles <= resident_tiles(c, fused) && c->heavy_first < 0 ? 0 : heavy_first_mode(c);
+  const int32_t hf = heavy_first_launch(c, total);
   sa.heavy_slots = hf ? (int32_t)std::min<int64_t>(swe::kHeavySlotsMax, (c->ntiles / 8) & ~7LL) : 0;
   // light tiles last (heavy-first mode 2, maps of 64 tiles or more): the
   // usual order is padded to a multiple of 8 so that slot b runs on XCD b % 8
