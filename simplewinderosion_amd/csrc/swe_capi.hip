@@ -1240,8 +1240,13 @@ int swe_autotune(swe_ctx* c, const int64_t* particles, int32_t trial_cycles, swe
     }
   }
   if (r == 0 && he == hipSuccess) r = swe_set_tune(c, SWE_TUNE_SHAPE, best_shape);
-  const int32_t heavy0 = heavy_first_mode(c);
-  int32_t best_order = 0, best_graph = 1, best_heavy = -1;
+  // the mode that trial ran, so that a setting kept from it is this one
+  // wherever it is read back and set again
+  int64_t total = 0;
+  for (int32_t k = 0; k < c->nterr; k++) total += particles[k];
+  c->heavy_first = -1;
+  const int32_t heavy0 = heavy_first_launch(c, total);
+  int32_t best_order = 0, best_graph = 1, best_heavy = heavy0;
   // heavy-first only changes anything where a launch has heavy slots
   const int32_t heavy_lo = c->ntiles / 8 >= 8 ? 0 : heavy0, heavy_hi = c->ntiles / 8 >= 8 ? 2 : heavy0;
   for (int32_t hv = heavy_hi; hv >= heavy_lo && r == 0 && he == hipSuccess; hv--)
