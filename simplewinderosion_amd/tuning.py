@@ -16,6 +16,9 @@ import os
 
 from . import capi
 
+# above this settling the automatic cascade order is the colour-ordered one
+MAX_SYNC_SETTLING = 0.25
+
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "simplewinderosion_amd", "tuning.json")
 
 
@@ -28,11 +31,14 @@ def device_arch(target):
 def _key(target, particles):
     p = target.params()
     sizes = getattr(target, "sizes", None) or [(target.nx, target.ny)]
-    return json.dumps({
+    key = {
         "arch": device_arch(target), "sizes": [list(s) for s in sizes], "particles": [int(n) for n in particles],
         "window": int(p.window), "layers": int(p.layers), "track": int(p.track), "periodic": int(p.periodic),
         "deposit": int(p.deposit_on_death), "max_age": int(p.max_age),
-    }, sort_keys=True)
+    }
+    if p.cascade_order == 1 or (p.cascade_order < 0 and p.settling > MAX_SYNC_SETTLING):
+        key["cascade"] = 1  # the colour-ordered cascade: another kernel, with other LDS
+    return json.dumps(key, sort_keys=True)
 
 
 def _load(path):
