@@ -535,9 +535,9 @@ int erode_global(swe_ctx* c, int64_t particles, int32_t n_cycles, int64_t nwin, 
   return 0;
 }
 
-// terrain records for the device: seed / pspeed from the params unless a
-// terrain overrides them
-int push_terrains(swe_ctx* c, const int64_t* particles, swe::Terrain* first) {
+// terrain records for the device (and a single map's among the arguments):
+// seed / pspeed from the params unless a terrain overrides them
+int push_terrains(swe_ctx* c, const int64_t* particles, swe::StepArgs* sa) {
   std::vector<swe::Terrain> t((size_t)c->nterr);
   int64_t part0 = 0;
   for (int32_t k = 0; k < c->nterr; k++) {
@@ -559,7 +559,8 @@ int push_terrains(swe_ctx* c, const int64_t* particles, swe::Terrain* first) {
     normalize3(ps, T.nps);
   }
   HIPCHK(c, hipMemcpyAsync(c->dterr, t.data(), sizeof(swe::Terrain) * t.size(), hipMemcpyHostToDevice, c->stream));
-  *first = t[0];
+  sa->one_terrain = c->nterr == 1 && !c->tseed_set[0] && !c->tps_set[0];
+  if (sa->one_terrain) sa->t0 = t[0];
   return 0;
 }
 
@@ -573,7 +574,7 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   for (int32_t k = 0; k < c->nterr; k++) total += particles[k];
   if ((r = ensure_step(c, total > 0 ? total : 1))) return r;
   swe::StepArgs sa{};
-  if ((r = push_terrains(c, particles, &sa.t0))) return r;
+  if ((r = push_terrains(c, particles, &sa))) return r;
   const bool layers2 = c->p.layers == 2;
   sa.trk = c->trk;
   sa.lost = c->lost;
@@ -581,7 +582,6 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
   sa.cycle = c->dcycle;
   sa.terr = c->dterr;
   sa.tile_terrain = c->dtile_terrain;
-  sa.nterr = c->nterr;
   sa.ncell = c->ncell;
   sa.ntiles = c->ntiles;
   sa.mapscale = c->p.mapscale;
@@ -739,7 +739,8 @@ int erode_tiled(swe_ctx* c, const int64_t* particles, int32_t n_cycles, int64_t 
     key.append((const char*)&c->shape, sizeof(c->shape));
     key.append((const char*)&nwin, sizeof(nwin));
     key.append((const char*)&c->alloc_gen, sizeof(c->alloc_gen));
-    key.append((const char*)&sa.t0, sizeof(sa.t0));  // a single map's terrain is a kernel argument
+    // (t0, when it is an argument, follows from these)
+    key.append((const char*)&sa.one_terrain, sizeof(sa.one_terrain));
   }
   const uint64_t windows_per_cycle = total > 0 ? (uint64_t)nwin + (colour ? 0 : 1) : 0;
 

@@ -160,8 +160,11 @@ struct StepArgs {
   const uint64_t* cycle;
   const Terrain* terr;
   const int32_t* tile_terrain;  // per global tile
-  int32_t nterr;                // 1: every tile is terrain t0 (no lookups)
-  Terrain t0;                   // a single map's terrain
+  // 1: every tile is terrain t0 (no lookups).  A single map with the context's
+  // seed and wind only: a captured cycle holds its arguments, and a terrain
+  // with its own may change them from call to call.
+  int32_t one_terrain;
+  Terrain t0;
   int64_t ncell;                // cells of all terrains (track plane stride)
   int32_t ntiles;
   float mapscale, boundarylayer, suspension, gravity, abrasion, maxdiff, settling;

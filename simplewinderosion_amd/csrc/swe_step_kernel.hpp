@@ -194,9 +194,9 @@ __device__ __forceinline__ void step_body() {
   // before it loads anything
   if ((hs | ls) > 0 && !listed && ap->hstamp[u] > (uint32_t)ap->window) return;
   // the terrain this tile belongs to; all map indices below are terrain-local
-  // (a single map's record is among the arguments: no dependent load)
+  // (a single map's record is among the arguments: no dependent load there)
   TerrainPtr tp = &ap->t0;
-  if (ap->nterr != 1) tp = (TerrainPtr)(uintptr_t)(ap->terr + ap->tile_terrain[u]);
+  if (!ap->one_terrain) tp = (TerrainPtr)(uintptr_t)(ap->terr + ap->tile_terrain[u]);
   const int32_t nx = tp->nx, ny = tp->ny;
   const int32_t tiles_x = tp->tiles_x, tiles_y = tp->tiles_y;
   const int32_t t0 = tp->tile0;
