@@ -842,6 +842,361 @@ __global__ __launch_bounds__(256) void k_wgrad_sum(const float* __restrict__ par
 }
 
 // ---------------------------------------------------------------------------
+// Weight and bias gradients of small layers.  k_wgrad's fixed costs (three X
+// rows before the first product, the waves' sums through LDS, partials of whole
+// 32 x 32 blocks) are most of its time there: 10.8 us for 32 -> 32 at 64^2,
+// batch 1, where k_wgrad_rows takes 9.3, and 12.5 for 192 -> 256 at 4^2, batch
+// 8, where k_wgrad_flat takes 11.1 (wgrad_plan chooses).
+//
+// k_wgrad_flat: a workgroup (4 waves) owns a 64 (co) x 64 (ci) block of one
+// tap and a chunk of the flattened batch's pixels; per step of 32 pixels every
+// thread loads one 16-byte run of dY (8 channels of a pixel) and one of the
+// tap-shifted X, and stores them channel-major into LDS (double buffered: the
+// next step's runs are loaded while the waves run the current MFMAs); each wave
+// accumulates a 32 x 32 sub-block.  The workgroups of tap 4 (no shift) and the
+// first ci block also sum their dY runs for the bias.  Each chunk writes its
+// partial block to `part` ([chunk][Cout * 9 * Cin + Cout]); k_reduce_parts adds
+// the chunks in a fixed order, so the result is deterministic.  Maps of a few
+// pixels waste no lanes on rows shorter than a strip.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_wgrad_flat(const bf16* __restrict__ x, const bf16* __restrict__ dy,
+                                                    float* __restrict__ part, int32_t N, int32_t H, int32_t W,
+                                                    int32_t Cin, int32_t Cout, int32_t chunk) {
+  constexpr int LD = 40;
+  __shared__ __attribute__((aligned(16))) bf16 s_dy[2][64 * LD];  // [co][pixel]
+  __shared__ __attribute__((aligned(16))) bf16 s_x[2][64 * LD];   // [ci][pixel]
+  __shared__ float s_b[32][65];                                    // bias partials [pixel lane][co]
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t cit = (Cin + 63) / 64;
+  int32_t bq = blockIdx.y;
+  const int32_t t = bq % 9;
+  bq /= 9;
+  const int32_t ciB = (bq % cit) * 64, coB = (bq / cit) * 64;
+  const bool do_bias = t == 4 && ciB == 0;
+  const int64_t npix = (int64_t)N * H * W;
+  const int64_t p0 = (int64_t)blockIdx.x * chunk;
+  const int64_t pend = p0 + chunk < npix ? p0 + chunk : npix;
+  const int32_t dyo = t / 3 - 1, dxo = t % 3 - 1;
+  // loader: pixel q of the step, channel group gg (8 channels)
+  const int32_t q = tid >> 3, gg = tid & 7;
+  const int32_t co_ld = coB + 8 * gg, ci_ld = ciB + 8 * gg;
+  const bool co_ok = co_ld < Cout, ci_ok = ci_ld < Cin;
+  const bf16x8 zero = {};
+  bf16x8 rdy, rx;
+  float bsum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  auto load = [&](int64_t q0) __attribute__((always_inline)) {
+    const int64_t p = q0 + q;
+    rdy = zero;
+    rx = zero;
+    if (p < pend) {
+      if (co_ok) rdy = *(const bf16x8*)(dy + p * Cout + co_ld);
+      if (ci_ok) {
+        const int32_t xx = (int32_t)(p % W);
+        const int64_t r = p / W;
+        const int32_t yy = (int32_t)(r % H);
+        const int64_t im = r / H;
+        const int32_t sy = wrapi(yy + dyo, H), sx = wrapi(xx + dxo, W);
+        rx = *(const bf16x8*)(x + ((im * H + sy) * W + sx) * Cin + ci_ld);
+      }
+    }
+  };
+  auto store = [&](int32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      s_dy[buf][(8 * gg + e) * LD + q] = rdy[e];
+      s_x[buf][(8 * gg + e) * LD + q] = rx[e];
+    }
+    if (do_bias) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) bsum[e] += bf2f(rdy[e]);
+    }
+  };
+  // consumer: wave (wave / 2, wave % 2) owns co rows 32 * (wave / 2) .., ci 32 * (wave % 2) ..
+  const int32_t wr = 32 * (wave >> 1), wc = 32 * (wave & 1);
+  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+  load(p0);
+  store(0);
+  __syncthreads();
+  int32_t buf = 0;
+  for (int64_t q0 = p0; q0 < pend; q0 += 32) {
+    const bool more = q0 + 32 < pend;
+    if (more) load(q0 + 32);
+    bf16x8 a[2], b[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) a[i] = *(const bf16x8*)&s_dy[buf][(wr + 16 * i + rl) * LD + kq];
+#pragma unroll
+    for (int j = 0; j < 2; j++) b[j] = *(const bf16x8*)&s_x[buf][(wc + 16 * j + rl) * LD + kq];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    if (more) store(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+  const int64_t nw = (int64_t)Cout * 9 * Cin;
+  float* out = part + (int64_t)blockIdx.x * (nw + Cout);
+  // D rows (co) = wr + 16 i + 4 (lane / 16) + e, column (ci) = wc + 16 j + lane % 16
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int32_t ci = ciB + wc + 16 * j + rl;
+    if (ci >= Cin) continue;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int32_t co = coB + wr + 16 * i + 4 * (lane >> 4) + e;
+        if (co < Cout) out[((int64_t)co * 9 + t) * Cin + ci] = acc[i][j][e];
+      }
+  }
+  if (do_bias) {  // the 32 pixel lanes' sums per channel, added in a fixed order
+#pragma unroll
+    for (int e = 0; e < 8; e++) s_b[q][8 * gg + e] = bsum[e];
+    __syncthreads();
+    if (tid < 64) {
+      float sb = 0.0f;
+      for (int k = 0; k < 32; k++) sb += s_b[k][tid];
+      if (coB + tid < Cout) out[nw + coB + tid] = sb;
+    }
+  }
+}
+
+// k_wgrad_rows (W % 32 == 0): a workgroup owns a 32 (co) x 32 (ci) block of all
+// nine taps and walks R rows of one 32-pixel column strip of one image.  Per
+// row y it loads the dY row (32 pixels x CB) and the X row y + 1 (34 pixels,
+// x0 - 1 .. x0 + 32, periodic); X rows y - 1, y, y + 1 stay in a four-row LDS
+// ring.  LDS rows are channel-major (pixels contiguous, the MFMA's k), 40
+// elements a row, with the 8-pixel blocks of columns 0..31 permuted per row
+// (block ^ (row / 8) % 4) so that the transposing two-byte stores of eight
+// channel rows fall in different banks.  The tap shift dx = -1, 0, +1 is a B
+// operand read at column offset 0, 1, 2: one aligned 16-byte read plus the next
+// dword, shifted by one element with v_alignbit for the odd offset.  Waves tile
+// the block 2 x 2; the workgroups of the first ci block also sum the dY rows
+// for the bias.  Partials as k_wgrad_flat's: of the layer's channels, not of
+// whole blocks.
+__device__ __forceinline__ int32_t wg_col(int32_t row, int32_t c) { return c < 32 ? c ^ (8 * ((row >> 3) & 3)) : c; }
+
+__global__ __launch_bounds__(256) void k_wgrad_rows(const bf16* __restrict__ x, const bf16* __restrict__ dy,
+                                                    float* __restrict__ part, int32_t N, int32_t H, int32_t W,
+                                                    int32_t Cin, int32_t Cout, int32_t R) {
+  constexpr int CB = 32, IB = 32;  // channels of a block
+  constexpr int LD = 40;
+  constexpr int TI = CB / 32, TJ = IB / 32;  // 16 x 16 tiles per wave along co and ci
+  constexpr int DG = CB / 8, XG = IB / 8;    // 16-byte channel groups of a pixel
+  constexpr int XITEMS = 34 * XG;            // X row loads (pixel, group)
+  __shared__ __attribute__((aligned(16))) bf16 s_x[4][IB * LD];
+  __shared__ __attribute__((aligned(16))) bf16 s_dy[2][CB * LD];
+  __shared__ float s_b[32][CB + 1];
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t segs = W / 32, cps = (H + R - 1) / R;
+  const int32_t chunk = blockIdx.x;
+  const int32_t rc = chunk % cps, sg = (chunk / cps) % segs, n = chunk / (cps * segs);
+  const int32_t nci = (Cin + IB - 1) / IB;
+  const int32_t ciB = (int32_t)(blockIdx.y % nci) * IB, coB = (int32_t)(blockIdx.y / nci) * CB;
+  const int32_t y0 = rc * R, rows = R < H - y0 ? R : H - y0, x0 = sg * 32;
+  const bool do_bias = ciB == 0;
+  const bf16x8 zero = {};
+
+  // dY loads: thread -> (pixel dpx, group dg), groups fastest (coalesced)
+  const bool dy_item = tid < 32 * DG;
+  const int32_t dpx = tid / DG, dg = tid % DG;
+  const bool dy_ok = dy_item && coB + 8 * dg < Cout;
+  const int64_t dy_col = (int64_t)(x0 + dpx) * Cout + coB + 8 * dg;
+  // X loads: items tid and tid + 256 -> (column c, group g)
+  int32_t xc[2], xg[2];
+  bool xok[2], xitem[2];
+  int64_t xcol[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int32_t u = tid + 256 * h;
+    xitem[h] = u < XITEMS;
+    xc[h] = u / XG;
+    xg[h] = u % XG;
+    xok[h] = xitem[h] && ciB + 8 * xg[h] < Cin;
+    xcol[h] = (int64_t)wrapi(x0 + xc[h] - 1, W) * Cin + ciB + 8 * xg[h];
+  }
+  const int64_t img = (int64_t)n * H;
+
+  struct Regs {
+    bf16x8 d, xa, xb;
+  };
+  // the loads of X row k (image row y0 - 1 + k) and dY row y
+  auto load = [&](int32_t k, int32_t y, bool with_dy) __attribute__((always_inline)) {
+    Regs r;
+    const int64_t xrow = (img + wrapi(y0 - 1 + k, H)) * W * Cin;
+    r.xa = xok[0] ? *(const bf16x8*)(x + xrow + xcol[0]) : zero;
+    r.xb = xok[1] ? *(const bf16x8*)(x + xrow + xcol[1]) : zero;
+    r.d = (with_dy && dy_ok) ? *(const bf16x8*)(dy + (img + y) * W * Cout + dy_col) : zero;
+    return r;
+  };
+  float bsum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  auto store_x = [&](const Regs& r, int32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      if (!xitem[h]) continue;
+      const bf16x8 v = h == 0 ? r.xa : r.xb;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int32_t row = 8 * xg[h] + e;
+        s_x[slot][row * LD + wg_col(row, xc[h])] = v[e];
+      }
+    }
+  };
+  auto store_dy = [&](const Regs& r, int32_t slot) __attribute__((always_inline)) {
+    if (!dy_item) return;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const int32_t row = 8 * dg + e;
+      s_dy[slot][row * LD + wg_col(row, dpx)] = r.d[e];
+    }
+    if (do_bias) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) bsum[e] += bf2f(r.d[e]);
+    }
+  };
+
+  const int32_t wr = (CB / 2) * (wave >> 1), wc = (IB / 2) * (wave & 1);
+  const int32_t kq = 8 * (lane >> 4), rl = lane & 15;
+  f32x4 acc[9][TI][TJ];
+#pragma unroll
+  for (int t = 0; t < 9; t++)
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+      for (int j = 0; j < TJ; j++) acc[t][i][j] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+
+  // prologue: X rows y0 - 1, y0, y0 + 1 and dY row y0, all loads in flight together
+  {
+    const Regs r0 = load(0, y0, true), r1 = load(1, y0, false), r2 = load(2, y0, false);
+    store_x(r0, 0);
+    store_x(r1, 1);
+    store_x(r2, 2);
+    store_dy(r0, 0);
+  }
+  __syncthreads();
+  for (int32_t s = 0; s < rows; s++) {
+    const bool more = s + 1 < rows;
+    Regs nx;
+    if (more) nx = load(s + 3, y0 + s + 1, true);
+    const int32_t ds = s & 1;
+    bf16x8 a[TI];
+#pragma unroll
+    for (int i = 0; i < TI; i++) {
+      const int32_t row = wr + 16 * i + rl;
+      a[i] = *(const bf16x8*)&s_dy[ds][row * LD + wg_col(row, kq)];
+    }
+#pragma unroll
+    for (int dyi = 0; dyi < 3; dyi++) {
+      const bf16* xr = s_x[(s + dyi) & 3];
+#pragma unroll
+      for (int j = 0; j < TJ; j++) {
+        const int32_t row = wc + 16 * j + rl;
+        const u32x4 v0 = *(const u32x4*)&xr[row * LD + wg_col(row, kq)];
+        const uint32_t v1 = *(const uint32_t*)&xr[row * LD + wg_col(row, kq + 8)];
+        const u32x4 vm = v0;  // columns kq .. kq + 7: pixel x + dx for dx = -1
+        const u32x4 vz = {__builtin_amdgcn_alignbit(v0[1], v0[0], 16), __builtin_amdgcn_alignbit(v0[2], v0[1], 16),
+                          __builtin_amdgcn_alignbit(v0[3], v0[2], 16), __builtin_amdgcn_alignbit(v1, v0[3], 16)};
+        const u32x4 vp = {v0[1], v0[2], v0[3], v1};
+        const bf16x8 bm = __builtin_bit_cast(bf16x8, vm), bz = __builtin_bit_cast(bf16x8, vz),
+                     bp = __builtin_bit_cast(bf16x8, vp);
+#pragma unroll
+        for (int i = 0; i < TI; i++) {
+          acc[3 * dyi + 0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bm, acc[3 * dyi + 0][i][j], 0, 0, 0);
+          acc[3 * dyi + 1][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bz, acc[3 * dyi + 1][i][j], 0, 0, 0);
+          acc[3 * dyi + 2][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bp, acc[3 * dyi + 2][i][j], 0, 0, 0);
+        }
+      }
+    }
+    if (more) {
+      store_x(nx, (s + 3) & 3);
+      store_dy(nx, ds ^ 1);
+    }
+    __syncthreads();
+  }
+
+  const int64_t nw = (int64_t)Cout * 9 * Cin;
+  float* out = part + (int64_t)chunk * (nw + Cout);
+  // D rows (co) = wr + 16 i + 4 (lane / 16) + e, column (ci) = wc + 16 j + lane % 16
+#pragma unroll
+  for (int j = 0; j < TJ; j++) {
+    const int32_t ci = ciB + wc + 16 * j + rl;
+    if (ci >= Cin) continue;
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int32_t co = coB + wr + 16 * i + 4 * (lane >> 4) + e;
+        if (co >= Cout) continue;
+#pragma unroll
+        for (int t = 0; t < 9; t++) out[((int64_t)co * 9 + t) * Cin + ci] = acc[t][i][j][e];
+      }
+  }
+  if (do_bias) {  // the 32 pixel columns' sums per channel, added in a fixed order
+    if (dy_item) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) s_b[dpx][8 * dg + e] = bsum[e];
+    }
+    __syncthreads();
+    if (tid < CB) {
+      float sb = 0.0f;
+      for (int k = 0; k < 32; k++) sb += s_b[k][tid];
+      if (coB + tid < Cout) out[nw + coB + tid] = sb;
+    }
+  }
+}
+
+// dw[i] (i < nw) and db[i - nw] (nw <= i < nw + Cout, when db is given):
+// the chunks' partials added in a fixed order.  A workgroup takes 64
+// consecutive entries; its 16 groups of 16 threads read them as float4 runs
+// from every 16th chunk (group g: chunks g, g + 16, ...), and the groups'
+// sums are added in group order.  Rows are nw + Cout floats, a multiple of
+// 8 (Cin % 8 == Cout % 8 == 0), so the runs are aligned.
+__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, float* __restrict__ dw,
+                                                      float* __restrict__ db, int64_t nw, int32_t Cout,
+                                                      int32_t nparts) {
+  __shared__ float s_sum[16][65];
+  const int32_t tid = threadIdx.x, c4 = tid & 15, g = tid >> 4;
+  const int64_t stride = nw + Cout;
+  const int64_t n = db ? stride : nw;
+  const int64_t i0 = (int64_t)blockIdx.x * 64 + 4 * c4;
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (i0 < n) {
+    const float* p = part + i0;
+    int32_t k = g;
+    // four chunks' loads in flight per step; the adds stay in chunk order
+    for (; k + 48 < nparts; k += 64) {
+      const f32x4 v0 = *(const f32x4*)(p + (int64_t)k * stride);
+      const f32x4 v1 = *(const f32x4*)(p + (int64_t)(k + 16) * stride);
+      const f32x4 v2 = *(const f32x4*)(p + (int64_t)(k + 32) * stride);
+      const f32x4 v3 = *(const f32x4*)(p + (int64_t)(k + 48) * stride);
+      acc += v0;
+      acc += v1;
+      acc += v2;
+      acc += v3;
+    }
+    for (; k < nparts; k += 16) acc += *(const f32x4*)(p + (int64_t)k * stride);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) s_sum[g][4 * c4 + e] = acc[e];
+  __syncthreads();
+  if (tid < 64) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + tid;
+    if (i < n) {
+      float s = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 16; q++) s += s_sum[q][tid];
+      if (i < nw) dw[i] = s;
+      else db[i - nw] = s;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Elementwise, pooling, resampling
 // ---------------------------------------------------------------------------
 // g16 = bf16(g32 * (y > 0)) (ReLU gradient through the layer output), or
@@ -1415,11 +1770,57 @@ int swe_nn_flip(const void* w, int32_t Cin, int32_t Cout, void* wt, void* stream
 // 14.2 / 15.0 / 15.2.  Chunks of at most eight rows in all become one, whose
 // workgroups write the result: 256 -> 192 at 4^2, batch 2, 12.7 -> 9.5; to
 // sixteen rows it loses (192 -> 256 at 8^2, batch 8, 14.6 -> 19.0).
+//
+// Small layers take the kernels above where those are estimated faster: times
+// in us, fitted to 1,341 measured layers (two launches of a graph each; mean
+// error 2% for k_wgrad and k_wgrad_rows, 5% for k_wgrad_flat), and only up to
+// 13.5 (k_wgrad_flat 15), past which k_wgrad's rate decides.  Measured (small kernel / k_wgrad):
+// 8 -> 32 at 128^2, batch 1, 9.5 / 12.1; 64 -> 32 there 11.5 / 12.6; 32 -> 32 at
+// 256^2 14.2 / 13.7; 32 -> 64 at 4^2, batch 8, 8.6 / 12.1; 256 -> 256 at 4^2,
+// batch 4, 10.2 / 9.4; 128 -> 192 at 8^2, batch 4, 13.3 / 12.4.
 constexpr int32_t kWgradMinRows = 6, kWgradOneChunk = 8;
+constexpr double kWgradSmallRows = 13.5, kWgradSmallFlat = 15.0;
+enum WgradKind { kWgradStrips, kWgradRows, kWgradFlat };
 struct WgradPlan {
+  WgradKind kind;
   int32_t R;
   int64_t blocks, units, per, chunks;
+  int64_t chunk;  // k_wgrad_flat: pixels
+  int64_t work;   // floats of partials
 };
+
+// whole 32-pixel strips, R rows a workgroup (at least eight), ~1024 workgroups
+static WgradPlan wgrad_rows_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout, double* us) {
+  WgradPlan p{};
+  p.kind = kWgradRows;
+  p.blocks = (int64_t)((Cout + 31) / 32) * ((Cin + 31) / 32);
+  const int64_t strips = (int64_t)N * (W / 32), cmax = (H + 7) / 8;
+  int64_t cps = (1024 + strips * p.blocks - 1) / (strips * p.blocks);
+  if (cps > cmax) cps = cmax;
+  p.R = (int32_t)((H + cps - 1) / cps);
+  p.chunks = strips * ((H + p.R - 1) / p.R);
+  const double part = (double)Cout * (9.0 * Cin + 1.0) * 1e-6;  // partials of a chunk, millions
+  p.work = p.chunks * ((int64_t)Cout * 9 * Cin + Cout);
+  *us = 5.07 + 0.483 * p.R + 0.00397 * (double)(p.chunks * p.blocks) + 1.8 * (double)p.chunks * part +
+        0.004 * (double)p.chunks;
+  return p;
+}
+
+// flattened pixels, a multiple of 32 and at least 256 a workgroup, ~1024 workgroups
+static WgradPlan wgrad_flat_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout, double* us) {
+  WgradPlan p{};
+  p.kind = kWgradFlat;
+  p.blocks = (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64);
+  const int64_t npix = (int64_t)N * H * W;
+  p.chunk = ((npix * p.blocks + 1023) / 1024 + 31) / 32 * 32;
+  if (p.chunk < 256) p.chunk = 256;
+  p.chunks = (npix + p.chunk - 1) / p.chunk;
+  const double part = (double)Cout * (9.0 * Cin + 1.0) * 1e-6, px = (double)(npix < p.chunk ? npix : p.chunk);
+  p.work = p.chunks * ((int64_t)Cout * 9 * Cin + Cout);
+  *us = 4.76 + 0.031 * px + (1.78 - 0.0028 * px) * part + 0.01315 * (double)(p.chunks * p.blocks) +
+        1.17 * (double)p.chunks * part - (p.chunks > 1 ? 1.68 : 0.0);
+  return p;
+}
 
 static WgradPlan wgrad_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   WgradPlan p{};
@@ -1438,28 +1839,47 @@ static WgradPlan wgrad_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_
     p.per *= p.chunks;
     p.chunks = 1;
   }
-  return p;
+  p.work = p.chunks * p.blocks * kWgradPart;
+  const double us = 5.90 + 0.432 * (double)p.R * (double)p.per + 1.04 * (double)(p.per - 1) +
+                    (p.chunks > 1 ? 1.21 : 0.0) + 0.024 * (double)(p.chunks * p.blocks) - 0.0161 * (double)p.blocks +
+                    0.30 * (double)(p.units < 4 ? p.units : 4);
+  double small = 0.0;
+  const WgradPlan q = W % 32 == 0 ? wgrad_rows_plan(N, H, W, Cin, Cout, &small) : wgrad_flat_plan(N, H, W, Cin, Cout, &small);
+  return small < us && small < (W % 32 == 0 ? kWgradSmallRows : kWgradSmallFlat) ? q : p;
 }
 
 int64_t swe_nn_wgrad_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   if (N < 1 || H < 1 || W < 1 || Cin < 1 || Cout < 1) return 0;
-  const WgradPlan p = wgrad_plan(N, H, W, Cin, Cout);
-  return p.chunks * p.blocks * kWgradPart;
+  return wgrad_plan(N, H, W, Cin, Cout).work;
 }
 int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout,
                  float* dw, float* db, float* work, int64_t work_len, void* stream) {
   if (!x || !dy || !dw || !work || (uintptr_t)work % 16) return -1;
   if (N < 1 || H < 1 || W < 1 || Cin < 8 || Cout < 8 || Cin % 8 || Cout % 8) return -1;
-  if (work_len < swe_nn_wgrad_work(N, H, W, Cin, Cout)) return -1;
   const WgradPlan p = wgrad_plan(N, H, W, Cin, Cout);
-  // what a grid's second axis once held: 64 x 64 blocks of one tap where a row
-  // is not whole strips
+  if (work_len < p.work) return -1;
+  // what a grid's second axis holds of the small layers' kernels, and held of
+  // every layer: 32 x 32 blocks, or 64 x 64 of one tap where a row is not whole
+  // strips
+  const int64_t blocks = (int64_t)((Cout + 31) / 32) * ((Cin + 31) / 32);
   const int64_t tall = W % 32 ? (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64) : 0;
-  if (p.blocks > 65535 || tall > 65535 || p.chunks * p.blocks > 0x7fffffffLL) return -1;
-  if (p.units + 4 * p.per > 0xffffffffLL || (int64_t)W * (Cin > Cout ? Cin : Cout) * 2 >= 0xffffffffLL) return -1;
-  const dim3 grid((unsigned)(p.chunks * p.blocks));
+  if (blocks > 65535 || tall > 65535 || p.chunks * p.blocks > 0x7fffffffLL) return -1;
   const bf16* xx = (const bf16*)x;
   const bf16* dd = (const bf16*)dy;
+  if (p.kind != kWgradStrips) {
+    const dim3 grid((unsigned)p.chunks, (unsigned)p.blocks);
+    if (p.kind == kWgradRows)
+      hipLaunchKernelGGL(k_wgrad_rows, grid, dim3(256), 0, S(stream), xx, dd, work, N, H, W, Cin, Cout, p.R);
+    else
+      hipLaunchKernelGGL(k_wgrad_flat, grid, dim3(256), 0, S(stream), xx, dd, work, N, H, W, Cin, Cout,
+                         (int32_t)p.chunk);
+    const int64_t nw = (int64_t)Cout * 9 * Cin, nred = db ? nw + Cout : nw;
+    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((nred + 63) / 64)), dim3(256), 0, S(stream), work, dw, db, nw,
+                       Cout, (int32_t)p.chunks);
+    SWENN_LAUNCH_CHECK();
+  }
+  if (p.units + 4 * p.per > 0xffffffffLL || (int64_t)W * (Cin > Cout ? Cin : Cout) * 2 >= 0xffffffffLL) return -1;
+  const dim3 grid((unsigned)(p.chunks * p.blocks));
   float* dw1 = p.chunks == 1 ? dw : nullptr;
   if (W % 32)
     hipLaunchKernelGGL(k_wgrad<true>, grid, dim3(256), kWgradLds, S(stream), xx, dd, work, dw1, db, H, W, Cin, Cout,
