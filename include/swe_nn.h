@@ -44,8 +44,7 @@ int swe_nn_flip(const void* w, int32_t Cin, int32_t Cout, void* wt, void* stream
 int64_t swe_nn_wgrad_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout);
 /* dw = sum_p dy[p] x[p + t]^T (float [Cout][9][Cin]); db = sum_p dy[p]
  * (float [Cout], optional); Cin % 8 == Cout % 8 == 0; deterministic
- * (per-chunk partials in `work`, 16-byte aligned, added in a fixed order).
- * Rows (W channels) of less than 4 GB. */
+ * (per-chunk partials in `work`, 16-byte aligned, added in a fixed order). */
 int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout,
                  float* dw, float* db, float* work, int64_t work_len, void* stream);
 /* g16 = bf16(g32 * (y > 0)); y may be NULL (conversion only) */

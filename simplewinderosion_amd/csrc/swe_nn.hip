@@ -1845,7 +1845,9 @@ static WgradPlan wgrad_plan(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_
                     0.30 * (double)(p.units < 4 ? p.units : 4);
   double small = 0.0;
   const WgradPlan q = W % 32 == 0 ? wgrad_rows_plan(N, H, W, Cin, Cout, &small) : wgrad_flat_plan(N, H, W, Cin, Cout, &small);
-  return small < us && small < (W % 32 == 0 ? kWgradSmallRows : kWgradSmallFlat) ? q : p;
+  // (k_wgrad counts units and addresses a row in 32 bits)
+  const bool wide = p.units + 4 * p.per > 0xffffffffLL || (int64_t)W * (Cin > Cout ? Cin : Cout) * 2 >= 0xffffffffLL;
+  return wide || (small < us && small < (W % 32 == 0 ? kWgradSmallRows : kWgradSmallFlat)) ? q : p;
 }
 
 int64_t swe_nn_wgrad_work(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
@@ -1863,7 +1865,8 @@ int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W,
   // strips
   const int64_t blocks = (int64_t)((Cout + 31) / 32) * ((Cin + 31) / 32);
   const int64_t tall = W % 32 ? (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64) : 0;
-  if (blocks > 65535 || tall > 65535 || p.chunks * p.blocks > 0x7fffffffLL) return -1;
+  if (blocks > 65535 || tall > 65535 || p.chunk > 0x7fffffffLL || p.chunks > 0x7fffffffLL / (p.kind == kWgradStrips ? p.blocks : 1))
+    return -1;
   const bf16* xx = (const bf16*)x;
   const bf16* dd = (const bf16*)dy;
   if (p.kind != kWgradStrips) {
@@ -1878,7 +1881,6 @@ int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W,
                        Cout, (int32_t)p.chunks);
     SWENN_LAUNCH_CHECK();
   }
-  if (p.units + 4 * p.per > 0xffffffffLL || (int64_t)W * (Cin > Cout ? Cin : Cout) * 2 >= 0xffffffffLL) return -1;
   const dim3 grid((unsigned)(p.chunks * p.blocks));
   float* dw1 = p.chunks == 1 ? dw : nullptr;
   if (W % 32)
