@@ -1570,6 +1570,11 @@ static inline unsigned G(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 extern "C" {
 
+// Layers of few input channels on maps of whole 32-pixel strips
+static bool conv_rows(int32_t W, int32_t Cin, int32_t Cout, int64_t P) {
+  return W % 32 == 0 && (Cin <= 32 || (Cin <= 64 && (int64_t)Cout * P <= ((int64_t)1 << 23)));
+}
+
 // Slices of a split reduction: layers whose grid of 128-pixel blocks has fewer
 // workgroups than the chip has CUs, ~768 over the slices, >= 8 steps of 32
 // channels each, at most 8.  The tile kernels sum the slices in one workgroup
@@ -1577,7 +1582,7 @@ extern "C" {
 // order of additions.
 static int32_t conv_slices(int32_t N, int32_t H, int32_t W, int32_t Cin, int32_t Cout) {
   const int64_t P = (int64_t)N * H * W;
-  if (W % 32 == 0 && (Cin <= 32 || (Cin <= 64 && (int64_t)Cout * P <= ((int64_t)1 << 23)))) return 1;
+  if (conv_rows(W, Cin, Cout, P)) return 1;
   const int64_t mt = (P + 127) / 128;
   const int32_t nt = Cout <= 16 ? 16 : (Cout <= 32 ? 32 : (Cout <= 64 || mt * ((Cout + 127) / 128) < 512 ? 64 : 128));
   const int64_t wgs = mt * ((Cout + nt - 1) / nt), ksteps = 9 * ((Cin + 31) / 32);
@@ -1671,6 +1676,9 @@ static int conv_launch(const void* x, int32_t N, int32_t H, int32_t W, int32_t C
   const int64_t P = (int64_t)N * H * W;
   // the kernels' buffer loads take 32-bit byte offsets below 2^31
   if (P * Cin * 2 >= ((int64_t)1 << 31) || (int64_t)Cout * 9 * Cin * 2 >= ((int64_t)1 << 31)) return -1;
+  // refused since these layers' 32-channel blocks were a grid's second axis
+  // (the tile kernels have no such limit)
+  if (conv_rows(W, Cin, Cout, P) && (Cout + 31) / 32 > 65535) return -1;
   const bf16* xx = (const bf16*)x;
   const bf16* ww = (const bf16*)w;
   const bf16* mm = (const bf16*)mask;
@@ -1860,9 +1868,8 @@ int swe_nn_wgrad(const void* x, const void* dy, int32_t N, int32_t H, int32_t W,
   if (N < 1 || H < 1 || W < 1 || Cin < 8 || Cout < 8 || Cin % 8 || Cout % 8) return -1;
   const WgradPlan p = wgrad_plan(N, H, W, Cin, Cout);
   if (work_len < p.work) return -1;
-  // what a grid's second axis holds of the small layers' kernels, and held of
-  // every layer: 32 x 32 blocks, or 64 x 64 of one tap where a row is not whole
-  // strips
+  // blocks a grid's second axis holds: 32 x 32, or 64 x 64 of one tap where a
+  // row is not whole strips (k_wgrad has no such limit; refused all the same)
   const int64_t blocks = (int64_t)((Cout + 31) / 32) * ((Cin + 31) / 32);
   const int64_t tall = W % 32 ? (int64_t)((Cout + 63) / 64) * 9 * ((Cin + 63) / 64) : 0;
   if (blocks > 65535 || tall > 65535 || p.chunk > 0x7fffffffLL || p.chunks > 0x7fffffffLL / (p.kind == kWgradStrips ? p.blocks : 1))
