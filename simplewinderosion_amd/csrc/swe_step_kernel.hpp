@@ -383,7 +383,9 @@ __device__ __forceinline__ void step_body() {
     constexpr int kWaves = kStepThreads / 64;
     constexpr int kRows = (kSX + kColourHaloMax.xl + kColourHaloMax.xh + kWaves - 1) / kWaves;
     constexpr int kChunks = (kSY + kColourHaloMax.yl + kColourHaloMax.yh + 63) / 64;
-    constexpr int kB = kRows < 8 ? kRows : 8;  // rows a wave has in flight
+    // rows a wave has in flight (eight overflow the registers of the closing
+    // launch of the largest shape)
+    constexpr int kMost = RELAX_ONLY && kStepThreads > 256 ? 4 : 8, kB = kRows < kMost ? kRows : kMost;
     const int32_t wv = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x >> 6), lane = (int32_t)threadIdx.x & 63;
     uint32_t where[kChunks][kRows];  // class << 16 | rank in the wave's part of it; 0: not listed
     uint32_t wcnt = 0;

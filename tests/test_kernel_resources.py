@@ -73,6 +73,18 @@ def test_step_kernel_budget(metadata, shape):
         assert groups_per_cu * f["group_segment_fixed_size"] <= LDS_PER_CU, (name, f["group_segment_fixed_size"])
 
 
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_colour_kernel_budget(metadata, shape):
+    """Every instance of k_colour_step: no scratch, the VGPRs of four waves per
+    SIMD."""
+    colour = {k: v for k, v in metadata[shape].items() if "k_colour_step" in k}
+    assert len(colour) == 32  # periodic x track x layers x deposit x mode (step + relax, relax only)
+    for name, f in colour.items():
+        assert f["private_segment_fixed_size"] == 0, (name, f["private_segment_fixed_size"])
+        assert f.get("vgpr_spill_count", 0) == 0, name
+        assert f["vgpr_count"] <= 128, (name, f["vgpr_count"])
+
+
 def test_colour_residency(metadata, tmp_path):
     """The workgroups that colour_resident (csrc/swe_step.h) says the chip
     holds of k_colour_step: what the compiled kernels' static LDS and registers
