@@ -363,11 +363,16 @@ int swe_normals_noalloc(swe_ctx* ctx, float* out);
  * nb_cell[8] their cells in the reference's offset order (world.hpp:83-92)
  * and nb_fx[8] the fixed-point amount each receives (the centre loses the
  * sum).
+ *
+ * swe_debug_root: the kernels' square root s of d and reciprocal of s against
+ * the device's IEEE operations, for the `count` floats whose bits follow
+ * `first`: how many differ, and the bits of the first of them (all ones: none).
  */
 int swe_debug_step(swe_ctx* ctx, int32_t n, float* state, int32_t* age, const uint64_t* key, int32_t* alive,
                    int64_t* pickup);
 int swe_debug_cascade(swe_ctx* ctx, int32_t x, int32_t y, uint32_t events, int32_t* count, int64_t* nb_cell,
                       int64_t* nb_fx);
+int swe_debug_root(swe_ctx* ctx, uint32_t first, int64_t count, uint64_t* mismatches, uint32_t* first_bad);
 
 /*
  * The particles' RNG seed (World::SEED, SimpleWindErosion.cpp:27-34, which

@@ -156,6 +156,8 @@ SIGNATURES = {
                                       ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_int32), _I64P]),
     "swe_debug_cascade": (ctypes.c_int, [_P, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint32,
                                          ctypes.POINTER(ctypes.c_int32), _I64P, _I64P]),
+    "swe_debug_root": (ctypes.c_int, [_P, ctypes.c_uint32, ctypes.c_int64, ctypes.POINTER(ctypes.c_uint64),
+                                      ctypes.POINTER(ctypes.c_uint32)]),
     "swe_set_rng": (ctypes.c_int, [_P, ctypes.c_uint64]),
     "swe_windmap": (ctypes.c_int, [_P, _FP]),
     "swe_mesh": (ctypes.c_int, [_P, _FP]),

@@ -1641,6 +1641,26 @@ int swe_debug_cascade(swe_ctx* c, int32_t x, int32_t y, uint32_t events, int32_t
   return 0;
 }
 
+int swe_debug_root(swe_ctx* c, uint32_t first, int64_t count, uint64_t* mismatches, uint32_t* first_bad) {
+  if (!c || !mismatches || !first_bad) return SWE_EINVAL;
+  if (count < 0 || count > ((int64_t)1 << 32)) return fail(c, SWE_EINVAL, "swe_debug_root: count out of range");
+  HIPCHK(c, hipSetDevice(c->device));
+  DevScratch buf;
+  if (hipMalloc(&buf.p, sizeof(uint64_t) * 2) != hipSuccess) {
+    buf.p = nullptr;
+    return fail(c, SWE_ENOMEM, "swe_debug_root: hipMalloc failed");
+  }
+  uint64_t h[2] = {0, 0xffffffffu};
+  HIPCHK(c, hipMemcpyAsync(buf.p, h, sizeof(h), hipMemcpyHostToDevice, c->stream));
+  swe::launch_debug_root(first, count, (uint64_t*)buf.p, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipMemcpyAsync(h, buf.p, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  *mismatches = h[0];
+  *first_bad = (uint32_t)h[1];
+  return 0;
+}
+
 int swe_set_rng(swe_ctx* c, uint64_t seed) {
   if (!c) return SWE_EINVAL;
   swe_params q = c->p;

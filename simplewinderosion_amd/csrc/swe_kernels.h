@@ -137,5 +137,7 @@ struct DebugCascadeArgs {
   swe_params p;
 };
 void launch_debug_cascade(const DebugCascadeArgs& a, hipStream_t s);
+// out: differing floats, then the lowest bits among them (both set before)
+void launch_debug_root(uint32_t first, int64_t count, uint64_t* out, hipStream_t s);
 
 }  // namespace swe

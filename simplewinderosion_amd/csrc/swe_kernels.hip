@@ -820,6 +820,22 @@ __global__ void k_debug_cascade(DebugCascadeArgs a) {
   *a.count = n;
 }
 
+__global__ void k_debug_root(uint32_t first, int64_t count, uint64_t* out) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256) {
+    const uint32_t u = first + (uint32_t)i;
+    const Root r = root_of(u2f(u));
+    const float s = __builtin_sqrtf(u2f(u)), q = 1.0f / s;
+    const bool same = (f2u(r.s) == f2u(s) || (r.s != r.s && s != s)) && (f2u(r.r) == f2u(q) || (r.r != r.r && q != q));
+    if (same) continue;
+    atomicAdd((unsigned long long*)&out[0], 1ull);
+    atomicMin((unsigned long long*)&out[1], (unsigned long long)u);
+  }
+}
+
+void launch_debug_root(uint32_t first, int64_t count, uint64_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_debug_root, dim3(8192), dim3(256), 0, s, first, count, out);
+}
+
 void launch_debug_fly(const DebugFlyArgs& a, hipStream_t s) {
   if (a.n <= 0) return;
   const dim3 g((unsigned)((a.n + 63) / 64));
