@@ -360,7 +360,7 @@ __device__ __forceinline__ void colour_relax_cell(const RelaxArgs& a, int64_t ba
   // eight accumulators (an indexed register array would live in scratch)
   cascade_cell_dev<LAYERS>(hn, sed_of, hc, sc, valid, settle_factor_dev(a.settling, v), a.maxdiff,
                            [&](int32_t k, int64_t amt) {
-                             if (amt == 0) return;
+                             if (!__any(amt != 0)) return;  // a wave's at a time: no divergence
 #pragma unroll
                              for (int j = 0; j < 8; j++) d[j] += k == j ? amt : 0;
                              centre -= amt;
