@@ -287,9 +287,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_tile_b
 // patch (up to KC = 256 channels; more run as blocks of KC) stays in LDS, and
 // the weights stream through it tap by tap, two taps ahead in registers: so
 // the reduction runs tap by tap and within a tap over the 32-channel chunks,
-// the order of the implicit GEMM's k = tap Cin + channel.  With kz > 1 the
-// k-steps are summed in kz slices [z K / kz, (z + 1) K / kz) whose sums are
-// added in order (a layer given the workspace of a split reduction).
+// the order of the implicit GEMM's k = tap Cin + channel; with several blocks of
+// KC, block by block.  With kz > 1 the k-steps are summed in kz slices
+// [z K / kz, (z + 1) K / kz) whose sums are added in order (a layer given the
+// workspace of a split reduction).
 // LDS rows are KC channels at a stride of KC + 8 elements (16 m + 4 dwords:
 // the 16 rows of a fragment read fall in different banks).
 //
@@ -306,7 +307,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(conv_tile_b
 // earlier 7% longer at 4 x 4.
 // ---------------------------------------------------------------------------
 // 32-channel chunks of a block at most: KC <= 256, for the largest workgroups
-// 192 (their patch of more would not fit the LDS)
+// 192 (their patch of more would not fit the LDS).  Those hold two workgroups a
+// CU at 256 registers, of which about 20 spill (80 to 88 bytes of scratch).
 constexpr int conv_wide_chunks(int pf, int cf) { return pf * cf > 8 ? 6 : 8; }
 
 template <int PF, int CF, int S, int ACT, bool SPLIT>

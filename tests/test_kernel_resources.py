@@ -118,3 +118,18 @@ int main() {
         by_lds = LDS_PER_CU // (-(-(static + lds) // 1280) * 1280)
         by_waves = 4 * min(512 // (-(-regs // 8) * 8), 8) // (threads // 64)
         assert resident == 256 * min(by_lds, by_waves), (i, h, t, layers)
+
+
+def test_network_kernel_scratch(tmp_path):
+    """The surrogate's kernels use no scratch but one shape of the wide
+    convolution: 256 pixels x 64 channels a workgroup keeps two workgroups on a
+    CU at 256 registers with some 20 spilled."""
+    out = str(tmp_path / "nn.s")
+    subprocess.run([B.hipcc()] + B.HIP_FLAGS + ["--cuda-device-only", "-S", "-o", out,
+                                                os.path.join(B.CSRC, B.NN_SOURCES[0])], check=True, capture_output=True)
+    kernels = _kernels(open(out).read())
+    assert sum("k_conv_tile" in k for k in kernels) == 36 and sum("k_conv_wide" in k for k in kernels) == 66
+    assert sum("k_wgrad" in k for k in kernels) == 6
+    for name, f in kernels.items():
+        assert f["vgpr_count"] <= 512 and f["private_segment_fixed_size"] <= (88 if "k_conv_wideILi4ELi4E" in name else 0), (
+            name, f["vgpr_count"], f["private_segment_fixed_size"])
