@@ -128,6 +128,10 @@ struct swe_ctx {
   int32_t* sp_tile = nullptr;
   uint32_t* sp_rank = nullptr;
 
+  // device staging of the mesh, normals and wind map (view_scratch)
+  float* view = nullptr;
+  size_t view_bytes = 0;
+
   // counters (device)
   int64_t* lost = nullptr;     // swe::kLostSlots per terrain
   uint64_t* dstat = nullptr;   // swe::kStatKinds x swe::kStatSlots device statistics
@@ -850,6 +854,7 @@ int swe_destroy(swe_ctx* c) {
   dfree(c->sp_rank);
   dfree(c->lost);
   dfree(c->dstat);
+  dfree(c->view);
   dfree(c->dcycle);
   dfree(c->dterr);
   dfree(c->dcolour);
@@ -1483,17 +1488,41 @@ int swe_reset_stats(swe_ctx* c) {
   return 0;
 }
 
+// Device staging of a call that derives what a viewer reads: the context's,
+// grown as needed and kept, up to kViewKept bytes; a larger one is the call's own
+// (`own`).  Allocated and freed by every call, the mesh's, the normals' and the
+// wind map's sizes in turn took the allocator 0 to 250 us each, by what else the
+// process had allocated (a frame of 512^2 1.25 or 1.85 ms).
+constexpr size_t kViewKept = (size_t)1 << 30;
+
+static int view_scratch(swe_ctx* c, size_t bytes, float** out, float** own) {
+  *own = nullptr;
+  if (bytes > kViewKept) {
+    HIPCHK(c, hipMalloc((void**)own, bytes));
+    *out = *own;
+    return 0;
+  }
+  if (bytes > c->view_bytes) {
+    dfree(c->view);  // (every call that uses it has waited for its copy)
+    c->view_bytes = 0;
+    HIPCHK(c, hipMalloc((void**)&c->view, bytes));
+    c->view_bytes = bytes;
+  }
+  *out = c->view;
+  return 0;
+}
+
 int swe_mesh(swe_ctx* c, float* out) {
   if (!c || !out) return SWE_EINVAL;
   if (c->nterr != 1) return fail(c, SWE_EINVAL, "not available on a batch context");
   HIPCHK(c, hipSetDevice(c->device));
-  float* tmp = nullptr;
-  HIPCHK(c, hipMalloc((void**)&tmp, sizeof(float) * 12 * c->ncell));
+  float *tmp, *own;
+  if (const int r = view_scratch(c, sizeof(float) * (size_t)(12 * c->ncell), &tmp, &own)) return r;
   swe::launch_mesh(c->zs[c->cur()], tmp, c->nx, c->ny, c->p.mapscale, c->p.periodic != 0, c->stream);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, sizeof(float) * 12 * c->ncell, hipMemcpyDeviceToHost, c->stream);
   hipError_t e2 = hipStreamSynchronize(c->stream);
-  (void)hipFree(tmp);
+  dfree(own);
   if (e != hipSuccess) return fail(c, SWE_EHIP, std::string("mesh: ") + hipGetErrorString(e));
   if (e2 != hipSuccess) return fail(c, SWE_EHIP, std::string("mesh sync: ") + hipGetErrorString(e2));
   return 0;
@@ -1504,14 +1533,14 @@ int swe_windmap_terrain(swe_ctx* c, int32_t k, float* out) {
   if (k < 0 || k >= c->nterr) return fail(c, SWE_EINVAL, "terrain index out of range");
   HIPCHK(c, hipSetDevice(c->device));
   const int64_t c0 = c->tcell0[(size_t)k], n = (int64_t)c->tnx[(size_t)k] * c->tny[(size_t)k];
-  float* tmp = nullptr;
-  HIPCHK(c, hipMalloc((void**)&tmp, sizeof(float) * 4 * n));
+  float *tmp, *own;
+  if (const int r = view_scratch(c, sizeof(float) * (size_t)(4 * n), &tmp, &own)) return r;
   // the momentum planes of terrain k: x at ema[ncell + c0], y and z a plane stride further
   swe::launch_windmap(c->ema + c->ncell + c0, c->ncell, tmp, n, c->stream);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, sizeof(float) * 4 * n, hipMemcpyDeviceToHost, c->stream);
   hipError_t e2 = hipStreamSynchronize(c->stream);
-  (void)hipFree(tmp);
+  dfree(own);
   if (e != hipSuccess) return fail(c, SWE_EHIP, std::string("windmap: ") + hipGetErrorString(e));
   if (e2 != hipSuccess) return fail(c, SWE_EHIP, std::string("windmap sync: ") + hipGetErrorString(e2));
   return 0;
@@ -1529,13 +1558,13 @@ int swe_normals_terrain(swe_ctx* c, int32_t k, float* out) {
   HIPCHK(c, hipSetDevice(c->device));
   const int32_t nx = c->tnx[(size_t)k], ny = c->tny[(size_t)k];
   const int64_t c0 = c->tcell0[(size_t)k], n = (int64_t)nx * ny;
-  float* tmp = nullptr;
-  HIPCHK(c, hipMalloc((void**)&tmp, sizeof(float) * 3 * n));
+  float *tmp, *own;
+  if (const int r = view_scratch(c, sizeof(float) * (size_t)(3 * n), &tmp, &own)) return r;
   swe::launch_normals(c->zs[c->cur()] + c0, tmp, nx, ny, c->p.mapscale, c->p.periodic != 0, c->stream);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, c->stream);
   hipError_t e2 = hipStreamSynchronize(c->stream);
-  (void)hipFree(tmp);
+  dfree(own);
   if (e != hipSuccess) return fail(c, SWE_EHIP, std::string("normals: ") + hipGetErrorString(e));
   if (e2 != hipSuccess) return fail(c, SWE_EHIP, std::string("normals sync: ") + hipGetErrorString(e2));
   return 0;
