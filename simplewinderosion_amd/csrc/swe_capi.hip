@@ -131,6 +131,7 @@ struct swe_ctx {
   // device staging of the mesh, normals and wind map (view_scratch)
   float* view = nullptr;
   size_t view_bytes = 0;
+  std::mutex view_mutex;  // held from the staging's choice to the end of its copy
 
   // counters (device)
   int64_t* lost = nullptr;     // swe::kLostSlots per terrain
@@ -1516,6 +1517,7 @@ int swe_mesh(swe_ctx* c, float* out) {
   if (!c || !out) return SWE_EINVAL;
   if (c->nterr != 1) return fail(c, SWE_EINVAL, "not available on a batch context");
   HIPCHK(c, hipSetDevice(c->device));
+  std::lock_guard<std::mutex> lock(c->view_mutex);
   float *tmp, *own;
   if (const int r = view_scratch(c, sizeof(float) * (size_t)(12 * c->ncell), &tmp, &own)) return r;
   swe::launch_mesh(c->zs[c->cur()], tmp, c->nx, c->ny, c->p.mapscale, c->p.periodic != 0, c->stream);
@@ -1533,6 +1535,7 @@ int swe_windmap_terrain(swe_ctx* c, int32_t k, float* out) {
   if (k < 0 || k >= c->nterr) return fail(c, SWE_EINVAL, "terrain index out of range");
   HIPCHK(c, hipSetDevice(c->device));
   const int64_t c0 = c->tcell0[(size_t)k], n = (int64_t)c->tnx[(size_t)k] * c->tny[(size_t)k];
+  std::lock_guard<std::mutex> lock(c->view_mutex);
   float *tmp, *own;
   if (const int r = view_scratch(c, sizeof(float) * (size_t)(4 * n), &tmp, &own)) return r;
   // the momentum planes of terrain k: x at ema[ncell + c0], y and z a plane stride further
@@ -1558,6 +1561,7 @@ int swe_normals_terrain(swe_ctx* c, int32_t k, float* out) {
   HIPCHK(c, hipSetDevice(c->device));
   const int32_t nx = c->tnx[(size_t)k], ny = c->tny[(size_t)k];
   const int64_t c0 = c->tcell0[(size_t)k], n = (int64_t)nx * ny;
+  std::lock_guard<std::mutex> lock(c->view_mutex);
   float *tmp, *own;
   if (const int r = view_scratch(c, sizeof(float) * (size_t)(3 * n), &tmp, &own)) return r;
   swe::launch_normals(c->zs[c->cur()] + c0, tmp, nx, ny, c->p.mapscale, c->p.periodic != 0, c->stream);

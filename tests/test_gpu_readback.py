@@ -76,3 +76,33 @@ def test_batch_views_of_several_sizes():
         assert np.array_equal(got, want), k
         w.close()
     b.close()
+
+
+def test_threads_read_one_context():
+    """The staging is held by one call at a time: views read by several threads
+    at once, growing it in between, are those read alone."""
+    import threading
+
+    print("case views threads", flush=True)
+    w = World(96, 160)
+    w.upload(np.random.default_rng(3).random((96, 160)).astype(np.float32))
+    bad = []
+
+    def read(names, want):
+        for i in range(40):
+            for nm in names:
+                if not np.array_equal(getattr(w, nm)(), want[nm]):
+                    bad.append((nm, i))
+
+    ref = World(96, 160)
+    ref.upload(np.random.default_rng(3).random((96, 160)).astype(np.float32))
+    want = _views(ref)
+    orders = (("windmap", "normals", "mesh"), ("normals", "mesh", "windmap"), ("mesh", "windmap", "normals"))
+    ts = [threading.Thread(target=read, args=(o, want)) for o in orders]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad[:4]
+    ref.close()
+    w.close()
