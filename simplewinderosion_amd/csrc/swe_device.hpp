@@ -82,10 +82,11 @@ __device__ __forceinline__ float exp_f32(float x) {
 
 // s = sqrt(d) and r = 1 / s, both correctly rounded.  In the normal range one
 // v_rsq_f32 seeds Goldschmidt's coupled iteration g -> sqrt, h -> 1 / (2 sqrt),
-// whose final residual rounds s; one residual step from v_rcp_f32 rounds r (from 2h in
-// its place 450 of the range's quotients come out one ulp low, at s with all
-// mantissa bits set).  Equal to the IEEE square root and quotient for every
-// float (tests/test_gpu_primitives.py): 13 instructions in place of 26.  Zero, tiny, huge, negative and NaN take the IEEE operations.
+// whose final residual rounds s; one residual step from v_rcp_f32 rounds r
+// (from 2h in its place 450 of the range's quotients come out one ulp low, at
+// s with all mantissa bits set).  Equal to the IEEE square root and quotient
+// for every float (tests/test_gpu_primitives.py): 13 instructions in place of
+// 26.  Zero, tiny, huge, negative and NaN take the IEEE operations.
 struct Root {
   float s, r;
 };

@@ -1213,15 +1213,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
 }
 
 // The colour-ordered cascade in the same single launch per window: the tile
-// re-runs every cascade its cells (and their one-cell halo) depend on from
-// an LDS copy of the masters, instead of one launch per class over the map
-// (9 to 25 launches, each two memory round trips: 7.5 us apiece on 512^2).
+// re-runs, on an LDS copy of the masters, the cascades of all visited cells
+// within the reach of its own cells and their one-cell halo (colour_halo: a
+// bound, not a search of what they depend on), instead of one launch per
+// class over the map (9 to 25 launches, each two memory round trips: 7.5 us
+// apiece on 512^2).  colour_fused has the line between the two.
 // Redundant work is 3.4 regions per tile, but a window pays one launch and
 // one load of the region; its time is the most crowded tile's rounds of
 // dependent cascades (1,500 to 5,000 cycles each).  Measured against the
-// class launches: 512^2 bounded, 4096 particles 46.2 -> 12.8 ms a cycle; 400 x
-// 301 periodic, two layers, 30,000 particles 85.4 -> 28.7 ms; 1024^2 with a
-// million particles, where a class launch fills the chip, 110 -> 95 ms.
+// class launches: 512^2 bounded, 4096 particles 46.1 -> 12.8 ms a cycle; 400 x
+// 301 periodic, two layers, 30,000 particles 85.3 -> 28.2 ms; 1024^2 with a
+// million particles, where a class launch fills the chip, 110 -> 92 ms.
 template <int SX, int SY, int NT, bool PERIODIC, bool TRACK, int LAYERS, bool DEPOSIT, int MODE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colour_step(StepArgs) {
   step_body<SX, SY, NT, PERIODIC, TRACK, LAYERS, DEPOSIT, MODE>();  // reads its arguments from the kernel argument segment
