@@ -33,7 +33,7 @@ static inline float __builtin_amdgcn_rcpf(float x) { return 1.0f / x; }
 """
 
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is needed to build the checker")
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ is needed to build the check")
 def test_primitives_match_their_references(tmp_path):
     os.makedirs(str(tmp_path / "hip"))
     (tmp_path / "hip" / "hip_runtime.h").write_text(STAND_IN)
